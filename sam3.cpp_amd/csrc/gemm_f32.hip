@@ -16,6 +16,10 @@
 // are walked XCD-aware (each XCD a contiguous band), so the n-tiles of one
 // m-tile read their activation rows through one L2.
 //
+// gemm_f32_split_kernel is the form that most calls take (2-D, K >= 128 in a MUL_MAT, every neck
+// convolution, both patch embeddings): each fp32 value as three bf16 ones on the bf16 matrix
+// cores. The kernels above it serve batches, short K and what its buffer offsets don't reach.
+//
 // The same kernel runs a 3x3 / stride-1 / pad-1 convolution as an implicit
 // GEMM over a token-major [H*W][C] map (C % 32 == 0): a stage of 32 K values
 // lies within one tap, so each A row is one 128-byte segment of the pixel the
@@ -245,8 +249,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiled_kernel(const GemmF32Arg
 
 // The tiled kernel with its operands staged by LDS DMA (buffer_load ... lds) into NB stage
 // buffers of 32 K values (A and B rows of 128 bytes, 32 KB per stage), filled NB - 1 stages
-// ahead, so no registers stage anything and no branch guards a load: rows past M or N,
-// taps outside the image and the chunks of a last partial stage past K get an offset past
+// ahead, so no registers stage anything and no branch guards a load: rows past M or N
+// and the chunks of a last partial stage past K get an offset past
 // the buffer's records, which reads zero. Rows hold chunk c (k values 4c .. 4c + 3) in slot
 // c ^ fswz(r), so the 16 rows of a ds_read_b128 quarter (two parities of eight rows) cover
 // the 64 banks. Lane group g of a fragment read takes chunks 2q + g (q < 4), and MFMA step
@@ -269,7 +273,7 @@ struct F32Stage {
 
 // KD: K values per stage (32 or 16); NB stage buffers, up to NB - 1 stages in flight past the
 // one computed. sps counts 32-deep stages (the launcher's unit) whatever KD.
-template <bool CONV, int KD, int NB>
+template <int KD, int NB>
 __global__ __launch_bounds__(256, NB * KD * 2 * 128 * 4 <= 54 * 1024 ? 3 : (NB * KD * 2 * 128 * 4 <= 80 * 1024 ? 2 : 1))
 void gemm_f32_dma_kernel(const GemmF32Args p, int ksplit, int sps) {
     using Stage = F32Stage<KD>;
@@ -298,18 +302,13 @@ void gemm_f32_dma_kernel(const GemmF32Args p, int ksplit, int sps) {
 
     // DMA instruction j (< NI) of wavefront wv: tile rows RPI (NI wv + j) + lane / CH of A and of
     // B, LDS slot lane % CH, global chunk slot ^ fswz(row)
-    const v4i xr = make_rsrc(Xb, CONV ? (int64_t)M * p.C * 4 : (int64_t)(M - 1) * p.x_nb1 + 4LL * K);
+    const v4i xr = make_rsrc(Xb, (int64_t)(M - 1) * p.x_nb1 + 4LL * K);
     const v4i wr = make_rsrc(Wb, (int64_t)(N - 1) * p.w_nb1 + 4LL * K);
-    int ach[NI], aoff[NI], boff[NI], py[NI], px[NI];
+    int ach[NI], aoff[NI], boff[NI];
 #pragma unroll
     for (int j = 0; j < NI; ++j) {
         const int row = RPI * (NI * wv + j) + lane / CH, m = m0 + row, n = n0 + row;
         ach[j] = (lane % CH) ^ fswz<KD>(row);  // the chunk this lane loads
-        py[j] = px[j] = 0;
-        if (CONV) {
-            py[j] = m < M ? m / p.Wd : -(1 << 20);  // past M: every tap lands outside the image
-            px[j] = m < M ? m - (m / p.Wd) * p.Wd : 0;
-        }
         aoff[j] = m < M ? (int)((int64_t)m * p.x_nb1) + 16 * ach[j] : F32_OOB;
         boff[j] = n < N ? (int)((int64_t)n * p.w_nb1) + 16 * ach[j] : F32_OOB;
     }
@@ -321,15 +320,7 @@ void gemm_f32_dma_kernel(const GemmF32Args p, int ksplit, int sps) {
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
             const bool kin = k0 + 4 * ach[j] < K;  // false only in a last partial stage
-            int off;
-            if (CONV) {
-                const int tap = k0 / p.C, c0 = k0 - tap * p.C;
-                const int iy = py[j] + tap / 3 - 1, ix = px[j] + tap % 3 - 1;
-                const bool in = iy >= 0 && iy < p.H && ix >= 0 && ix < p.Wd;
-                off = in ? ((iy * p.Wd + ix) * p.C + c0) * 4 + 16 * ach[j] : F32_OOB;
-            } else {
-                off = aoff[j] != F32_OOB && kin ? aoff[j] + 4 * k0 : F32_OOB;
-            }
+            const int off = aoff[j] != F32_OOB && kin ? aoff[j] + 4 * k0 : F32_OOB;
             dma_b128_so(xr, base + (uint32_t)offsetof(Stage, A) + 1024u * (NI * wv + j), off, 0);
         }
 #pragma unroll
@@ -437,6 +428,369 @@ void gemm_f32_dma_kernel(const GemmF32Args p, int ksplit, int sps) {
     }
 }
 
+// The same GEMM on the bf16 matrix cores: an fp32 value is the exact sum of three bf16 values
+// (x = h + m + l, each rounded to nearest even from what the ones before left: 8 + 8 + 8 bits),
+// and six of the nine products, hh + hm + mh + hl + lh + mm, carry everything down to 2^-24 of
+// the term. v_mfma_f32_32x32x16_bf16 makes the sixteen products of one pair in 32 cycles where
+// eight v_mfma_f32_32x32x2f32 take 512, so six pairs cost 192: 2.7 times less matrix time for
+// the same fp32 accumulators, which round six times per 16 terms instead of eight.
+//
+// The weights come split already (split_w_kernel: per row and 32 of K the three planes' 64 bytes
+// side by side, 192 bytes); the activations arrive as fp32 by LDS DMA and are split as the
+// fragments are read, eleven VALU instructions per pair of values. A wavefront therefore owns
+// 32 whole rows of the 128 x 128 tile: each value is split once per workgroup, and its rows are
+// read by no other wavefront. Stages of 32 K (16 KB + 24 KB), two buffers, two workgroups per CU.
+//
+// Measured: the 288 x 288 3x3 convolution of 256 channels (97.8 GFLOP, 587 of them as bf16)
+// 1014 -> 510 us (1.15 PFLOP/s of bf16; 421 without the stage DMA, 387 without the split too: the
+// MFMAs alone run at the chip's power limit), 5184 x 1024 x 588 90 -> 57 us, weight pass included;
+// error against 64 bits 5.7e-7 -> 4.9e-7 at K = 1024. With 32 x 32 x 16 MFMAs 539 us.
+//
+// Infinities and NaN: a split infinity leaves NaN in m, and an infinite weight times a zero
+// plane is NaN too, so any output that is not finite is summed again in plain fp32 from the
+// unsplit operands (the weight planes add up to the weight exactly; an infinite weight has
+// m = l = 0). Among finite operands only activations that round up to an infinite bf16 need it.
+namespace {
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+typedef __bf16 v2b __attribute__((ext_vector_type(2)));
+struct SplitStage {
+    float A[TM * 32];
+    uint16_t B[TN * 96];  // row: plane p (h, m, l), 32 K each; chunk q of plane p in slot 4 p + (q ^ (row >> 2 & 3))
+};
+constexpr int SPLIT_NL = 10;  // DMA instructions per wavefront and stage: 4 activation, 6 weight
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
+    const v2f v = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, v2b));
+}
+// eight fp32 values -> their three bf16 planes
+__device__ __forceinline__ void split8(const v4f (&x)[2], v8b& h, v8b& m, v8b& l) {
+    v4i hh, mm, ll;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a = x[i >> 1][2 * (i & 1)], b = x[i >> 1][2 * (i & 1) + 1];
+        const uint32_t u = pk_bf16(a, b);
+        const float ra = a - __uint_as_float(u << 16), rb = b - __uint_as_float(u & 0xffff0000u);
+        const uint32_t v = pk_bf16(ra, rb);
+        hh[i] = (int)u;
+        mm[i] = (int)v;
+        ll[i] = (int)pk_bf16(ra - __uint_as_float(v << 16), rb - __uint_as_float(v & 0xffff0000u));
+    }
+    h = __builtin_bit_cast(v8b, hh);
+    m = __builtin_bit_cast(v8b, mm);
+    l = __builtin_bit_cast(v8b, ll);
+}
+}  // namespace
+
+// planes of weight rows [N][K] (row pitch nb1 bytes; F32 or F16; or, taps == 9, a 3x3 kernel
+// [N][C][3][3] read in (tap, channel) order) -> [N][KP / 32][3][32] bf16, zero past K. One thread
+// per eight consecutive K.
+__global__ __launch_bounds__(256) void split_w_kernel(const char* __restrict__ w, int64_t nb1, int f16, int taps, int N, int K,
+                                                      int KP, uint16_t* __restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int k8 = KP / 8;
+    if (i >= (int64_t)N * k8) return;
+    const int n = (int)(i / k8), k0 = (int)(i - (int64_t)n * k8) * 8;
+    const int C = K / taps;
+    uint16_t h[8], m[8], l[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int k = k0 + j;
+        float x = 0.0f;
+        if (k < K) {
+            const int64_t e = taps == 1 ? k : (int64_t)(k % C) * taps + k / C;
+            const char* row = w + (int64_t)n * nb1;
+            x = f16 ? h2f(reinterpret_cast<const uint16_t*>(row)[e]) : reinterpret_cast<const float*>(row)[e];
+        }
+        const uint32_t u = __float_as_uint(x);
+        uint32_t a = pk_bf16(x, 0.0f) & 0xffffu;
+        if ((a & 0x7f80u) == 0x7f80u) a = u >> 16;  // infinite, NaN, or rounded up to infinity: the top bits
+        if ((u & 0x7f800000u) == 0x7f800000u) {
+            if (u & 0x007fffffu) a |= 0x40u;  // a NaN stays one
+            h[j] = (uint16_t)a;
+            m[j] = l[j] = 0;
+            continue;
+        }
+        const float r = x - __uint_as_float(a << 16);
+        const uint32_t b = pk_bf16(r, 0.0f) & 0xffffu;
+        h[j] = (uint16_t)a;
+        m[j] = (uint16_t)b;
+        l[j] = (uint16_t)(pk_bf16(r - __uint_as_float(b << 16), 0.0f) & 0xffffu);
+    }
+    uint16_t* o = out + (int64_t)n * KP * 3 + (k0 >> 5) * 96 + (k0 & 31);
+    auto put = [&](uint16_t* d, const uint16_t (&v)[8]) {
+        *reinterpret_cast<uint4*>(d) = make_uint4(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16,
+                                                  v[4] | (uint32_t)v[5] << 16, v[6] | (uint32_t)v[7] << 16);
+    };
+    put(o, h);
+    put(o + 32, m);
+    put(o + 64, l);
+}
+
+template <bool CONV>
+__global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const GemmF32Args p, int ksplit, int sps) {
+    __shared__ __attribute__((aligned(16))) SplitStage sb[2];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // XCD-aware order with the K split as the slowest index, as the tiled kernel
+    const int M = p.M, N = p.N, K = p.K;
+    const int tiles_n = (N + TN - 1) / TN, tiles = ((M + TM - 1) / TM) * tiles_n;
+    const int TT = tiles * ksplit, per_xcd = (TT + 7) / 8;
+    const int tls = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (tls >= TT) return;
+    const int split = tls / tiles, tl = tls - split * tiles;
+    const int m0 = (tl / tiles_n) * TM, n0 = (tl % tiles_n) * TN;
+    const int s0 = split * sps, nst = min((K + 31) / 32 - s0, sps);
+    const char* Xb = reinterpret_cast<const char*>(p.X);
+    const int wrow = (K + 31) / 32 * 192;  // bytes of a split weight row
+
+    // DMA: activation instruction j of wavefront wv loads its own rows 32 wv + 8 j + lane / 8,
+    // LDS slot lane % 8, global chunk slot ^ fswz(row); weight instruction j loads LDS chunks
+    // 64 (6 wv + j) + lane of the stage's 128 rows x 12
+    const v4i xr = make_rsrc(Xb, CONV ? (int64_t)M * p.C * 4 : (int64_t)(M - 1) * p.x_nb1 + 4LL * K);
+    const v4i wr = make_rsrc(p.wsplit, (int64_t)N * wrow);
+    int ach[4], aoff[4], py[4], px[4], boff[6];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int row = 32 * wv + 8 * j + (lane >> 3), m = m0 + row;
+        ach[j] = (lane & 7) ^ fswz<32>(row);
+        py[j] = px[j] = 0;
+        if (CONV) {
+            py[j] = m < M ? m / p.Wd : -(1 << 20);  // past M: every tap lands outside the image
+            px[j] = m < M ? m - (m / p.Wd) * p.Wd : 0;
+        }
+        aoff[j] = m < M ? (int)((int64_t)m * p.x_nb1) + 16 * ach[j] : F32_OOB;
+    }
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+        const int c = 64 * (6 * wv + j) + lane, row = c / 12, slot = c - 12 * row, n = n0 + row;
+        boff[j] = n < N ? n * wrow + 16 * (slot ^ ((row >> 2) & 3)) : F32_OOB;
+    }
+    const uint32_t lb[2] = {(uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[0])),
+                            (uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[1]))};
+    auto dma = [&](int s, uint32_t base) __attribute__((always_inline)) {
+        const int k0 = (s0 + s) * 32;
+        const int tap = CONV ? k0 / p.C : 0, c0 = k0 - tap * p.C;
+        const int dy = CONV ? tap / 3 - 1 : 0, dx = CONV ? tap - (tap / 3) * 3 - 1 : 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            int off;
+            if (CONV) {
+                const int iy = py[j] + dy, ix = px[j] + dx;
+                const bool in = iy >= 0 && iy < p.H && ix >= 0 && ix < p.Wd;
+                off = in ? ((iy * p.Wd + ix) * p.C + c0) * 4 + 16 * ach[j] : F32_OOB;
+            } else {
+                off = aoff[j] != F32_OOB && k0 + 4 * ach[j] < K ? aoff[j] + 4 * k0 : F32_OOB;
+            }
+            dma_b128_so(xr, base + (uint32_t)offsetof(SplitStage, A) + 1024u * (4 * wv + j), off, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < 6; ++j)
+            dma_b128_so(wr, base + (uint32_t)offsetof(SplitStage, B) + 1024u * (6 * wv + j), boff[j], (s0 + s) * 192);
+    };
+
+    // MFMA operands swapped (A = weight rows, B = activation rows): lane l holds activation row
+    // l % 16 of a 16 x 16 tile and weight rows 4 (l / 16) .. + 3, four consecutive outputs. The
+    // 16 x 16 x 32 form moves half the accumulator traffic per product of 32 x 32 x 16, and the
+    // chip runs it at 1.89 PFLOP/s on random data against 1.64 (both power-limited).
+    // One stage is one K step of 32: 96 MFMAs per wavefront in four groups of two weight tiles.
+    // While a group runs, the next one's weight fragments are read; under the last group the next
+    // stage's activations are read and split, so no LDS latency or VALU work stands before an
+    // MFMA. The barrier lies before that last group: by then every wavefront holds the rest of
+    // stage s in registers, so its buffer is free for stage s + 2, and stage s + 1 is readable.
+    const int r16 = lane & 15, kg = lane >> 4;
+    v4f acc[2][8];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[i][j] = v4f{0, 0, 0, 0};
+    v4f x[2][2];  // activations of the next stage
+    auto read_a = [&](const SplitStage& st) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int ra = 32 * wv + 16 * i + r16;
+                x[i][h] = *reinterpret_cast<const v4f*>(&st.A[ra * 32 + (((2 * kg + h) ^ fswz<32>(ra)) << 2)]);
+            }
+    };
+    auto read_b = [&](v8b (&f)[2][3], const SplitStage& st, int grp) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                const int rb = 16 * (2 * grp + j) + r16;
+                f[j][q] = *reinterpret_cast<const v8b*>(&st.B[rb * 96 + ((4 * q + (kg ^ ((rb >> 2) & 3))) << 3)]);
+            }
+    };
+    // products [q0, q1) of the six, the small ones first: (l, h), (h, l), (m, m), (m, h), (h, m), (h, h)
+    auto mul = [&](const v8b (&a)[2][3], const v8b (&f)[2][3], int grp, int q0 = 0, int q1 = 6) __attribute__((always_inline)) {
+        constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+        for (int q = q0; q < q1; ++q)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][2 * grp + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[j][PB[q]], a[i][PA[q]], acc[i][2 * grp + j], 0, 0, 0);
+    };
+    v8b a0[2][3], a1[2][3], b0[2][3], b1[2][3];
+    auto stage = [&](int s, const v8b (&a)[2][3], v8b (&an)[2][3]) __attribute__((always_inline)) {
+        const SplitStage& st = sb[s & 1];
+        read_b(b1, st, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        mul(a, b0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        read_b(b0, st, 2);
+        __builtin_amdgcn_sched_barrier(0);
+        mul(a, b1, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        read_b(b1, st, 3);
+        __builtin_amdgcn_sched_barrier(0);
+        mul(a, b0, 2);
+        __builtin_amdgcn_sched_barrier(0);
+        if (s + 1 < nst) {
+            wait_vmcnt<0>();  // stage s + 1 has landed
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // and stage s's buffer is read
+            if (s + 2 < nst) dma(s + 2, lb[s & 1]);
+            read_a(sb[(s + 1) & 1]);
+            read_b(b0, sb[(s + 1) & 1], 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        mul(a, b1, 3, 0, 2);  // eight MFMAs under which the new fragments arrive
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" : "+v"(x[0][0]), "+v"(x[0][1]), "+v"(x[1][0]), "+v"(x[1][1]));  // the split stays below
+        split8(x[0], an[0][0], an[0][1], an[0][2]);  // (after the last stage, of values already used)
+        split8(x[1], an[1][0], an[1][1], an[1][2]);
+        mul(a, b1, 3, 2, 6);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // VALU
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // and above the loop's branches
+        asm volatile("" : "+v"(an[0][0]), "+v"(an[0][1]), "+v"(an[0][2]), "+v"(an[1][0]), "+v"(an[1][1]), "+v"(an[1][2]));
+    };
+
+    dma(0, lb[0]);
+    if (nst > 1) {
+        dma(1, lb[1]);
+        wait_vmcnt<SPLIT_NL>();
+    } else {
+        wait_vmcnt<0>();
+    }
+    __syncthreads();
+    read_a(sb[0]);
+    read_b(b0, sb[0], 0);
+    split8(x[0], a0[0][0], a0[0][1], a0[0][2]);
+    split8(x[1], a0[1][0], a0[1][1], a0[1][2]);
+    for (int s = 0; s < nst; s += 2) {
+        stage(s, a0, a1);
+        if (s + 1 < nst) stage(s + 1, a1, a0);
+    }
+
+    // outputs that are not finite: summed again in fp32, sixteen rows at a time through the
+    // wavefront's own rows of the stage buffers (every DMA has landed, and no other wavefront
+    // reads them)
+    float* own0 = &sb[0].A[1024 * wv];
+    float* own1 = &sb[1].A[1024 * wv];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        bool bad = false;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) bad |= !(fabsf(acc[i][j][r]) < __builtin_inff());
+        if (!__any(bad)) continue;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) (j < 4 ? own0 : own1)[64 * (4 * (j & 3) + r) + lane] = acc[i][j][r];
+        const int m = m0 + 32 * wv + 16 * i + r16;
+        for (int e = 0; e < 32; ++e) {
+            float* slot = &(e < 16 ? own0 : own1)[64 * (e & 15) + lane];
+            const int n = n0 + 16 * (e >> 2) + 4 * kg + (e & 3);
+            float v = *slot;
+            if (fabsf(v) < __builtin_inff() || m >= M || n >= N) continue;
+            const uint16_t* wp = p.wsplit + (int64_t)n * (wrow / 2);
+            v = 0.0f;
+            for (int k = 32 * s0; k < min(K, 32 * (s0 + nst)) && !(v != v); ++k) {
+                const uint16_t* w = wp + (k >> 5) * 96 + (k & 31);
+                const float wf = (__uint_as_float((uint32_t)w[0] << 16) + __uint_as_float((uint32_t)w[32] << 16)) +
+                                 __uint_as_float((uint32_t)w[64] << 16);
+                float av;
+                if (CONV) {
+                    const int tap = k / p.C, py_ = m / p.Wd + tap / 3 - 1, px_ = m % p.Wd + tap % 3 - 1;
+                    const bool in = py_ >= 0 && py_ < p.H && px_ >= 0 && px_ < p.Wd;
+                    av = in ? p.X[((int64_t)py_ * p.Wd + px_) * p.C + (k - tap * p.C)] : 0.0f;
+                } else {
+                    av = *reinterpret_cast<const float*>(Xb + (int64_t)m * p.x_nb1 + 4LL * k);
+                }
+                v = fmaf(av, wf, v);
+            }
+            *slot = v;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[i][j][r] = (j < 4 ? own0 : own1)[64 * (4 * (j & 3) + r) + lane];
+    }
+
+    // outputs leave as float4 where the rows allow it: this split's partial sums without bias
+    // (part [split][M][N]), or D with the bias and the addend (all loaded before the first store:
+    // D may alias it)
+    const bool parts = ksplit > 1;
+    char* D = reinterpret_cast<char*>(parts ? p.part + (int64_t)split * M * N : p.D);
+    const int64_t pitch = parts ? 4LL * N : p.d_nb1;
+    const float* add = parts ? nullptr : p.add;
+    const bool v4 = N % 4 == 0 && ((reinterpret_cast<uintptr_t>(D) | (uintptr_t)pitch | reinterpret_cast<uintptr_t>(add)) & 15) == 0;
+    v4f ad[2][8];
+    if (add) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int m = m0 + 32 * wv + 16 * i + r16, n = n0 + 16 * j + 4 * kg;
+                const float* src = add + (int64_t)m * N + n;
+                if (v4 && m < M && n < N) {
+                    ad[i][j] = *reinterpret_cast<const v4f*>(src);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) ad[i][j][r] = m < M && n + r < N ? src[r] : 0.0f;
+                }
+            }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int n = n0 + 16 * j + 4 * kg;
+        float bn[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bn[r] = !parts && p.bias && n + r < N ? p.bias[n + r] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int m = m0 + 32 * wv + 16 * i + r16;
+            if (m >= M) continue;
+            v4f v = acc[i][j];
+            if (!parts) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = v[r] + bn[r];
+            }
+            if (add) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = v[r] + ad[i][j][r];
+            }
+            float* d = reinterpret_cast<float*>(D + (int64_t)m * pitch) + n;
+            if (v4) {
+                if (n < N) *reinterpret_cast<v4f*>(d) = v;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (n + r < N) d[r] = v[r];
+            }
+        }
+    }
+}
+
 // D = bias + part[0] + part[1] + ... (in split order) over an M x N tile set, float4 columns
 // (f16out: D holds fp16, the sums rounded RNE)
 __global__ __launch_bounds__(256) void gemm_f32_split_reduce_kernel(const float* __restrict__ part, int S, int M, int N,
@@ -465,11 +819,11 @@ namespace {
 // out-of-range offset
 bool dma_ok(int64_t x_bytes, int64_t w_bytes) { return x_bytes < F32_OOB - 4096 && w_bytes < F32_OOB - 4096; }
 constexpr int F32_KD = 32, F32_NB = 2;  // K per stage and stage buffers of the DMA kernel
-// the fp32 MFMA kernels split grids below two tiles per CU; one 32-deep stage of a
-// 128 x 128 tile takes about 2.5 us alone on a CU
+// grids below two tiles per CU split K; one 32-deep stage of a 128 x 128 tile takes about 1.3 us
+// alone on a CU (64 x 1024 with K = 4096 against 1024: 180 and 52 us)
 int f32_ksplit(int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = ((M + TM - 1) / TM) * ((N + TN - 1) / TN);
-    return gemm_ksplit(tiles, 512, M, N, (K + TK - 1) / TK, 2.5);
+    return gemm_ksplit(tiles, 512, M, N, (K + TK - 1) / TK, 1.3);
 }
 }  // namespace
 
@@ -486,6 +840,24 @@ hipError_t launch_split_reduce(const float* part, int S, int M, int N, const flo
     const int64_t n = (int64_t)M * (N / 4);
     if (n > 0)
         gemm_f32_split_reduce_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(part, S, M, N, bias, D, d_nb1, f16out ? 1 : 0);
+    return hipGetLastError();
+}
+
+size_t gemm_f32_split_bytes(int64_t N, int64_t K) { return (size_t)(N * ((K + 31) / 32) * 192); }
+
+bool gemm_f32_split_ok(const GemmF32Args& a, int Z) {
+    if (Z != 1 || a.M <= 0 || a.N <= 0 || a.K <= 0) return false;
+    if (gemm_f32_split_bytes(a.N, a.K) >= (size_t)F32_OOB - 4096) return false;
+    if (reinterpret_cast<uintptr_t>(a.X) & 15) return false;
+    if (a.conv) return a.C % 32 == 0 && (int64_t)a.M * a.C * 4 < F32_OOB - 4096;
+    return a.K % 4 == 0 && (a.x_nb1 & 15) == 0 && (int64_t)(a.M - 1) * a.x_nb1 + 4LL * a.K < F32_OOB - 4096;
+}
+
+hipError_t launch_split_w(const void* w, int64_t nb1, bool f16, int taps, int N, int K, uint16_t* out, hipStream_t st) {
+    const int KP = (K + 31) / 32 * 32;
+    const int64_t n = (int64_t)N * (KP / 8);
+    if (n > 0)
+        split_w_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(static_cast<const char*>(w), nb1, f16 ? 1 : 0, taps, N, K, KP, out);
     return hipGetLastError();
 }
 
@@ -510,14 +882,18 @@ hipError_t launch_gemm_f32(const GemmF32Args& a, int Z, hipStream_t st) {
         if (S == 1 || e != hipSuccess) return e;
         return launch_split_reduce(a.part, S, a.M, a.N, a.bias, a.D, a.d_nb1, st);
     };
+    if (a.wsplit) {
+        if (!gemm_f32_split_ok(a, Z) || (reinterpret_cast<uintptr_t>(a.wsplit) & 15)) return hipErrorInvalidValue;
+        const unsigned nb = (unsigned)((tiles * S + 7) / 8 * 8);
+        if (a.conv) gemm_f32_split_kernel<true><<<nb, 256, 0, st>>>(a, S, sps);
+        else gemm_f32_split_kernel<false><<<nb, 256, 0, st>>>(a, S, sps);
+        return reduce();
+    }
     if (a.conv) {
         if (a.C % TK != 0 || a.K != 9 * a.C || (int64_t)a.H * a.Wd != a.M || Z != 1 ||
             (reinterpret_cast<uintptr_t>(a.X) & 15) || (reinterpret_cast<uintptr_t>(a.W) & 15) || (a.w_nb1 & 15))
             return hipErrorInvalidValue;
-        if (dma_ok((int64_t)a.M * a.C * 4, (int64_t)(a.N - 1) * a.w_nb1 + 4LL * a.K))
-            gemm_f32_dma_kernel<true, F32_KD, F32_NB><<<dim3((unsigned)((tiles * S + 7) / 8 * 8), 1), 256, 0, st>>>(a, S, sps);
-        else
-            gemm_f32_tiled_kernel<true><<<dim3((unsigned)((tiles * S + 7) / 8 * 8), 1), 256, 0, st>>>(a, S, sps);
+        gemm_f32_tiled_kernel<true><<<dim3((unsigned)((tiles * S + 7) / 8 * 8), 1), 256, 0, st>>>(a, S, sps);
         return reduce();
     }
     const bool tiled = a.K % 4 == 0 &&
@@ -527,7 +903,7 @@ hipError_t launch_gemm_f32(const GemmF32Args& a, int Z, hipStream_t st) {
     if (tiled) {
         // the DMA kernel's 32-bit buffer offsets must reach every operand of every batch
         if (dma_ok((int64_t)(a.M - 1) * a.x_nb1 + 4LL * a.K, (int64_t)(a.N - 1) * a.w_nb1 + 4LL * a.K))
-            gemm_f32_dma_kernel<false, F32_KD, F32_NB><<<dim3((unsigned)((tiles * S + 7) / 8 * 8), (unsigned)Z), 256, 0, st>>>(a, S, sps);
+            gemm_f32_dma_kernel<F32_KD, F32_NB><<<dim3((unsigned)((tiles * S + 7) / 8 * 8), (unsigned)Z), 256, 0, st>>>(a, S, sps);
         else
             gemm_f32_tiled_kernel<false><<<dim3((unsigned)((tiles * S + 7) / 8 * 8), (unsigned)Z), 256, 0, st>>>(a, S, sps);
         return reduce();

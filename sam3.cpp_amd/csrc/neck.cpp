@@ -66,17 +66,20 @@ size_t deconv_scratch(int64_t P, int64_t Cin, int64_t Cout) {
 }
 // the implicit-GEMM kernels take maps whose rows are 16-byte aligned with Cin % 32 == 0
 bool implicit_ok(const float* x, int64_t Cin) { return (reinterpret_cast<uintptr_t>(x) & 15) == 0 && Cin % 32 == 0; }
-// implicit 3x3: the kernel repacked to (tap, channel) rows; otherwise the im2col
-// columns in the kernel's type (x_aligned: the map's rows are 16-byte aligned). The
-// implicit-GEMM kernels' K-split partial sums follow (1x1 and 3x3).
+// F32 kernels the GEMM takes: their bf16 planes (more than the repacked rows of maps past its
+// buffer offsets); F16 3x3: the kernel repacked to (tap, channel) rows; otherwise a 3x3's im2col
+// columns in the kernel's type (x_aligned: the map's base is 16-byte aligned). The GEMMs' K-split
+// partial sums follow (1x1 and 3x3).
 size_t conv_scratch(int64_t P, int64_t Cin, int64_t Cout, int k, int wtype, bool x_aligned) {
     const bool implicit = x_aligned && Cin % 32 == 0;
     const size_t part = wtype == T_F32 ? gemm_f32_part_bytes(P, Cout, (int64_t)k * k * Cin)
                         : implicit     ? conv_f16_part_bytes(k * k, P, Cin, Cout)
                                        : 0;
-    if (k == 1) return part;
     const int64_t es = wtype == T_F32 ? 4 : 2;
-    if (x_aligned && Cin % 32 == 0) return align_up((size_t)(9 * Cin * Cout * es)) + part;
+    if (wtype == T_F32 && x_aligned && (k == 1 ? Cin % 4 == 0 : implicit))
+        return align_up(gemm_f32_split_bytes(Cout, (int64_t)k * k * Cin)) + part;
+    if (k == 1) return part;
+    if (implicit) return align_up((size_t)(9 * Cin * Cout * es)) + part;
     return align_up((size_t)(P * 9 * Cin * es));
 }
 
@@ -136,17 +139,10 @@ mi355_status conv(mi355_context* ctx, const mi355_tensor* w, const float* b, con
                           (k == 3 || (reinterpret_cast<uintptr_t>(w->data) & 15) == 0)))
         return fail(ctx, MI355_STATUS_FAILED, "neck_conv: fp16 maps off the implicit F16 path");
     if (w->type == T_F32 && aligned && (k == 1 || implicit_ok(x, Cin))) {
-        if (k == 3) {
-            Timed t(ctx, "neck_conv3x3_pack");
-            st = hip_check(ctx, t.done(launch_conv3x3_pack(static_cast<const float*>(w->data), Cin, Cout,
-                                                           reinterpret_cast<float*>(scratch), ctx->stream)),
-                           "conv3x3 pack");
-            if (st != MI355_STATUS_SUCCESS) return st;
-        }
         GemmF32Args g;
         g.W = k == 3 ? reinterpret_cast<const float*>(scratch) : static_cast<const float*>(w->data);
-        // the K split's partial sums follow the repacked kernel
-        g.part = reinterpret_cast<float*>(scratch + (k == 3 ? align_up((size_t)(K * Cout * 4)) : 0));
+        // the K split's partial sums follow the kernel's planes (or its repacked rows)
+        g.part = reinterpret_cast<float*>(scratch + align_up(gemm_f32_split_bytes(Cout, K)));
         g.part_bytes = gemm_f32_part_bytes(P, Cout, K);
         g.w_nb1 = 4 * K;
         g.w_nb2 = g.w_nb3 = 4 * K * Cout;
@@ -165,6 +161,19 @@ mi355_status conv(mi355_context* ctx, const mi355_tensor* w, const float* b, con
         g.H = H;
         g.Wd = W;
         g.C = Cin;
+        if (gemm_f32_split_ok(g, 1)) {
+            g.wsplit = reinterpret_cast<const uint16_t*>(scratch);
+            Timed t(ctx, "neck_conv_split_w");
+            st = hip_check(ctx, t.done(launch_split_w(w->data, 4 * K, false, k * k, Cout, (int)K,
+                                                      reinterpret_cast<uint16_t*>(scratch), ctx->stream)),
+                           "conv kernel split");
+        } else if (k == 3) {
+            Timed t(ctx, "neck_conv3x3_pack");
+            st = hip_check(ctx, t.done(launch_conv3x3_pack(static_cast<const float*>(w->data), Cin, Cout,
+                                                           reinterpret_cast<float*>(scratch), ctx->stream)),
+                           "conv3x3 pack");
+        }
+        if (st != MI355_STATUS_SUCCESS) return st;
         Timed t(ctx, k == 3 ? "neck_conv3x3_f32" : "neck_conv1x1_f32");
         return hip_check(ctx, t.done(launch_gemm_f32(g, 1, ctx->stream)), "gemm_f32 launch");
     }
@@ -294,7 +303,8 @@ mi355_status mi355_neck_conv(mi355_context* ctx, const mi355_tensor* w, const fl
     (void)hipSetDevice(ctx->device);
     char* scr = nullptr;
     const int k = (int)w->ne[0];
-    const size_t sb = conv_scratch((int64_t)H * W, w->ne[2], w->ne[3], k, w->type, implicit_ok(x, w->ne[2]));
+    const size_t sb = conv_scratch((int64_t)H * W, w->ne[2], w->ne[3], k, w->type,
+                                   (reinterpret_cast<uintptr_t>(x) & 15) == 0);
     mi355_status st = scratch_for(ctx, sb, &scr);
     if (st != MI355_STATUS_SUCCESS) return st;
     return conv(ctx, w, b, x, H, W, y, scr);

@@ -1,0 +1,109 @@
+"""F32 MUL_MATs and neck convolutions on the bf16-MFMA kernel (each fp32 value
+as three bf16 ones, six products): against float64, at the edges of its tiles
+(128 x 128, 32 of K), its K remainders and its K split, and with infinities
+and NaN.
+
+Bound: an output adds six products per 32 of K into an fp32 accumulator, each
+addition rounding by at most 2^-23 of a running sum that stays below
+S = sum |w x|, and drops three products of at most 2^-24 S each:
+(6 ceil(K / 32) + 4) 2^-23 S; a K split adds one rounding per range."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _mul_mat(mi, ctx, w, x, noalloc=False):
+    wd, xd = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda()
+    out = torch.full((x.shape[0], w.shape[0]), float("nan"), dtype=torch.float32, device="cuda")
+    call = ctx.mul_mat_noalloc if noalloc else ctx.mul_mat
+    K = w.shape[1]
+    call(mi.from_torch(wd, mi.F32, [K, w.shape[0]]), mi.from_torch(xd, mi.F32, [K, x.shape[0]]),
+         mi.from_torch(out, mi.F32, [w.shape[0], x.shape[0]]))
+    ctx.synchronize()
+    return out.cpu().numpy()
+
+
+def _bound(K, s, extra=0):
+    return (6 * -(-K // 32) + 4 + extra) * 2.0 ** -23 * s + 1e-37
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 128), (128, 128, 128), (129, 127, 132), (127, 130, 160), (33, 17, 588),
+                                   (300, 257, 1020), (5, 260, 2304)])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_mul_mat_f32_split(mi, ctx, M, N, K, noalloc):
+    rng = np.random.default_rng(M * 7 + N + K)
+    w = (rng.standard_normal((N, K)) * np.exp(rng.uniform(-3, 3, (N, 1)))).astype(np.float32)
+    x = (rng.standard_normal((M, K)) * np.exp(rng.uniform(-8, 8, (M, K)))).astype(np.float32)
+    got = _mul_mat(mi, ctx, w, x, noalloc).astype(np.float64)
+    ref, s = x.astype(np.float64) @ w.astype(np.float64).T, np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    assert (np.abs(got - ref) <= _bound(K, s)).all(), float((np.abs(got - ref) / s).max())
+
+
+def test_mul_mat_f32_split_exact_integers(mi, ctx):
+    """Whole numbers whose sums stay below 2^24 come out exact (24-bit operands use all three planes)."""
+    rng = np.random.default_rng(3)
+    x = np.zeros((70, 256), np.float32)
+    x[np.arange(70), rng.integers(0, 256, 70)] = rng.integers(-(2 ** 24) + 1, 2 ** 24, 70)
+    w = rng.integers(-1, 2, (90, 256)).astype(np.float32)
+    assert np.array_equal(_mul_mat(mi, ctx, w, x), x @ w.T)
+
+
+def test_mul_mat_f32_split_non_finite(mi, ctx):
+    """Infinities, NaN, and activations that round up to an infinite bf16 give what fp32 products
+    and sums give: weights of one significant bit have two zero planes."""
+    M, N, K = 140, 150, 192
+    rng = np.random.default_rng(5)
+    w = np.exp2(rng.integers(-3, 4, (N, K))).astype(np.float32) * rng.choice([-1, 1], (N, K)).astype(np.float32)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    inf, top = np.float32(np.inf), np.float32(3.4e38)
+    x[3, 5], x[9, 7], x[9, 100] = inf, inf, -inf
+    x[77, 191], x[139, 0] = np.nan, -inf
+    w[20, 7] = 0.0           # 0 * inf
+    w[:, 33] = np.abs(w[:, 33]) * 0 + 0.5
+    x[50, 33] = top          # finite: its bf16 rounds to infinity
+    x[50, :33] = x[50, 34:] = 0
+    w[149, 64], w[0, 191] = inf, np.nan
+    got = _mul_mat(mi, ctx, w, x)
+    with np.errstate(all="ignore"):
+        ref = np.zeros((M, N), np.float32)
+        for k in range(K):
+            ref = ref + x[:, k:k + 1] * w[:, k][None, :]
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(np.isinf(got), np.isinf(ref)) and np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    ok = np.isfinite(ref)
+    with np.errstate(all="ignore"):
+        s = np.abs(x.astype(np.float64)) @ np.abs(w.astype(np.float64)).T
+    assert (np.abs(got[ok].astype(np.float64) - ref[ok]) <= 4 * _bound(K, s[ok])).all()
+
+
+@pytest.mark.parametrize("H,W,Cin,Cout,k", [(8, 8, 32, 32, 3), (17, 11, 64, 36, 3), (23, 20, 256, 256, 3), (9, 13, 36, 20, 1),
+                                            (40, 33, 160, 132, 1)])
+@pytest.mark.parametrize("special", [False, True])
+def test_neck_conv_f32_split(mi, ctx, H, W, Cin, Cout, k, special):
+    rng = np.random.default_rng(H * W + Cin + k)
+    w = rng.standard_normal((Cout, Cin, k, k)).astype(np.float32)
+    b = rng.standard_normal(Cout).astype(np.float32)
+    x = rng.standard_normal((H, W, Cin)).astype(np.float32)
+    if special:  # one infinite pixel channel: the outputs its taps reach are infinite, the others untouched
+        x[H // 2, W // 2, Cin - 1] = np.inf
+    wd, bd, xd = (torch.from_numpy(a).cuda() for a in (w, b, x))
+    y = torch.full((H * W, Cout), float("nan"), dtype=torch.float32, device="cuda")
+    ctx.neck_conv(mi.from_torch(wd, mi.F32, [k, k, Cin, Cout]), bd.data_ptr(), xd.data_ptr(), H, W, y.data_ptr())
+    ctx.synchronize()
+    pad = np.zeros((H + k - 1, W + k - 1, Cin))
+    pad[k // 2:k // 2 + H, k // 2:k // 2 + W] = x
+    ref, s = np.zeros((H * W, Cout)), np.zeros((H * W, Cout))
+    with np.errstate(all="ignore"):
+        for i in range(k):
+            for j in range(k):
+                a, t = pad[i:i + H, j:j + W].reshape(H * W, Cin), w[:, :, i, j].astype(np.float64)
+                ref += a @ t.T
+                s += np.abs(a) @ np.abs(t).T
+    got = y.cpu().numpy().astype(np.float64)
+    fin = np.isfinite(ref)
+    assert fin.all() != special
+    assert np.array_equal(np.isinf(got), np.isinf(ref)) and np.array_equal(got[~fin], ref[~fin])
+    err = np.abs(got[fin] - (ref + b)[fin])
+    assert (err <= _bound(Cin * k * k, s[fin], 20) + 2.0 ** -23 * (np.abs(ref[fin]) + np.abs(np.broadcast_to(b, ref.shape)[fin]))).all()
