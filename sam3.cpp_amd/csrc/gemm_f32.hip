@@ -442,8 +442,8 @@ void gemm_f32_dma_kernel(const GemmF32Args p, int ksplit, int sps) {
 // read by no other wavefront. Stages of 32 K (16 KB + 24 KB), two buffers, two workgroups per CU.
 //
 // Measured: the 288 x 288 3x3 convolution of 256 channels (97.8 GFLOP, 587 of them as bf16)
-// 1014 -> 510 us (1.15 PFLOP/s of bf16; 421 without the stage DMA, 387 without the split too: the
-// MFMAs alone run at the chip's power limit), 5184 x 1024 x 588 90 -> 57 us, weight pass included;
+// 1014 -> 489 us (1.2 PFLOP/s of bf16; about 400 without the stage DMA, 370 without the split too:
+// the MFMAs alone run at the chip's power limit), 5184 x 1024 x 588 90 -> 57 us, weight pass included;
 // error against 64 bits 5.7e-7 -> 4.9e-7 at K = 1024. With 32 x 32 x 16 MFMAs 539 us.
 //
 // Infinities and NaN: a split infinity leaves NaN in m, and an infinite weight times a zero
@@ -548,17 +548,20 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const GemmF32Arg
     // 64 (6 wv + j) + lane of the stage's 128 rows x 12
     const v4i xr = make_rsrc(Xb, CONV ? (int64_t)M * p.C * 4 : (int64_t)(M - 1) * p.x_nb1 + 4LL * K);
     const v4i wr = make_rsrc(p.wsplit, (int64_t)N * wrow);
-    int ach[4], aoff[4], py[4], px[4], boff[6];
+    int ach[4], aoff[4], tmask[4], boff[6];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int row = 32 * wv + 8 * j + (lane >> 3), m = m0 + row;
-        ach[j] = (lane & 7) ^ fswz<32>(row);
-        py[j] = px[j] = 0;
-        if (CONV) {
-            py[j] = m < M ? m / p.Wd : -(1 << 20);  // past M: every tap lands outside the image
-            px[j] = m < M ? m - (m / p.Wd) * p.Wd : 0;
+        ach[j] = 16 * ((lane & 7) ^ fswz<32>(row));
+        aoff[j] = m < M ? (int)((int64_t)m * (CONV ? 4LL * p.C : p.x_nb1)) + ach[j] : F32_OOB;
+        tmask[j] = 0;  // the taps inside the image
+        if (CONV && m < M) {
+            const int py = m / p.Wd, px = m - py * p.Wd;
+            for (int t = 0; t < 9; ++t) {
+                const int iy = py + t / 3 - 1, ix = px + t % 3 - 1;
+                tmask[j] |= (iy >= 0 && iy < p.H && ix >= 0 && ix < p.Wd) << t;
+            }
         }
-        aoff[j] = m < M ? (int)((int64_t)m * p.x_nb1) + 16 * ach[j] : F32_OOB;
     }
 #pragma unroll
     for (int j = 0; j < 6; ++j) {
@@ -567,25 +570,36 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const GemmF32Arg
     }
     const uint32_t lb[2] = {(uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[0])),
                             (uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[1]))};
-    auto dma = [&](int s, uint32_t base) __attribute__((always_inline)) {
-        const int k0 = (s0 + s) * 32;
-        const int tap = CONV ? k0 / p.C : 0, c0 = k0 - tap * p.C;
-        const int dy = CONV ? tap / 3 - 1 : 0, dx = CONV ? tap - (tap / 3) * 3 - 1 : 0;
+    // stages are loaded in order; a convolution's lane offsets change only with the tap, a GEMM's
+    // only in a last partial stage, and the rest of a stage's offset is the loads' scalar one
+    const int cps = CONV ? p.C / 32 : 1;
+    int ds = s0, dtap = CONV ? s0 / cps : 0, dcs = CONV ? s0 - dtap * cps : s0;
+    int voff[4];
+    auto at_tap = [&]() __attribute__((always_inline)) {
+        const int off = CONV ? ((dtap / 3 - 1) * p.Wd + dtap % 3 - 1) * p.C * 4 : 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            int off;
-            if (CONV) {
-                const int iy = py[j] + dy, ix = px[j] + dx;
-                const bool in = iy >= 0 && iy < p.H && ix >= 0 && ix < p.Wd;
-                off = in ? ((iy * p.Wd + ix) * p.C + c0) * 4 + 16 * ach[j] : F32_OOB;
-            } else {
-                off = aoff[j] != F32_OOB && k0 + 4 * ach[j] < K ? aoff[j] + 4 * k0 : F32_OOB;
-            }
-            dma_b128_so(xr, base + (uint32_t)offsetof(SplitStage, A) + 1024u * (4 * wv + j), off, 0);
+        for (int j = 0; j < 4; ++j)
+            voff[j] = aoff[j] != F32_OOB && (!CONV || ((tmask[j] >> dtap) & 1)) ? aoff[j] + off : F32_OOB;
+    };
+    at_tap();
+    auto dma = [&](uint32_t base) __attribute__((always_inline)) {
+        if (!CONV && 32 * ds + 32 > K) {  // chunks past K read zero
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (128 * ds + ach[j] >= 4 * K) voff[j] = F32_OOB;
         }
 #pragma unroll
+        for (int j = 0; j < 4; ++j)
+            dma_b128_so(xr, base + (uint32_t)offsetof(SplitStage, A) + 1024u * (4 * wv + j), voff[j], dcs * 128);
+#pragma unroll
         for (int j = 0; j < 6; ++j)
-            dma_b128_so(wr, base + (uint32_t)offsetof(SplitStage, B) + 1024u * (6 * wv + j), boff[j], (s0 + s) * 192);
+            dma_b128_so(wr, base + (uint32_t)offsetof(SplitStage, B) + 1024u * (6 * wv + j), boff[j], ds * 192);
+        ++ds;
+        if (++dcs == cps && CONV) {
+            dcs = 0;
+            ++dtap;
+            at_tap();
+        }
     };
 
     // MFMA operands swapped (A = weight rows, B = activation rows): lane l holds activation row
@@ -651,7 +665,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const GemmF32Arg
         if (s + 1 < nst) {
             wait_vmcnt<0>();  // stage s + 1 has landed
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // and stage s's buffer is read
-            if (s + 2 < nst) dma(s + 2, lb[s & 1]);
+            if (s + 2 < nst) dma(lb[s & 1]);
             read_a(sb[(s + 1) & 1]);
             read_b(b0, sb[(s + 1) & 1], 0);
         }
@@ -672,9 +686,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const GemmF32Arg
         asm volatile("" : "+v"(an[0][0]), "+v"(an[0][1]), "+v"(an[0][2]), "+v"(an[1][0]), "+v"(an[1][1]), "+v"(an[1][2]));
     };
 
-    dma(0, lb[0]);
+    dma(lb[0]);
     if (nst > 1) {
-        dma(1, lb[1]);
+        dma(lb[1]);
         wait_vmcnt<SPLIT_NL>();
     } else {
         wait_vmcnt<0>();

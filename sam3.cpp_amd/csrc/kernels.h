@@ -371,16 +371,18 @@ hipError_t launch_conv3x3_pack_f16(const uint16_t* w, int Cin, int Cout, uint16_
 // N = 4 * Cout, y the 2x map, GELU-erf after the bias if gelu). Taps 1 and 9 may split K
 // into ranges whose partial sums go to part [split][M][N] (at most part_bytes; none without
 // part) and are added, with the bias, by launch_split_reduce.
-// x16 / y16: the map in / out is fp16 (the f32 values rounded RNE, which the kernel's own rounding
-// of an F32 map gives: the same products), for maps only these kernels read.
+// x16: the map is fp16 (the f32 values rounded RNE), for the DMA kernel (conv_f16_dma_fits); an F32
+// map takes the register-staged kernel, which rounds it as it loads. y16: the output too (x16 only).
 hipError_t launch_conv_f16(int taps, const void* x, bool x16, const uint16_t* w, const float* bias, int H, int W, int C,
                            int N, bool gelu, void* y, bool y16, hipStream_t st, float* part = nullptr,
                            size_t part_bytes = 0);
+// whether the DMA kernel's buffer offsets reach an M-pixel map of C channels and N weight rows
+bool conv_f16_dma_fits(int taps, int64_t M, int64_t C, int64_t N);
 // partial-sum bytes launch_conv_f16 uses for taps 1 or 9 over M pixels, C input and N output
 // channels (0: no K split)
 size_t conv_f16_part_bytes(int taps, int64_t M, int64_t C, int64_t N);
 hipError_t launch_bias_rows(float* y, const float* b, int64_t rows, int C, hipStream_t st);
-hipError_t launch_maxpool2(const float* x, int H, int W, int C, float* y, hipStream_t st);
+hipError_t launch_maxpool2(const void* x, int H, int W, int C, void* y, hipStream_t st, bool f16 = false);
 hipError_t launch_hiera_pos_embed(const float* bkg, int E, int bh, int bw, const float* win, int ws, int H, int W,
                                   float* out, hipStream_t st);
 

@@ -61,13 +61,14 @@ mi355_status check_kernel(mi355_context* ctx, const mi355_tensor* w, const float
 
 // scratch bytes of each op (the MUL_MAT's own workspace is the context's); the
 // conv-transpose's GEMM output D is only written when the map takes the MUL_MAT path
+// (the map rounded to fp16 for the implicit path lies in its place)
 size_t deconv_scratch(int64_t P, int64_t Cin, int64_t Cout) {
-    return align_up((size_t)(4 * Cout * Cin * 2)) + align_up((size_t)(P * 4 * Cout * 4));
+    return align_up((size_t)(4 * Cout * Cin * 2)) + align_up((size_t)std::max(P * 4 * Cout * 4, P * Cin * 2));
 }
 // the implicit-GEMM kernels take maps whose rows are 16-byte aligned with Cin % 32 == 0
 bool implicit_ok(const float* x, int64_t Cin) { return (reinterpret_cast<uintptr_t>(x) & 15) == 0 && Cin % 32 == 0; }
 // F32 kernels the GEMM takes: their bf16 planes (more than the repacked rows of maps past its
-// buffer offsets); F16 3x3: the kernel repacked to (tap, channel) rows; otherwise a 3x3's im2col
+// buffer offsets); F16 kernels: a 3x3's repacked (tap, channel) rows and the fp16 map; otherwise a 3x3's im2col
 // columns in the kernel's type (x_aligned: the map's base is 16-byte aligned). The GEMMs' K-split
 // partial sums follow (1x1 and 3x3).
 size_t conv_scratch(int64_t P, int64_t Cin, int64_t Cout, int k, int wtype, bool x_aligned) {
@@ -78,9 +79,18 @@ size_t conv_scratch(int64_t P, int64_t Cin, int64_t Cout, int k, int wtype, bool
     const int64_t es = wtype == T_F32 ? 4 : 2;
     if (wtype == T_F32 && x_aligned && (k == 1 ? Cin % 4 == 0 : implicit))
         return align_up(gemm_f32_split_bytes(Cout, (int64_t)k * k * Cin)) + part;
+    // F16 kernels on the implicit path: the repacked 3x3, then the map rounded to fp16
+    if (implicit && wtype == T_F16) return (k == 3 ? align_up((size_t)(9 * Cin * Cout * 2)) : 0) + align_up((size_t)(P * Cin * 2)) + part;
     if (k == 1) return part;
-    if (implicit) return align_up((size_t)(9 * Cin * Cout * es)) + part;
     return align_up((size_t)(P * 9 * Cin * es));
+}
+
+// an F32 map rounded to fp16 (RNE, as ggml rounds the operands of its F16 convolutions) for the
+// DMA kernels
+mi355_status half_map(mi355_context* ctx, const float* x, int64_t P, int64_t C, void* out) {
+    const mi355_tensor t = dev_t(x, T_F32, C, P);
+    Timed tm(ctx, "neck_convert_f16");
+    return hip_check(ctx, tm.done(launch_convert_f16(view_of(&t), static_cast<uint16_t*>(out), C, ctx->stream)), "map to f16");
 }
 
 // conv_transpose_2d_p0(kernel [2, 2, Cout, Cin], stride 2) + bias (+ GELU):
@@ -104,8 +114,15 @@ mi355_status deconv(mi355_context* ctx, const mi355_tensor* w, const float* b, c
     }
     if (implicit_ok(x, Cin)) {
         // one fp16-MFMA GEMM whose epilogue adds the bias (+ GELU) and scatters to the 2x map
+        const void* xm = x;
+        if (!x16 && conv_f16_dma_fits(4, P, Cin, 4LL * Cout)) {
+            st = half_map(ctx, x, P, Cin, D);
+            if (st != MI355_STATUS_SUCCESS) return st;
+            xm = D;
+            x16 = true;
+        }
         Timed t(ctx, "neck_deconv_f16");
-        return hip_check(ctx, t.done(launch_conv_f16(4, x, x16, packed, b, H, W, Cin, 4 * Cout, gelu, y, y16, ctx->stream)),
+        return hip_check(ctx, t.done(launch_conv_f16(4, xm, x16, packed, b, H, W, Cin, 4 * Cout, gelu, y, y16, ctx->stream)),
                          "deconv_f16 launch");
     }
     if (x16 || y16) return fail(ctx, MI355_STATUS_FAILED, "neck_deconv: fp16 maps off the implicit path");
@@ -188,10 +205,18 @@ mi355_status conv(mi355_context* ctx, const mi355_tensor* w, const float* b, con
             if (st != MI355_STATUS_SUCCESS) return st;
         }
         const uint16_t* wk = k == 3 ? reinterpret_cast<const uint16_t*>(scratch) : static_cast<const uint16_t*>(w->data);
-        // the K split's partial sums follow the repacked kernel
-        float* part = reinterpret_cast<float*>(scratch + (k == 3 ? align_up((size_t)(K * Cout * 2)) : 0));
+        // the fp16 map and the K split's partial sums follow the repacked kernel
+        char* next = scratch + (k == 3 ? align_up((size_t)(K * Cout * 2)) : 0);
+        const void* xm = x;
+        if (!x16 && conv_f16_dma_fits(k * k, P, Cin, Cout)) {
+            st = half_map(ctx, x, P, Cin, next);
+            if (st != MI355_STATUS_SUCCESS) return st;
+            xm = next;
+            x16 = true;
+        }
+        float* part = reinterpret_cast<float*>(next + align_up((size_t)(P * Cin * 2)));
         Timed t(ctx, k == 3 ? "neck_conv3x3_f16" : "neck_conv1x1_f16");
-        return hip_check(ctx, t.done(launch_conv_f16(k * k, x, x16, wk, b, H, W, Cin, Cout, false, y, y16, ctx->stream,
+        return hip_check(ctx, t.done(launch_conv_f16(k * k, xm, x16, wk, b, H, W, Cin, Cout, false, y, y16, ctx->stream,
                                                      part, conv_f16_part_bytes(k * k, P, Cin, Cout))),
                          "conv_f16 launch");
     }
@@ -211,10 +236,10 @@ mi355_status conv(mi355_context* ctx, const mi355_tensor* w, const float* b, con
     return hip_check(ctx, t.done(launch_bias_rows(y, b, P, Cout, ctx->stream)), "bias");
 }
 
-mi355_status pool(mi355_context* ctx, const float* x, int H, int W, int C, float* y) {
+mi355_status pool(mi355_context* ctx, const void* x, int H, int W, int C, void* y, bool f16 = false) {
     if (C % 4 != 0) return fail(ctx, MI355_STATUS_UNSUPPORTED, "neck_maxpool: C %% 4 != 0");
     Timed t(ctx, "neck_maxpool");
-    return hip_check(ctx, t.done(launch_maxpool2(x, H, W, C, y, ctx->stream)), "maxpool");
+    return hip_check(ctx, t.done(launch_maxpool2(x, H, W, C, y, ctx->stream, f16)), "maxpool");
 }
 
 mi355_status scratch_for(mi355_context* ctx, size_t bytes, char** p) {
@@ -238,10 +263,11 @@ bool fp16_maps(const float* x, int E, const mi355_neck_scale* s) {
     return f16(s[0].deconv2_w) && s[0].deconv2_w->ne[3] % 32 == 0;
 }
 
-// Buffer plan of the whole neck: two map buffers plus the largest op scratch.
+// Buffer plan of the whole neck: two map buffers, the input rounded to fp16, and the largest op
+// scratch.
 struct NeckPlan {
-    size_t map = 0, scratch = 0;
-    size_t total() const { return 2 * map + scratch; }
+    size_t map = 0, half = 0, scratch = 0;
+    size_t total() const { return 2 * map + half + scratch; }
 };
 
 bool neck_plan(int E, int G, const mi355_neck_scale* s, NeckPlan* pl) {
@@ -250,6 +276,7 @@ bool neck_plan(int E, int G, const mi355_neck_scale* s, NeckPlan* pl) {
         if (!ok(s[i].conv1x1_w) || !ok(s[i].conv3x3_w) || (i < 2 && !ok(s[i].deconv1_w)) || (i == 0 && !ok(s[0].deconv2_w)))
             return false;
     const int64_t G2 = (int64_t)G * G;
+    pl->half = align_up((size_t)(G2 * E * 2));
     auto mapb = [&](int64_t P, int64_t C) { pl->map = std::max(pl->map, align_up((size_t)(P * C * 4))); };
     auto scr = [&](size_t b) { pl->scratch = std::max(pl->scratch, b); };
     // scale 0: deconv E->C1 (2G), GELU, deconv C1->D (4G), 1x1, 3x3
@@ -346,7 +373,8 @@ mi355_status mi355_sam3_neck(mi355_context* ctx, const float* x, int E, int G, c
     char* base = static_cast<char*>(ctx->neck);
     float* A = reinterpret_cast<float*>(base);
     float* B = reinterpret_cast<float*>(base + pl.map);
-    char* scr = base + 2 * pl.map;
+    char* xh = base + 2 * pl.map;
+    char* scr = xh + pl.half;
 #define TRY(e)                                     \
     do {                                           \
         st = (e);                                  \
@@ -360,21 +388,29 @@ mi355_status mi355_sam3_neck(mi355_context* ctx, const float* x, int E, int G, c
     // and inputs to F16), so scale 0's first one hands the second an fp16 map whenever both
     // take the implicit path
     const bool hd = h || (implicit_ok(x, E) && s[0].deconv1_w->ne[2] % 32 == 0);
+    // what reads the input in fp16 (both first conv-transposes; scale 2's 1x1 and the pool with F16
+    // kernels throughout) reads one rounded copy; the pool's maximum commutes with the rounding
+    const int64_t P = (int64_t)G * G;
+    const bool xh_ok = implicit_ok(x, E) && conv_f16_dma_fits(4, P, E, 4 * std::max(s[0].deconv1_w->ne[2], s[1].deconv1_w->ne[2])) &&
+                       conv_f16_dma_fits(1, P, E, s[2].conv1x1_w->ne[3]);
+    if (xh_ok) TRY(half_map(ctx, x, P, E, xh));
+    const void* xd = xh_ok ? static_cast<const void*>(xh) : x;
+    const bool hx = h && xh_ok;
     // scale 0 (4x): deconv + GELU, deconv, 1x1, 3x3
-    TRY(deconv(ctx, s[0].deconv1_w, s[0].deconv1_b, x, G, G, true, A, scr, false, hd));
+    TRY(deconv(ctx, s[0].deconv1_w, s[0].deconv1_b, xd, G, G, true, A, scr, xh_ok, hd));
     TRY(deconv(ctx, s[0].deconv2_w, s[0].deconv2_b, A, 2 * G, 2 * G, false, B, scr, hd, h));
     TRY(conv(ctx, s[0].conv1x1_w, s[0].conv1x1_b, B, 4 * G, 4 * G, A, scr, h, h));
     TRY(conv(ctx, s[0].conv3x3_w, s[0].conv3x3_b, A, 4 * G, 4 * G, out[0], scr, h, false));
     // scale 1 (2x): deconv, 1x1, 3x3
-    TRY(deconv(ctx, s[1].deconv1_w, s[1].deconv1_b, x, G, G, false, A, scr, false, h));
+    TRY(deconv(ctx, s[1].deconv1_w, s[1].deconv1_b, xd, G, G, false, A, scr, xh_ok, h));
     TRY(conv(ctx, s[1].conv1x1_w, s[1].conv1x1_b, A, 2 * G, 2 * G, B, scr, h, h));
     TRY(conv(ctx, s[1].conv3x3_w, s[1].conv3x3_b, B, 2 * G, 2 * G, out[1], scr, h, false));
     // scale 2 (1x): 1x1, 3x3
-    TRY(conv(ctx, s[2].conv1x1_w, s[2].conv1x1_b, x, G, G, A, scr, false, h));
+    TRY(conv(ctx, s[2].conv1x1_w, s[2].conv1x1_b, hx ? xd : x, G, G, A, scr, hx, h));
     TRY(conv(ctx, s[2].conv3x3_w, s[2].conv3x3_b, A, G, G, out[2], scr, h, false));
     // scale 3 (0.5x): max-pool, 1x1, 3x3
-    TRY(pool(ctx, x, G, G, E, B));
-    TRY(conv(ctx, s[3].conv1x1_w, s[3].conv1x1_b, B, G / 2, G / 2, A, scr, false, h));
+    TRY(pool(ctx, hx ? xd : x, G, G, E, B, hx));
+    TRY(conv(ctx, s[3].conv1x1_w, s[3].conv1x1_b, B, G / 2, G / 2, A, scr, hx, h));
     TRY(conv(ctx, s[3].conv3x3_w, s[3].conv3x3_b, A, G / 2, G / 2, out[3], scr, h, false));
 #undef TRY
     return MI355_STATUS_SUCCESS;

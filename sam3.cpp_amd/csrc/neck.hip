@@ -225,42 +225,48 @@ __global__ __launch_bounds__(256, 2) void conv_f16_kernel(const float* __restric
     }
 }
 
-// conv_f16_kernel's implicit GEMM with its operands staged by LDS DMA (buffer_load ... lds):
-// per 32-deep K step the fp32 map rows (128 bytes of one tap's channel slice per output
-// pixel, zero by the buffer's range check outside the image or past M) and the fp16 weight
-// rows (64 bytes), two stage buffers (48 KB: three workgroups per CU; three buffers filled
-// two stages ahead left two per CU and measured slower), no staging registers.  The
-// map is rounded to fp16 (RNE, f2h) as the MFMA fragments are read from LDS: the operands,
-// products and accumulation order of conv_f16_kernel, so the same bits.
-// LDS rows: map rows of 8 chunks of 16 bytes, chunk c of row r in slot c ^ ((r >> 1) & 7),
-// so the 16 rows of a ds_read_b128 quarter (rows of two parities) cover all 64 banks;
-// weight rows as conv_f16_kernel's (csw<4>).
+// conv_f16_kernel's implicit GEMM over an fp16 map, both operands staged by LDS DMA
+// (buffer_load ... lds) in 64-deep K stages, two slices of 32 channels of a tap: rows of 128 bytes
+// per output pixel (zero by the buffer's range check outside the image or past M) and per weight
+// row: whole lines, which the L2 feeds to the LDS at 35 TB/s, twice the rate of 64-byte rows.
+// What bounds it: the 288 x 288 3x3 convolution of 256 channels takes 121 us (810 TFLOP/s; 152 with
+// 32-deep stages, 32 x 32 x 16 MFMAs and offsets worked out per stage), 81 without its MFMAs and 78
+// without its DMA. Three and five stages in flight (32-deep) or 256-row workgroups were no faster.
+// The 72 x 72 conv-transpose 1024 -> 4 x 512 62 -> 40 us, 144 x 144 512 -> 4 x 256 64 -> 47 us.
+// Two stage buffers, 64 KB: two workgroups per CU, four wavefronts of 64 x 64.
+// v_mfma_f32_16x16x32_f16 with the operands swapped (A = weight rows, B = pixels): a lane holds
+// four consecutive channels of one pixel, which leave in one store, and the chip runs this form
+// faster at its power limit than 32 x 32 x 16 (1.89 against 1.64 PFLOP/s on random data).
+// A slice's fragments are read while the slice before it is multiplied (two register sets). The
+// barrier lies before a stage's second half: by then both halves are in registers everywhere, so
+// the buffer takes stage s + 2, and stage s + 1 is readable.
+// LDS rows of eight 16-byte chunks, chunk c of row r in slot c ^ (r >> 1 & 7): the 16 rows of a
+// ds_read_b128 quarter (two to a line of the 64 banks) cover all of them.
 namespace {
-struct ConvDmaStage {
-    float A[CT * 32];     // 128 map rows x 32 channels, fp32
-    uint16_t B[CT * 32];  // 128 weight rows x 32 K, fp16
+constexpr int CONV_OOB = 0x7ffffff0;  // a buffer offset past every operand the launcher admits
+struct ConvStage {
+    uint16_t A[CT * 64];  // map rows (pixels) x two slices of 32 channels
+    uint16_t B[CT * 64];  // weight rows x 64 K
 };
-constexpr int CONV_OOB = 0x7ffffff0;
-constexpr int CONV_NB = 2;  // stage buffers  // a buffer offset past every operand the launcher admits
-__device__ __forceinline__ int aswz(int r) { return (r >> 1) & 7; }
+__device__ __forceinline__ int hswz(int r) { return (r >> 1) & 7; }
 }  // namespace
 
-// AH: the map is fp16 already (a producer of this file rounded it, RNE): its rows are 64 bytes
-// per stage, staged and read as the weights are, with no conversion. OH: the output is fp16
-// (the f32 result rounded, RNE), for a map only another of these kernels reads.
-template <int TAPS, int NB, bool AH = false, bool OH = false>
-__global__ __launch_bounds__(256, NB == 3 ? 2 : 3) void conv_f16_dma_kernel(const void* __restrict__ xv, const uint16_t* __restrict__ w,
+// OH: the output is fp16 (the f32 result rounded, RNE), for a map only another of these kernels reads.
+// PAIR: C % 64 == 0, so both slices of a stage lie in one tap: the lanes' map offsets change only
+// with the tap, and a stage's DMA is eight loads with a scalar offset. (Working the offsets out
+// for every stage took as many cycles as the stage's MFMAs.)
+template <int TAPS, bool OH, bool PAIR>
+__global__ __launch_bounds__(256, 2) void conv_f16_dma_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
                                                               const float* __restrict__ bias, int H, int W, int C, int N,
                                                               int gelu, void* __restrict__ yv, int ksplit, int sps,
                                                               float* __restrict__ part) {
-    constexpr int NL = AH ? 4 : 6;  // DMA instructions per wavefront and stage: 4 (fp16: 2) map, 2 weight
-    constexpr int NA = AH ? 2 : 4;  // map DMA instructions per wavefront and stage
-    __shared__ __attribute__((aligned(16))) ConvDmaStage sb[NB];
-    const int M = H * W, K = TAPS == 9 ? 9 * C : C, cps = C / 32;
+    constexpr int NL = 8;  // DMA instructions per wavefront and stage: 4 map, 4 weight
+    __shared__ __attribute__((aligned(16))) ConvStage sb[2];
+    const int M = H * W, K = TAPS == 9 ? 9 * C : C, cps = C / 32, nsl = K / 32;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wv & 1, wn = wv >> 1;
-    const int lr = lane & 31, g = lane >> 5;
+    const int wm = wv >> 1, wn = wv & 1;
+    const int r16 = lane & 15, kg = lane >> 4;
     // XCD-aware tile order (each XCD a contiguous band of tiles); with a K split (taps 1 and
     // 9) the split is the slowest index: slot (split, tile) runs stages [split * sps, + sps)
     const int tiles_n = (N + CT - 1) / CT, tiles = ((M + CT - 1) / CT) * tiles_n;
@@ -269,140 +275,185 @@ __global__ __launch_bounds__(256, NB == 3 ? 2 : 3) void conv_f16_dma_kernel(cons
     if (tls >= TT) return;
     const int split = tls / tiles, tl = tls - split * tiles;
     const int m0 = (tl / tiles_n) * CT, n0 = (tl % tiles_n) * CT;
+    const int s0 = split * sps, nst = min((nsl + 1) / 2 - s0, sps);  // this split's first stage and stage count
 
-    // map DMA instruction j of wavefront wv: tile rows 8 (4 wv + j) + lane / 8, LDS slot lane % 8,
-    // global chunk slot ^ aswz(row) (fp16 map: rows 16 (2 wv + j) + lane / 4, slot lane % 4, as
-    // the weights); weight instruction j: rows 16 (2 wv + j) + lane / 4, slot lane % 4
-    constexpr int XES = AH ? 2 : 4;  // map element bytes
-    const v4i xr = make_rsrc(xv, (int64_t)M * C * XES), wr = make_rsrc(w, (int64_t)N * K * 2);
-    int py[NA], px[NA], ach[NA];
+    // DMA instruction j moves rows 8 (4 wv + j) + lane / 8: LDS slot lane % 8, global chunk
+    // slot ^ hswz(row), slice chunk / 4. Per lane the byte offset of its chunk within the slice at
+    // the pixel itself and, for the 3x3, which taps lie inside
+    const v4i xr = make_rsrc(x, (int64_t)M * C * 2), wr = make_rsrc(w, (int64_t)N * K * 2);
+    int xoff[4], tmask[4], woff[4], half[4];
 #pragma unroll
-    for (int j = 0; j < NA; ++j) {
-        const int row = AH ? 16 * (2 * wv + j) + (lane >> 2) : 8 * (4 * wv + j) + (lane >> 3), p = m0 + row;
-        py[j] = p < M ? p / W : -(1 << 20);  // past M: every tap lands outside the image
-        px[j] = p < M ? p - (p / W) * W : 0;
-        ach[j] = AH ? (((lane & 3) ^ csw<4>(row)) << 4) : (((lane & 7) ^ aswz(row)) << 4);
-    }
-    int woff[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int row = 16 * (2 * wv + j) + (lane >> 2), n = n0 + row;
-        woff[j] = n < N ? n * K * 2 + (((lane & 3) ^ csw<4>(row)) << 4) : CONV_OOB;
-    }
-    uint32_t lb[NB];
-#pragma unroll
-    for (int i = 0; i < NB; ++i) lb[i] = (uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[i]));
-    auto dma = [&](int s, uint32_t base) __attribute__((always_inline)) {
-        const int tap = TAPS == 9 ? s / cps : 0, c0 = (s - tap * cps) * 32;
-        const int dy = TAPS == 9 ? tap / 3 - 1 : 0, dx = TAPS == 9 ? tap % 3 - 1 : 0;
-#pragma unroll
-        for (int j = 0; j < NA; ++j) {
-            const int iy = py[j] + dy, ix = px[j] + dx;
-            const bool in = iy >= 0 && iy < H && ix >= 0 && ix < W;
-            const int off = in ? ((iy * W + ix) * C + c0) * XES + ach[j] : CONV_OOB;
-            dma_b128_so(xr, base + (uint32_t)offsetof(ConvDmaStage, A) + 1024u * (NA * wv + j), off, 0);
-        }
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-            dma_b128_so(wr, base + (uint32_t)offsetof(ConvDmaStage, B) + 1024u * (2 * wv + j), woff[j], s * 64);
-    };
-
-    const v16f zf = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    v16f acc[2][2] = {{zf, zf}, {zf, zf}};
-    auto compute = [&](const ConvDmaStage& b) __attribute__((always_inline)) {
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            v8h a[2], bf[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int ra = wm * 64 + i * 32 + lr, rb = wn * 64 + i * 32 + lr;
-                if (AH) {
-                    const uint16_t* ah = reinterpret_cast<const uint16_t*>(b.A);
-                    a[i] = *reinterpret_cast<const v8h*>(&ah[ra * 32 + (((2 * kk + g) ^ csw<4>(ra)) << 3)]);
-                } else {
-                    const int c = 4 * kk + 2 * g;  // the lane's 8 channels: chunks c, c + 1 of its map row
-                    const v4f lo = *reinterpret_cast<const v4f*>(&b.A[ra * 32 + ((c ^ aswz(ra)) << 2)]);
-                    const v4f hi = *reinterpret_cast<const v4f*>(&b.A[ra * 32 + (((c + 1) ^ aswz(ra)) << 2)]);
-                    const uint4 q = {(uint32_t)f2h(lo[0]) | ((uint32_t)f2h(lo[1]) << 16), (uint32_t)f2h(lo[2]) | ((uint32_t)f2h(lo[3]) << 16),
-                                     (uint32_t)f2h(hi[0]) | ((uint32_t)f2h(hi[1]) << 16), (uint32_t)f2h(hi[2]) | ((uint32_t)f2h(hi[3]) << 16)};
-                    a[i] = __builtin_bit_cast(v8h, q);
-                }
-                bf[i] = *reinterpret_cast<const v8h*>(&b.B[rb * 32 + (((2 * kk + g) ^ csw<4>(rb)) << 3)]);
+    for (int j = 0; j < 4; ++j) {
+        const int row = 8 * (4 * wv + j) + (lane >> 3), p = m0 + row, n = n0 + row;
+        const int c = (lane & 7) ^ hswz(row), py = p / W, px = p - py * W;
+        half[j] = c >> 2;
+        xoff[j] = p < M ? p * C * 2 + ((c & 3) << 4) : CONV_OOB;
+        woff[j] = n < N ? n * K * 2 + (c << 4) : CONV_OOB;
+        tmask[j] = 0;
+        if (TAPS == 9 && p < M)
+            for (int t = 0; t < 9; ++t) {
+                const int iy = py + t / 3 - 1, ix = px + t % 3 - 1;
+                tmask[j] |= (iy >= 0 && iy < H && ix >= 0 && ix < W) << t;
             }
+    }
+    const uint32_t lb[2] = {(uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[0])),
+                            (uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[1]))};
+    // the next stage to load, in order: its first slice, that slice's tap and channel slice
+    int dsl = 2 * s0, dtap = TAPS == 9 ? dsl / cps : 0, dcs = dsl - dtap * cps;
+    int voff[4];  // PAIR: the lanes' map offsets of tap dtap
+    auto at_tap = [&]() __attribute__((always_inline)) {
+        const int off = TAPS == 9 ? ((dtap / 3 - 1) * W + dtap % 3 - 1) * C * 2 : 0;
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], bf[j], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < 4; ++j) {
+            const bool in = TAPS != 9 || ((tmask[j] >> dtap) & 1);
+            voff[j] = in && xoff[j] != CONV_OOB ? xoff[j] + off + 64 * half[j] : CONV_OOB;
         }
     };
-
-    const int s0 = split * sps, nst = min(K / 32 - s0, sps);  // this split's first stage and stage count
-    // NB buffers filled NB - 1 stages ahead
-    dma(s0, lb[0]);
-    if (nst > 1) dma(s0 + 1, lb[1]);
-    if (NB == 3 && nst > 2) dma(s0 + 2, lb[NB - 1]);
-    if (NB == 3 && nst > 2) wait_vmcnt<2 * NL>();
-    else if (nst > 1) wait_vmcnt<NL>();
-    else wait_vmcnt<0>();
-    __syncthreads();
-    for (int s = 0; s < nst; ++s) {
-        const int cb = s % NB;
-        compute(sb[cb]);
-        if (s + 1 < nst) {
-            if (NB == 3 && s + 2 < nst) wait_vmcnt<NL>();  // stage s + 1 has landed (s + 2 may be in flight)
-            else wait_vmcnt<0>();
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // and stage s's buffer is read
-            if (s + NB < nst) dma(s0 + s + NB, lb[cb]);
+    if (PAIR) at_tap();
+    auto dma = [&](uint32_t base) __attribute__((always_inline)) {
+        if (PAIR) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                dma_b128_so(xr, base + (uint32_t)offsetof(ConvStage, A) + 1024u * (4 * wv + j), voff[j], dcs * 64);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                dma_b128_so(wr, base + (uint32_t)offsetof(ConvStage, B) + 1024u * (4 * wv + j), woff[j], dsl * 64);
+            dsl += 2;
+            dcs += 2;
+            if (TAPS == 9 && dcs == cps) {
+                dcs = 0;
+                ++dtap;
+                at_tap();
+            }
+            return;
         }
+        // byte offset of each of the two slices' map rows from the pixel's own row
+        int tap[2], off[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            tap[h] = dtap;
+            off[h] = (TAPS == 9 ? ((dtap / 3 - 1) * W + dtap % 3 - 1) * C * 2 : 0) + dcs * 64;
+            if (TAPS == 9 && ++dcs == cps) {
+                dcs = 0;
+                ++dtap;
+            } else if (TAPS != 9) {
+                ++dcs;
+            }
+        }
+        const bool odd = dsl + 1 >= nsl;  // no second slice (the last stage of an odd count)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const bool in = !(odd && half[j]) && (TAPS != 9 || ((tmask[j] >> (half[j] ? tap[1] : tap[0])) & 1));
+            const int o = in && xoff[j] != CONV_OOB ? xoff[j] + (half[j] ? off[1] : off[0]) : CONV_OOB;
+            dma_b128_so(xr, base + (uint32_t)offsetof(ConvStage, A) + 1024u * (4 * wv + j), o, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            dma_b128_so(wr, base + (uint32_t)offsetof(ConvStage, B) + 1024u * (4 * wv + j), odd && half[j] ? CONV_OOB : woff[j],
+                        dsl * 64);
+        dsl += 2;
+    };
+
+    v4f acc[4][4];  // [pixel tile][channel tile]
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0, 0, 0, 0};
+    struct Frag {
+        v8h a[4], b[4];
+    };
+    auto read = [&](Frag& f, const ConvStage& st, int h) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int ra = 64 * wm + 16 * i + r16, rb = 64 * wn + 16 * i + r16;
+            f.a[i] = *reinterpret_cast<const v8h*>(&st.A[ra * 64 + (((4 * h + kg) ^ hswz(ra)) << 3)]);
+            f.b[i] = *reinterpret_cast<const v8h*>(&st.B[rb * 64 + (((4 * h + kg) ^ hswz(rb)) << 3)]);
+        }
+    };
+    auto mul = [&](const Frag& f) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.b[j], f.a[i], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    dma(lb[0]);
+    if (nst > 1) {
+        dma(lb[1]);
+        wait_vmcnt<NL>();
+    } else {
+        wait_vmcnt<0>();
     }
-    if (TAPS != 4 && ksplit > 1) {  // this split's partial sums, no bias: part [split][M][N]
+    __syncthreads();
+    Frag f0, f1;
+    read(f0, sb[0], 0);
+    for (int s = 0; s < nst; ++s) {
+        read(f1, sb[s & 1], 1);
+        mul(f0);
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): both halves are in registers (a wait the compiler sees)
+        if (s + 1 < nst) {
+            wait_vmcnt<0>();  // stage s + 1 has landed
+            asm volatile("s_barrier" ::: "memory");
+            if (s + 2 < nst) dma(lb[s & 1]);
+            read(f0, sb[(s + 1) & 1], 0);
+        }
+        mul(f1);
+    }
+
+    if (TAPS != 4 && ksplit > 1) {  // this split's partial sums, no bias: part [split][M][N] (N % 4 == 0)
         float* P = part + (int64_t)split * M * N;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int n = n0 + wn * 64 + j * 32 + lr;
-            if (n >= N) continue;
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
-                    if (m < M) P[(int64_t)m * N + n] = acc[i][j][r];
-                }
-        }
+            for (int j = 0; j < 4; ++j) {
+                const int m = m0 + 64 * wm + 16 * i + r16, n = n0 + 64 * wn + 16 * j + 4 * kg;
+                if (m < M && n < N) *reinterpret_cast<v4f*>(&P[(int64_t)m * N + n]) = acc[i][j];
+            }
         return;
     }
+    // four channels n .. n + 3 of one pixel per lane and tile: one store where the rows allow it
+    // (they lie in one tap of a conv-transpose: Cout % 4 == 0)
+    const int Cout = TAPS == 4 ? N >> 2 : N;
+    const bool v4 = Cout % 4 == 0 && (reinterpret_cast<uintptr_t>(yv) & (OH ? 7 : 15)) == 0;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int n = n0 + wn * 64 + j * 32 + lr;
+    for (int j = 0; j < 4; ++j) {
+        const int n = n0 + 64 * wn + 16 * j + 4 * kg;
         if (n >= N) continue;
-        if (TAPS == 4) {
-            const int Cout = N >> 2, t = n / Cout, co = n - t * Cout;
-            const float bv = bias[co];
+        const int t = TAPS == 4 ? n / Cout : 0, co = n - t * Cout;
+        float bv[4];
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+        for (int r = 0; r < 4; ++r) bv[r] = n + r < N ? bias[co + r] : 0.0f;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
-                    if (m >= M) continue;
-                    const int qy = m / W, qx = m - (m / W) * W;
-                    const int64_t pix = (int64_t)(2 * qy + (t >> 1)) * (2 * W) + 2 * qx + (t & 1);
-                    const float sv = acc[i][j][r] + bv;
-                    const float o = gelu ? gelu_erf(sv) : sv;
-                    if (OH) static_cast<uint16_t*>(yv)[pix * Cout + co] = f2h(o);
-                    else static_cast<float*>(yv)[pix * Cout + co] = o;
-                }
-        } else {
-            const float bv = bias[n];
+        for (int i = 0; i < 4; ++i) {
+            const int m = m0 + 64 * wm + 16 * i + r16;
+            if (m >= M) continue;
+            int64_t pix = m;
+            if (TAPS == 4) {
+                const int qy = m / W, qx = m - (m / W) * W;
+                pix = (int64_t)(2 * qy + (t >> 1)) * (2 * W) + 2 * qx + (t & 1);
+            }
+            v4f o;
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int r = 0; r < 4; ++r) {
+                const float sv = acc[i][j][r] + bv[r];
+                o[r] = TAPS == 4 && gelu ? gelu_erf(sv) : sv;
+            }
+            const int64_t at = pix * Cout + co;
+            if (v4) {
+                if (OH)
+                    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(yv) + at) =
+                        make_uint2((uint32_t)f2h(o[0]) | ((uint32_t)f2h(o[1]) << 16), (uint32_t)f2h(o[2]) | ((uint32_t)f2h(o[3]) << 16));
+                else *reinterpret_cast<v4f*>(static_cast<float*>(yv) + at) = o;
+            } else {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
-                    if (m >= M) continue;
-                    const float o = acc[i][j][r] + bv;
-                    if (OH) static_cast<uint16_t*>(yv)[(int64_t)m * N + n] = f2h(o);
-                    else static_cast<float*>(yv)[(int64_t)m * N + n] = o;
-                }
+                for (int r = 0; r < 4; ++r)
+                    if (n + r < N) {
+                        if (OH) static_cast<uint16_t*>(yv)[at + r] = f2h(o[r]);
+                        else static_cast<float*>(yv)[at + r] = o[r];
+                    }
+            }
         }
     }
 }
@@ -420,21 +471,29 @@ __global__ __launch_bounds__(256) void bias_rows_kernel(float* __restrict__ y, c
 }
 
 // ggml_pool_2d MAX, 2x2 window, stride 2, no padding: four channels per thread
-__global__ __launch_bounds__(256) void maxpool2_kernel(const float* __restrict__ x, int H, int W, int C,
-                                                       float* __restrict__ y) {
+// (F16: an fp16 map in and out)
+template <bool F16>
+__global__ __launch_bounds__(256) void maxpool2_kernel(const void* __restrict__ x, int H, int W, int C, void* __restrict__ y) {
     const int c4 = C / 4, H2 = H / 2, W2 = W / 2;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (int64_t)H2 * W2 * c4) return;
     const int c = (int)(i % c4) * 4;
     const int64_t q = i / c4;
     const int py = (int)(q / W2), px = (int)(q % W2);
-    const float* s = x + ((int64_t)(2 * py) * W + 2 * px) * C + c;
-    const v4f a = *reinterpret_cast<const v4f*>(s), b = *reinterpret_cast<const v4f*>(s + C);
-    const v4f d = *reinterpret_cast<const v4f*>(s + (int64_t)W * C), e = *reinterpret_cast<const v4f*>(s + (int64_t)W * C + C);
+    const int64_t at = ((int64_t)(2 * py) * W + 2 * px) * C + c;
+    auto load = [&](int64_t o) -> v4f {
+        if (!F16) return *reinterpret_cast<const v4f*>(static_cast<const float*>(x) + o);
+        const uint2 u = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(x) + o);
+        return v4f{h2f(u.x & 0xffff), h2f(u.x >> 16), h2f(u.y & 0xffff), h2f(u.y >> 16)};
+    };
+    const v4f a = load(at), b = load(at + C), d = load(at + (int64_t)W * C), e = load(at + (int64_t)W * C + C);
     v4f m;
 #pragma unroll
     for (int j = 0; j < 4; ++j) m[j] = fmaxf(fmaxf(a[j], b[j]), fmaxf(d[j], e[j]));
-    *reinterpret_cast<v4f*>(&y[q * C + c]) = m;
+    if (F16)
+        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(y) + q * C + c) =
+            make_uint2((uint32_t)f2h(m[0]) | ((uint32_t)f2h(m[1]) << 16), (uint32_t)f2h(m[2]) | ((uint32_t)f2h(m[3]) << 16));
+    else *reinterpret_cast<v4f*>(static_cast<float*>(y) + q * C + c) = m;
 }
 
 hipError_t launch_deconv_pack(const void* w, int wtype, int Cin, int Cout, uint16_t* out, hipStream_t st) {
@@ -471,17 +530,17 @@ hipError_t launch_conv3x3_pack_f16(const uint16_t* w, int Cin, int Cout, uint16_
     return hipGetLastError();
 }
 
-namespace {
 // operands the DMA kernel's 32-bit buffer offsets reach (with the out-of-range offset above)
-bool conv_dma_ok(int taps, int64_t M, int64_t C, int64_t N) {
+bool conv_f16_dma_fits(int taps, int64_t M, int64_t C, int64_t N) {
     return M * C * 4 < CONV_OOB - 4096 && N * (taps == 9 ? 9 : 1) * C * 2 < CONV_OOB - 4096;
 }
-// K split of the DMA kernel (taps 1 and 9): grids below one tile per CU; one 32-deep stage of
+namespace {
+// K split of the DMA kernel (taps 1 and 9): grids below one tile per CU; one 64-deep stage of
 // a tile takes about 0.9 us alone on a CU
 int conv_f16_ksplit(int taps, int64_t M, int64_t C, int64_t N) {
-    if (taps == 4 || !conv_dma_ok(taps, M, C, N)) return 1;
+    if (taps == 4 || !conv_f16_dma_fits(taps, M, C, N)) return 1;
     const int64_t tiles = ((M + CT - 1) / CT) * ((N + CT - 1) / CT);
-    return gemm_ksplit(tiles, 256, M, N, (taps == 9 ? 9 : 1) * C / 32, 0.9);
+    return gemm_ksplit(tiles, 256, M, N, ((taps == 9 ? 9 : 1) * C / 32 + 1) / 2, 0.9);
 }
 }  // namespace
 
@@ -493,43 +552,41 @@ size_t conv_f16_part_bytes(int taps, int64_t M, int64_t C, int64_t N) {
 hipError_t launch_conv_f16(int taps, const void* x, bool x16, const uint16_t* w, const float* bias, int H, int W, int C,
                            int N, bool gelu, void* y, bool y16, hipStream_t st, float* part, size_t part_bytes) {
     if ((taps != 1 && taps != 4 && taps != 9) || C % 32 != 0 || (reinterpret_cast<uintptr_t>(x) & 15) ||
-        (reinterpret_cast<uintptr_t>(w) & 15) || (taps == 4 && N % 4 != 0))
+        (reinterpret_cast<uintptr_t>(w) & 15) || (taps == 4 && N % 16 != 0))
         return hipErrorInvalidValue;
     const int64_t M = (int64_t)H * W;
     if (M <= 0 || N <= 0) return hipSuccess;
     const int tiles = (int)(((M + CT - 1) / CT) * ((N + CT - 1) / CT));
     const unsigned grid = (unsigned)((tiles + 7) / 8 * 8);
     const int gl = gelu ? 1 : 0;
-    if (conv_dma_ok(taps, M, C, N)) {
+    if (x16) {
+        if (!conv_f16_dma_fits(taps, M, C, N)) return hipErrorInvalidValue;
         // the K split, when the caller gave room for its partial sums
         // (the reduce stores float4 rows: y and part on 16 bytes; N % 4 == 0 in the split choice)
         const bool a16 = ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(part) |
                            reinterpret_cast<uintptr_t>(bias)) & 15) == 0;
         int S = part && a16 ? conv_f16_ksplit(taps, M, C, N) : 1;
         if ((size_t)S * (size_t)M * (size_t)N * 4 > part_bytes) S = 1;
-        const int nst = (taps == 9 ? 9 : 1) * C / 32, sps = (nst + S - 1) / S;
+        const int nst = ((taps == 9 ? 9 : 1) * C / 32 + 1) / 2, sps = (nst + S - 1) / S;
         const unsigned gs = (unsigned)((tiles * S + 7) / 8 * 8);
-        // the map formats the neck uses: F32 in and out (the per-op entry points), and in the
-        // fused neck fp16 intermediates (a 3x3 reads one and writes a neck output; a
-        // conv-transpose or 1x1 reads the ViT output, the pool output or one, and writes one;
-        // with F32 convolution kernels scale 0's second conv-transpose reads one, writes F32)
-        const int f = (x16 ? 2 : 0) + (y16 ? 1 : 0);
-        if (taps == 9 && f == 0) conv_f16_dma_kernel<9, CONV_NB><<<gs, 256, 0, st>>>(x, w, bias, H, W, C, N, gl, y, S, sps, part);
-        else if (taps == 9 && f == 2) conv_f16_dma_kernel<9, CONV_NB, true, false><<<gs, 256, 0, st>>>(x, w, bias, H, W, C, N, gl, y, S, sps, part);
-        else if (taps == 4 && f == 0) conv_f16_dma_kernel<4, CONV_NB><<<grid, 256, 0, st>>>(x, w, bias, H, W, C, N, gl, y, 1, nst, nullptr);
-        else if (taps == 4 && f == 1) conv_f16_dma_kernel<4, CONV_NB, false, true><<<grid, 256, 0, st>>>(x, w, bias, H, W, C, N, gl, y, 1, nst, nullptr);
-        else if (taps == 4 && f == 3) conv_f16_dma_kernel<4, CONV_NB, true, true><<<grid, 256, 0, st>>>(x, w, bias, H, W, C, N, gl, y, 1, nst, nullptr);
-        else if (taps == 4 && f == 2) conv_f16_dma_kernel<4, CONV_NB, true, false><<<grid, 256, 0, st>>>(x, w, bias, H, W, C, N, gl, y, 1, nst, nullptr);
-        else if (taps == 1 && f == 0) conv_f16_dma_kernel<1, CONV_NB><<<gs, 256, 0, st>>>(x, w, bias, H, W, C, N, gl, y, S, sps, part);
-        else if (taps == 1 && f == 1) conv_f16_dma_kernel<1, CONV_NB, false, true><<<gs, 256, 0, st>>>(x, w, bias, H, W, C, N, gl, y, S, sps, part);
-        else if (taps == 1 && f == 3) conv_f16_dma_kernel<1, CONV_NB, true, true><<<gs, 256, 0, st>>>(x, w, bias, H, W, C, N, gl, y, S, sps, part);
+        const uint16_t* xh = static_cast<const uint16_t*>(x);
+        const bool pair = C % 64 == 0;
+        auto go = [&](auto even, auto any) {
+            if (pair) even<<<gs, 256, 0, st>>>(xh, w, bias, H, W, C, N, gl, y, S, sps, part);
+            else any<<<gs, 256, 0, st>>>(xh, w, bias, H, W, C, N, gl, y, S, sps, part);
+        };
+        if (taps == 9 && !y16) go(conv_f16_dma_kernel<9, false, true>, conv_f16_dma_kernel<9, false, false>);
+        else if (taps == 4 && y16) go(conv_f16_dma_kernel<4, true, true>, conv_f16_dma_kernel<4, true, false>);
+        else if (taps == 4) go(conv_f16_dma_kernel<4, false, true>, conv_f16_dma_kernel<4, false, false>);
+        else if (taps == 1 && y16) go(conv_f16_dma_kernel<1, true, true>, conv_f16_dma_kernel<1, true, false>);
+        else if (taps == 1) go(conv_f16_dma_kernel<1, false, true>, conv_f16_dma_kernel<1, false, false>);
         else return hipErrorInvalidValue;
         const hipError_t e = hipGetLastError();
         if (S == 1 || e != hipSuccess) return e;
         return launch_split_reduce(part, S, (int)M, N, bias, static_cast<float*>(y), (y16 ? 2LL : 4LL) * N, st, y16);
     }
     // K step 32: a 64-deep step (64 KB of LDS, two workgroups per CU) measured slower
-    if (x16 || y16) return hipErrorInvalidValue;  // fp16 maps: the DMA kernel only
+    if (y16) return hipErrorInvalidValue;  // fp16 maps: the DMA kernel only
     const float* xf = static_cast<const float*>(x);
     float* yf = static_cast<float*>(y);
     if (taps == 9)
@@ -548,10 +605,11 @@ hipError_t launch_bias_rows(float* y, const float* b, int64_t rows, int C, hipSt
     return hipGetLastError();
 }
 
-hipError_t launch_maxpool2(const float* x, int H, int W, int C, float* y, hipStream_t st) {
+hipError_t launch_maxpool2(const void* x, int H, int W, int C, void* y, hipStream_t st, bool f16) {
     if (C % 4 != 0) return hipErrorInvalidValue;
     const int64_t n = (int64_t)(H / 2) * (W / 2) * (C / 4);
-    if (n > 0) maxpool2_kernel<<<nblk(n), 256, 0, st>>>(x, H, W, C, y);
+    if (n > 0 && f16) maxpool2_kernel<true><<<nblk(n), 256, 0, st>>>(x, H, W, C, y);
+    else if (n > 0) maxpool2_kernel<false><<<nblk(n), 256, 0, st>>>(x, H, W, C, y);
     return hipGetLastError();
 }
 

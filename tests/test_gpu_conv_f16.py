@@ -1,0 +1,57 @@
+"""The F16 neck kernels (fp16-MFMA implicit GEMM in 64-deep stages of two
+32-channel slices) at the edges of their tiles: odd slice counts (Cin % 64 ==
+32, where a stage crosses taps or ends half empty), one-slice maps, ragged
+pixel counts and output channels, K splits.
+
+Bound against float64 over the fp16-rounded operands: exact products, one fp32
+accumulation per 32 of K plus the K split's, each rounding by at most 2^-23 of
+S = sum |w x|, and the bias add's rounding."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(got, ref, s, b, K):
+    bound = (K // 32 + 20) * 2.0 ** -23 * s + 2.0 ** -23 * (np.abs(ref) + np.abs(b))
+    err = np.abs(got.astype(np.float64) - (ref + b))
+    assert (err <= bound).all(), float((err / bound).max())
+
+
+@pytest.mark.parametrize("H,W,Cin,Cout", [(3, 5, 32, 4), (16, 8, 64, 128), (19, 13, 96, 132), (23, 17, 160, 68), (40, 37, 224, 260),
+                                          (9, 9, 1024, 36)])
+@pytest.mark.parametrize("k", [1, 3])
+def test_conv_f16_tiles(mi, ctx, H, W, Cin, Cout, k):
+    rng = np.random.default_rng(H * W + Cin + k)
+    w = rng.standard_normal((Cout, Cin, k, k)).astype(np.float16)
+    b = rng.standard_normal(Cout).astype(np.float32)
+    x = rng.standard_normal((H, W, Cin)).astype(np.float32)
+    wd, bd, xd = torch.from_numpy(w.view(np.int16)).cuda(), torch.from_numpy(b).cuda(), torch.from_numpy(x).cuda()
+    y = torch.full((H * W, Cout), float("nan"), dtype=torch.float32, device="cuda")
+    ctx.neck_conv(mi.from_torch(wd, mi.F16, [k, k, Cin, Cout]), bd.data_ptr(), xd.data_ptr(), H, W, y.data_ptr())
+    ctx.synchronize()
+    pad = np.zeros((H + k - 1, W + k - 1, Cin))
+    pad[k // 2:k // 2 + H, k // 2:k // 2 + W] = x.astype(np.float16)
+    ref, s = np.zeros((H * W, Cout)), np.zeros((H * W, Cout))
+    for i in range(k):
+        for j in range(k):
+            a, t = pad[i:i + H, j:j + W].reshape(H * W, Cin), w[:, :, i, j].astype(np.float64)
+            ref += a @ t.T
+            s += np.abs(a) @ np.abs(t).T
+    _close(y.cpu().numpy(), ref, s, b, Cin * k * k)
+
+
+@pytest.mark.parametrize("H,W,Cin,Cout", [(3, 5, 32, 4), (16, 8, 64, 32), (13, 11, 96, 36), (21, 10, 160, 68)])
+def test_deconv_f16_tiles(mi, ctx, H, W, Cin, Cout):
+    rng = np.random.default_rng(H * W + Cin)
+    w = rng.standard_normal((Cin, Cout, 2, 2)).astype(np.float32)
+    b = rng.standard_normal(Cout).astype(np.float32)
+    x = rng.standard_normal((H * W, Cin)).astype(np.float32)
+    wd, bd, xd = torch.from_numpy(w).cuda(), torch.from_numpy(b).cuda(), torch.from_numpy(x).cuda()
+    y = torch.full((4 * H * W, Cout), float("nan"), dtype=torch.float32, device="cuda")
+    ctx.neck_deconv(mi.from_torch(wd, mi.F32, [2, 2, Cout, Cin]), bd.data_ptr(), xd.data_ptr(), H, W, False, y.data_ptr())
+    ctx.synchronize()
+    a, t = x.astype(np.float16).astype(np.float64), w.astype(np.float16).astype(np.float64).reshape(Cin, -1)
+    place = lambda v: v.reshape(H, W, Cout, 2, 2).transpose(0, 3, 1, 4, 2).reshape(4 * H * W, Cout)
+    _close(y.cpu().numpy(), place(a @ t), place(np.abs(a) @ np.abs(t)), b, Cin)
