@@ -12,7 +12,7 @@
 // acc = fma(isum, S, acc).  The Q4_1 offset term sum_b m_w s_a is a plain
 // fp16 GEMM over blocks, accumulated straight into acc by MFMA.
 //
-// F16 weights: the same tiles, acc = MFMA(a, w, acc) over k.
+// F16 weights: mmq_f16_kernel.
 //
 // Tiling: workgroup 128(m) x 128(n), four wavefronts; wavefront w owns all
 // 128 rows and the 32 columns n0+32w..+31 (4 MFMA tiles along m).  K
@@ -131,15 +131,13 @@ __device__ __forceinline__ void stage_barrier() { asm volatile("s_waitcnt lgkmcn
 // DMA still landing in the stage after next.
 template <int WT>
 struct Stage {
-    static constexpr bool QUANT = WT != T_F16;
-    static constexpr int SKH = QUANT ? BKH : 32;         // halves of K per stage (F16: 32, keeps 3 stages in LDS)
+    static constexpr int SKH = BKH;                      // halves of K per stage
     static constexpr int CH = SKH / 8;                   // 16-byte chunks per tile row
-    static constexpr int WB = WInfo<WT == T_F16 ? T_Q8_0 : WT>::bytes;
+    static constexpr int WB = WInfo<WT>::bytes;
     static constexpr int RD = (2 * WB) / 4;              // dwords of a row's 2-block stage segment
     static constexpr int RLD = (BN * RD + NT - 1) / NT;  // raw dword DMA instructions per wavefront
     _Float16 A[BM * SKH];                                // activation tile, swizzled 16-byte chunks
-    _Float16 Bf[QUANT ? 8 : BN * SKH];                   // F16 weight tile (same swizzle)
-    uint32_t W[QUANT ? RLD * NT : 4];                    // raw weight segments, lane-linear dwords
+    uint32_t W[RLD * NT];                                // raw weight segments, lane-linear dwords
     _Float16 Ad[BM][BKB];                                // activation scales of the two blocks, per row
     _Float16 As[WT == T_Q4_1 ? BM : 1][BKB];             // Q8_1 sums (Q4_1), per row
 };
@@ -160,14 +158,13 @@ struct Stage {
 template <int WT, bool DOTS, int EPI>
 __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEpi e) {
     using St = Stage<WT>;
-    constexpr bool QUANT = St::QUANT;
-    constexpr int WB = St::WB, HDR = WInfo<WT == T_F16 ? T_Q8_0 : WT>::hdr;
+    constexpr int WB = St::WB, HDR = WInfo<WT>::hdr;
     constexpr int RD = St::RD, RLD = St::RLD, SKH = St::SKH, CH = St::CH;
     constexpr int MT = BM / 32;       // m tiles per wavefront
     constexpr int RPI = 64 / CH;      // tile rows per DMA instruction
     constexpr int NI = BM / 4 / RPI;  // tile DMA instructions per wavefront
     // per-wavefront DMA instructions of one stage (plus one scale load on some wavefronts)
-    constexpr int NL = QUANT ? NI + RLD : 2 * NI;
+    constexpr int NL = NI + RLD;
     __shared__ __attribute__((aligned(16))) St st0;
     __shared__ __attribute__((aligned(16))) St st1;
     __shared__ __attribute__((aligned(16))) St st2;
@@ -194,35 +191,34 @@ __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEp
     const int k0s = split * p.sps * SKH;
     const int M = p.M, N = p.N, K = min(p.K - k0s, p.sps * SKH);
     const int nb = K / QK;
-    const int nstage = QUANT ? (nb + BKB - 1) / BKB : (K + SKH - 1) / SKH;
-    const int64_t wsh = QUANT ? (int64_t)(k0s / QK) * WB : 2LL * k0s;  // weight bytes skipped per row
+    const int nstage = (nb + BKB - 1) / BKB;
+    const int64_t wsh = (int64_t)(k0s / QK) * WB;  // weight bytes skipped per row
     const uint8_t* Wz = p.W + (int64_t)(i12 / p.r2) * p.w_nb2 + (int64_t)(i13 / p.r3) * p.w_nb3 + wsh;
     const int64_t w_extent = p.w_extent - wsh, a_extent = p.a_extent - 2LL * k0s;
     const _Float16* Az = p.A + (int64_t)i12 * p.a_s2 + (int64_t)i13 * p.a_s3 + k0s;
     const int dp = p.dp;
     const int64_t sc_extent = 2LL * M * dp - 2LL * (k0s / QK);
-    const _Float16* Adz = QUANT ? p.Ad + (int64_t)z * M * dp + k0s / QK : nullptr;
+    const _Float16* Adz = p.Ad + (int64_t)z * M * dp + k0s / QK;
     const _Float16* Asz = WT == T_Q4_1 ? p.As + (int64_t)z * M * dp + k0s / QK : nullptr;
     // wavefronts 0, 1 load the two blocks' d; for Q4_1, 2 and 3 load the two blocks' s
-    const bool xload = QUANT && (wn < 2 || WT == T_Q4_1);
+    const bool xload = wn < 2 || WT == T_Q4_1;
 
     // ---- DMA offsets, fixed for the whole K loop
-    // activation / F16-weight tile, instruction i of wavefront w: rows (NI*w+i)*RPI + lane/CH,
+    // activation tile, instruction i of wavefront w: rows (NI*w+i)*RPI + lane/CH,
     // slot lane%CH <- chunk (lane%CH) ^ (row%CH)
     const int trow = lane / CH;
-    int aoff[NI], foff[NI], tch[NI];
+    int aoff[NI], tch[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int row = (wn * NI + i) * RPI + trow;
         tch[i] = (lane % CH) ^ swz<CH>(row);
         aoff[i] = m0 + row < M ? ((m0 + row) * (int)p.a_s1 + tch[i] * 8) * 2 : OOB;
-        foff[i] = !QUANT && n0 + row < N ? (n0 + row) * (int)p.w_nb1 + tch[i] * 16 : OOB;
     }
-    int woff[QUANT ? RLD : 1];  // raw weight dword j = NT*i + 64w + lane -> (row j / RD, dword j % RD)
+    int woff[RLD];  // raw weight dword j = NT*i + 64w + lane -> (row j / RD, dword j % RD)
 #pragma unroll
-    for (int i = 0; i < (QUANT ? RLD : 1); ++i) {
+    for (int i = 0; i < RLD; ++i) {
         const int j = tid + NT * i, row = j / RD, c = j - row * RD;
-        woff[i] = QUANT && j < BN * RD && n0 + row < N ? (n0 + row) * (int)p.w_nb1 + 4 * c : OOB;
+        woff[i] = j < BN * RD && n0 + row < N ? (n0 + row) * (int)p.w_nb1 + 4 * c : OOB;
     }
 
     auto dma_stage = [&](int s, St& b) {
@@ -232,7 +228,7 @@ __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEp
 #pragma unroll
         for (int i = 0; i < NI; ++i)
             dma_b128(ar, &b.A[(wn * NI + i) * RPI * SKH], tail && k0 + tch[i] * 8 >= K ? OOB : aoff[i]);
-        if (QUANT) {
+        {
             const int64_t seg = (int64_t)s * BKB * WB;
             const auto wrs = make_rsrc(Wz + seg, w_extent - seg);
 #pragma unroll
@@ -246,11 +242,6 @@ __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEp
             } else if (WT == T_Q4_1) {
                 dma_b32(make_rsrc(Asz, sc_extent), &b.As[WT == T_Q4_1 ? 64 * (wn & 1) : 0][0], soff);
             }
-        } else {
-            const auto fr = make_rsrc(Wz + 2LL * k0, w_extent - 2LL * k0);
-#pragma unroll
-            for (int i = 0; i < NI; ++i)
-                dma_b128(fr, &b.Bf[(wn * NI + i) * RPI * SKH], tail && k0 + tch[i] * 8 >= K ? OOB : foff[i]);
         }
     };
 
@@ -269,7 +260,7 @@ __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEp
     };
 
     auto compute = [&](int s, const St& b) {
-        if (QUANT) {
+        {
             const uint32_t* rowp = &b.W[wrow * RD];
             const uint16_t* hrow = reinterpret_cast<const uint16_t*>(rowp);
             if (WT == T_Q4_1 && !DOTS) {
@@ -345,15 +336,6 @@ __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEp
                         }
                     }
                 }
-            }
-        } else {
-#pragma unroll
-            for (int kk = 0; kk < SKH / 16; ++kk) {
-                const v8h bfr = frag(b.Bf, wrow, 2 * kk + g);
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-                    acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag(b.A, mt * 32 + lr, 2 * kk + g), bfr,
-                                                                     acc[mt], 0, 0, 0);
             }
         }
     };
@@ -500,32 +482,13 @@ __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEp
         }
         stage_barrier();
         if (s + 2 < nstage) dma_stage(s + 2, refill);
-        if (QUANT && !DOTS) {
+        if (!DOTS) {
             compute_q(s, cur);
         } else {
             compute(s, cur);
         }
     };
 
-    // F16 weights, residual epilogue: the thread's sixteen residual float4 (the epilogue's rows
-    // and columns below) are loaded before the first stage's DMA, so their latency passes
-    // under the K loop instead of being paid per group of rows after it (80 VGPRs, which the
-    // quantized types' fragments leave no room for).  Issued ahead of the stage DMAs they
-    // complete before stage 0 by the in-order vmcnt, so the K loop's waits are unchanged;
-    // each element is read and later written by this thread only (in place is safe).
-    constexpr bool PRE = EPI == MMQ_EPI_RESIDUAL && WT == T_F16;
-    int rr_pre[PRE ? 16 : 1];
-    v4f xs_pre[PRE ? 16 : 1];
-    if (PRE) {
-        const int nc = n0 + 4 * (tid % (BN / 4));
-#pragma unroll
-        for (int q = 0; q < (PRE ? 16 : 1); ++q) {
-            const int m = m0 + (q >> 3) * 64 + (q & 7) * (NT / (BN / 4)) + tid / (BN / 4);
-            rr_pre[q] = m < M && nc < N ? map_row32(e.map, m) : -1;
-            xs_pre[q] = rr_pre[q] >= 0 ? *reinterpret_cast<const v4f*>(&e.res[(int64_t)rr_pre[q] * N + nc])
-                                       : v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-    }
     dma_stage(0, st0);
     if (nstage > 1) dma_stage(1, st1);
     for (int s = 0; s < nstage; s += 3) {
@@ -624,11 +587,6 @@ __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEp
                 v4f xs[4];
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    if (PRE) {
-                        rr[k] = rr_pre[PRE ? half * 8 + i0 + k : 0];
-                        xs[k] = xs_pre[PRE ? half * 8 + i0 + k : 0];
-                        continue;
-                    }
                     const int m = m0 + half * 64 + (i0 + k) * (NT / CPR) + tid / CPR;
                     rr[k] = m < M && cv ? map_row32(e.map, m) : -1;
                     xs[k] = rr[k] >= 0 ? *reinterpret_cast<const v4f*>(&e.res[(int64_t)rr[k] * N + nc])
@@ -640,6 +598,192 @@ __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEp
                     const v4f v = *reinterpret_cast<const v4f*>(&(it < IT / 2 ? t0 : t1)[(r & 31) * TP + ((4 * c + 32 * ((r >> 2) & 1)) & (BN - 1))]);
                     if (rr[k] >= 0) *reinterpret_cast<v4f*>(&e.out[(int64_t)rr[k] * N + nc]) = xs[k] + (v + bv);
                 }
+            }
+        }
+    }
+}
+
+// F16 weights: dst = MFMA(a, w) over k, fp16 operands, fp32 accumulation. Workgroup 128 x 128,
+// four wavefronts of 64 x 64, K staged 64 at a time by LDS DMA: rows of 128 bytes, whole lines,
+// which the L2 feeds to the LDS at 35 TB/s (64-byte rows at half that). Two stage buffers (64 KB:
+// two workgroups per CU). v_mfma_f32_16x16x32_f16 with the operands swapped (A = weight rows,
+// B = activation rows): a lane holds four consecutive columns of one row, so every epilogue works
+// on float4 straight from the accumulators, and at the chip's power limit this form runs faster
+// than 32 x 32 x 16 (1.89 against 1.64 PFLOP/s on random data). A half stage's fragments are read
+// while the half before it is multiplied (two register sets); the barrier lies before a stage's
+// second half, when both are in registers everywhere: the buffer then takes stage s + 2.
+// LDS rows of eight 16-byte chunks, chunk c of row r in slot c ^ (r >> 1 & 7).
+namespace {
+struct StageH {
+    _Float16 A[BM * 64];
+    _Float16 B[BN * 64];
+};
+__device__ __forceinline__ int hswz(int r) { return (r >> 1) & 7; }
+}  // namespace
+template <int EPI>
+__global__ __launch_bounds__(NT, 2) void mmq_f16_kernel(const MmqArgs p, const MmqEpi e) {
+    constexpr int NL = 8;  // DMA instructions per wavefront and stage: 4 activation, 4 weight
+    __shared__ __attribute__((aligned(16))) StageH sb[2];
+    // tile order as mmq_kernel's
+    const int TT = p.tiles_m * p.tiles_n * p.ksplit;
+    const int per_xcd = (TT + 7) / 8;
+    const int tl = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (tl >= TT) return;
+    const int t = tl / p.ksplit, split = tl - t * p.ksplit;
+    const int gsz = p.gm * p.tiles_n, grp = t / gsz, gr = t - grp * gsz;
+    const int gmr = min(p.gm, p.tiles_m - grp * p.gm);
+    const int m0 = (grp * p.gm + gr % gmr) * BM, n0 = (gr / gmr) * BN;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wv >> 1, wn = wv & 1, r16 = lane & 15, kg = lane >> 4;
+    const int z = blockIdx.y, i12 = z % p.ne12, i13 = z / p.ne12;
+    const int M = p.M, N = p.N, K = p.K;  // K % 8 == 0
+    const int s0 = split * p.sps, nst = min((K + 63) / 64 - s0, p.sps);
+    const uint8_t* Wz = p.W + (int64_t)(i12 / p.r2) * p.w_nb2 + (int64_t)(i13 / p.r3) * p.w_nb3;
+    const _Float16* Az = p.A + (int64_t)i12 * p.a_s2 + (int64_t)i13 * p.a_s3;
+
+    // DMA instruction j of wavefront wv: rows 8 (4 wv + j) + lane / 8, LDS slot lane % 8, global
+    // chunk slot ^ hswz(row); the stage is the loads' scalar offset
+    const v4i ar = make_rsrc(Az, p.a_extent), wr = make_rsrc(Wz, p.w_extent);
+    int aoff[4], woff[4], ch[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int row = 8 * (4 * wv + j) + (lane >> 3);
+        ch[j] = (lane & 7) ^ hswz(row);
+        aoff[j] = m0 + row < M ? ((m0 + row) * (int)p.a_s1 + ch[j] * 8) * 2 : OOB;
+        woff[j] = n0 + row < N ? (n0 + row) * (int)p.w_nb1 + ch[j] * 16 : OOB;
+    }
+    const uint32_t lb[2] = {(uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[0])),
+                            (uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[1]))};
+    auto dma = [&](int s, uint32_t base) __attribute__((always_inline)) {
+        const int st = s0 + s;
+        if (64 * st + 64 > K) {  // the last stage: chunks past K read zero (rows continue in memory)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (64 * st + 8 * ch[j] >= K) aoff[j] = woff[j] = OOB;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dma_b128_so(ar, base + (uint32_t)offsetof(StageH, A) + 1024u * (4 * wv + j), aoff[j], 128 * st);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dma_b128_so(wr, base + (uint32_t)offsetof(StageH, B) + 1024u * (4 * wv + j), woff[j], 128 * st);
+    };
+
+    // the lane's four columns of each column tile and four rows (one per row tile)
+    int nc[4], rr[4];
+    v4f xs[4][4];  // residual rows, loaded ahead of the first stage's DMA: their latency passes under it
+#pragma unroll
+    for (int j = 0; j < 4; ++j) nc[j] = n0 + 64 * wn + 16 * j + 4 * kg;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int m = m0 + 64 * wm + 16 * i + r16;
+        rr[i] = m < M ? (EPI == MMQ_EPI_RESIDUAL ? map_row32(e.map, m) : m) : -1;
+        if (EPI == MMQ_EPI_RESIDUAL) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                xs[i][j] = rr[i] >= 0 && nc[j] < N ? *reinterpret_cast<const v4f*>(&e.res[(int64_t)rr[i] * N + nc[j]]) : v4f{0, 0, 0, 0};
+        }
+    }
+
+    v4f acc[4][4];  // [row tile][column tile]
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0, 0, 0, 0};
+    struct Frag {
+        v8h a[4], b[4];
+    };
+    auto read = [&](Frag& f, const StageH& st, int h) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int ra = 64 * wm + 16 * i + r16, rb = 64 * wn + 16 * i + r16;
+            f.a[i] = *reinterpret_cast<const v8h*>(&st.A[ra * 64 + (((4 * h + kg) ^ hswz(ra)) << 3)]);
+            f.b[i] = *reinterpret_cast<const v8h*>(&st.B[rb * 64 + (((4 * h + kg) ^ hswz(rb)) << 3)]);
+        }
+    };
+    auto mul = [&](const Frag& f) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.b[j], f.a[i], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    dma(0, lb[0]);
+    if (nst > 1) {
+        dma(1, lb[1]);
+        wait_vmcnt<NL>();
+    } else {
+        wait_vmcnt<0>();
+    }
+    __syncthreads();
+    Frag f0, f1;
+    read(f0, sb[0], 0);
+    for (int s = 0; s < nst; ++s) {
+        read(f1, sb[s & 1], 1);
+        mul(f0);
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): both halves are in registers (a wait the compiler sees)
+        if (s + 1 < nst) {
+            wait_vmcnt<0>();  // stage s + 1 has landed
+            asm volatile("s_barrier" ::: "memory");
+            if (s + 2 < nst) dma(s + 2, lb[s & 1]);
+            read(f0, sb[(s + 1) & 1], 0);
+        }
+        mul(f1);
+    }
+
+    if (EPI == MMQ_EPI_STORE) {
+        char* Dz = reinterpret_cast<char*>(p.D) + (int64_t)i12 * p.d_nb2 + (int64_t)i13 * p.d_nb3 + split * p.d_split;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (rr[i] < 0) continue;
+            char* row = Dz + (int64_t)rr[i] * p.d_nb1;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float* d = reinterpret_cast<float*>(row) + nc[j];
+                if (p.d_v4) {
+                    if (nc[j] < N) *reinterpret_cast<v4f*>(d) = acc[i][j];
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (nc[j] + r < N) d[r] = acc[i][j][r];
+                }
+            }
+        }
+        return;
+    }
+    // u = dst + bias, each add rounded to fp32 as ggml's ADD nodes (N % 4 == 0)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if (nc[j] >= N) continue;
+        const v4f bv = *reinterpret_cast<const v4f*>(&e.bias[nc[j]]);
+        if (EPI == MMQ_EPI_RESIDUAL) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (rr[i] >= 0) *reinterpret_cast<v4f*>(&e.out[(int64_t)rr[i] * N + nc[j]]) = xs[i][j] + (acc[i][j] + bv);
+        } else {
+            const int E = e.nh * e.hd, which = nc[j] / E, col = nc[j] - which * E, hh = col / e.hd, d = col - hh * e.hd;
+            _Float16* dst = which == 0 ? e.q : which == 1 ? e.k : e.v;
+            const bool rope = which < 2 && e.rope;
+            int bw[4], tn[4];
+            v4f cs[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                bw[i] = max(rr[i], 0) / e.ntok;
+                tn[i] = max(rr[i], 0) - bw[i] * e.ntok;
+                cs[i] = rope ? *reinterpret_cast<const v4f*>(&e.rope[(int64_t)tn[i] * e.hd + d]) : v4f{1, 0, 1, 0};
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (rr[i] < 0) continue;
+                const v4f uv = acc[i][j] + bv;
+                float u0 = uv[0], u1 = uv[1], u2 = uv[2], u3 = uv[3];
+                if (rope) {
+                    rope_pair(u0, u1, cs[i][0], cs[i][1]);
+                    rope_pair(u2, u3, cs[i][2], cs[i][3]);
+                }
+                const uint32_t h0 = (uint32_t)f2h(u0) | ((uint32_t)f2h(u1) << 16);
+                const uint32_t h1 = (uint32_t)f2h(u2) | ((uint32_t)f2h(u3) << 16);
+                *reinterpret_cast<uint2*>(&dst[(((int64_t)bw[i] * e.nh + hh) * e.ntok + tn[i]) * e.hd + d]) = make_uint2(h0, h1);
             }
         }
     }
@@ -715,6 +859,15 @@ __global__ __launch_bounds__(256) void mmq_reduce_kernel(const float* __restrict
     }
 }
 
+// F16 weights
+static void launch_f16(const MmqArgs& a, int Z, const MmqEpi* e, hipStream_t st) {
+    const int TT = a.tiles_m * a.tiles_n * a.ksplit;
+    const dim3 grid((unsigned)(((TT + 7) / 8) * 8), (unsigned)Z);
+    if (a.ksplit > 1 || !e || e->kind == MMQ_EPI_STORE) mmq_f16_kernel<MMQ_EPI_STORE><<<grid, NT, 0, st>>>(a, MmqEpi{});
+    else if (e->kind == MMQ_EPI_RESIDUAL) mmq_f16_kernel<MMQ_EPI_RESIDUAL><<<grid, NT, 0, st>>>(a, *e);
+    else mmq_f16_kernel<MMQ_EPI_QKV><<<grid, NT, 0, st>>>(a, *e);
+}
+
 template <int WT>
 static void launch_t(const MmqArgs& a, int Z, bool dots, const MmqEpi* e, hipStream_t st) {
     if (a.ksplit > 1) {  // partial sums (STORE into the split buffer), then the reduction with the epilogue
@@ -759,11 +912,10 @@ int mmq_ksplit(int type, int64_t M, int64_t N, int64_t K, int64_t Z, int cus) {
     // block-quantized weights split as the int8 kernel splits them: both routes then add the
     // same K ranges in the same order and stay bit-identical
     if (type != T_F16 && K % QK == 0) return mmq8_ksplit(M, N, K, cus);
-    const bool quant = type != T_F16;
     const int64_t T = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    const int64_t nstage = quant ? ((K / QK) + BKB - 1) / BKB : (K + 31) / 32;
-    const int64_t slots = (int64_t)cus * (quant ? 2 : 3);
-    const double t_stage = quant ? 2.0 : 0.85;           // us per stage of one round of workgroups
+    const int64_t nstage = (K + 63) / 64;
+    const int64_t slots = (int64_t)cus * 2;
+    const double t_stage = 1.2;                          // us per 64-deep stage of one round of workgroups
     const double unit = (double)M * N * 4 / 4.0e6;       // us to move one M x N f32 array
     int best = 1;
     double best_cost = (double)((T + slots - 1) / slots) * nstage * t_stage;
@@ -1138,7 +1290,7 @@ static hipError_t run_mmq(const MatW& w_in, const ActF16& a, const MatD& d, int6
             }
         }
     }
-    const int nstage = w.type != T_F16 ? (int)(((a.K / QK) + BKB - 1) / BKB) : (int)((kk + 31) / 32);
+    const int nstage = w.type != T_F16 ? (int)(((a.K / QK) + BKB - 1) / BKB) : (int)((kk + 63) / 64);
     const bool split = sp.ks > 1 && !dots && ne12 * ne13 == 1;
     p.ksplit = split ? sp.ks : 1;
     p.sps = split ? (nstage + sp.ks - 1) / sp.ks : nstage;
@@ -1159,7 +1311,7 @@ static hipError_t run_mmq(const MatW& w_in, const ActF16& a, const MatD& d, int6
         case T_Q8_0: launch_t<T_Q8_0>(p, Z, dots, epi, st); break;
         case T_Q4_0: launch_t<T_Q4_0>(p, Z, dots, epi, st); break;
         case T_Q4_1: launch_t<T_Q4_1>(p, Z, dots, epi, st); break;
-        case T_F16: launch_t<T_F16>(p, Z, false, epi, st); break;
+        case T_F16: launch_f16(p, Z, epi, st); break;
         default: return hipErrorInvalidValue;
     }
     if (split) {
