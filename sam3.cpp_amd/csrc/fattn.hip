@@ -115,7 +115,11 @@ __device__ __forceinline__ uint2 lds_read_tr16(const void* a) {
 // several times more windows are in flight; the arithmetic per query is the same.
 // KDMA: fp16 K and V with 16-byte rows reach LDS by DMA (buffer_load ... lds) and the loop
 // is software-pipelined; otherwise they pass through registers.
-template <int D, bool QF32, bool KVF32, bool KDMA, int NW = 4, int NBUF = 2>
+// RESET (key-split launches): halfway through its range a workgroup takes the reference of the
+// probabilities anew from that tile's own maximum, as at the range's start, rescaling O and the
+// sums. The largest probability of each half is then exactly 1 in fp16, so one workgroup's range
+// is as precise as two ranges of half its length.
+template <int D, bool QF32, bool KVF32, bool KDMA, int NW = 4, int NBUF = 2, bool RESET = false>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fattn_kernel(const FaArgs p) {
     static_assert(!KDMA || (!KVF32 && (D == 64 || D == 96 || D == 128)), "K/V DMA staging: fp16 K and V, D = 64, 96 or 128");
     static_assert((NW == 4 && NBUF == 2) || (!KDMA && NBUF == 1 && (NW == 1 || NW == 2)), "workgroup shape");
@@ -301,7 +305,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fattn_kernel(const F
     // against the raised max, rescaling O and the sum.  Every probability is at most its
     // lane's sum, so P stays below 2^12 (fp16), and most tiles skip the max altogether.
     // The two lanes of a query pair compute the same max, so they agree on the reference.
-    auto softmax = [&](const v16f* S, uint32_t (*P)[8]) {
+    auto softmax = [&](const v16f* S, uint32_t (*P)[8], bool fresh) {
         const h2v ones = {(_Float16)1.0f, (_Float16)1.0f};
         // probabilities rounded to fp16 in pairs (the PV operand); the row sum adds the same
         // rounded values (one dot2 per pair), so numerator and denominator agree
@@ -320,7 +324,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fattn_kernel(const F
             return ls;
         };
         float ls = probs(m_run);
-        if (__builtin_amdgcn_ballot_w64(!(ls <= 4096.0f))) {
+        if ((RESET && fresh) || __builtin_amdgcn_ballot_w64(!(ls <= 4096.0f))) {
             // four independent max chains, then the pair of lanes holding the same query
             float m4[4];
 #pragma unroll
@@ -331,7 +335,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fattn_kernel(const F
                               fmaxf(fmaxf(sv[o + 4], sv[o + 5]), fmaxf(sv[o + 6], sv[o + 7])));
             }
             const float mx = xmax32(fmaxf(fmaxf(m4[0], m4[1]), fmaxf(m4[2], m4[3])));
-            const float m_new = fmaxf(m_run, mx * c);
+            float m_new = fmaxf(m_run, mx * c);
+            if (RESET && fresh && m_run - mx * c < 8.0f) m_new = mx * c;  // (a far lower maximum weighs nothing)
             const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
             m_run = m_new;
             ls = probs(m_new);
@@ -410,7 +415,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fattn_kernel(const F
             if (t + 1 < ntile) dma_v(kv0 + FA_BKV, cb ^ 1);
             if (kv0 + FA_BKV > nkv) mask(Sc, kv0);
             score(cb ^ 1, Sn);  // tile t + 1 (past the last tile: stale LDS, never used)
-            softmax(Sc, P);
+            softmax(Sc, P, RESET && t == ntile / 2);
             pv(cb, P);
         };
         for (int t = 0; t < ntile; t += 2) {
@@ -432,7 +437,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fattn_kernel(const F
             uint32_t P[2][8];
             score(cb, S);
             if (kv0 + FA_BKV > nkv) mask(S, kv0);
-            softmax(S, P);
+            softmax(S, P, RESET && t == ntile / 2);
             pv(cb, P);
             if (NBUF == 2 && t + 1 < ntile) {
                 store_tile(cb ^ 1);
@@ -521,8 +526,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fattn_kernel(const F
 
 // Key-split combine: thread per (batch, head, query, 4 outputs); m* = max of the
 // ranges' maxima, O = sum_s 2^(m_s - m*) O_s, l likewise, out = O / l.  The
-// operand output keeps 8 consecutive threads on one 32-block.
-template <int D>
+// operand output keeps 8 consecutive threads on one 32-block.  Bound by the partial outputs it
+// reads and by their latency, so the loads of all (at most KS) ranges are issued before the
+// first is used; with the ranges in a runtime loop each one's latency was paid in turn.
+template <int D, int KS>
 __global__ __launch_bounds__(256) void fattn_combine_kernel(const FaArgs p, int B) {
     constexpr int CPR = D / 4;
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -531,15 +538,30 @@ __global__ __launch_bounds__(256) void fattn_combine_kernel(const FaArgs p, int 
     const int64_t pr = t / CPR;
     const int c = (int)(t - pr * CPR);
     const int qi = (int)(pr % p.nq), h = (int)((pr / p.nq) % p.nh), b = (int)(pr / ((int64_t)p.nq * p.nh));
-    const float* ml = p.part + (int64_t)p.kv_split * rows * D;
-    float mx = -__builtin_inff();
-    for (int s = 0; s < p.kv_split; ++s) mx = fmaxf(mx, ml[(s * rows + pr) * 2]);
+    const float* ml = p.part + (int64_t)p.kv_split * rows * D + 2 * pr;
+    const float* po = p.part + pr * D + 4 * c;
+    v2f m[KS];
+    v4f v[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+        m[s] = v2f{-__builtin_inff(), 0.0f};
+        v[s] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        if (s < p.kv_split) {
+            m[s] = *reinterpret_cast<const v2f*>(&ml[2 * s * rows]);
+            v[s] = *reinterpret_cast<const v4f*>(&po[s * rows * D]);
+        }
+    }
+    float mx = m[0][0];
+#pragma unroll
+    for (int s = 1; s < KS; ++s) mx = fmaxf(mx, m[s][0]);
     float l = 0.0f;
     v4f o = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int s = 0; s < p.kv_split; ++s) {
-        const float wgt = __builtin_amdgcn_exp2f(ml[(s * rows + pr) * 2] - mx);
-        l = l + wgt * ml[(s * rows + pr) * 2 + 1];
-        o = o + wgt * *reinterpret_cast<const v4f*>(&p.part[(s * rows + pr) * D + 4 * c]);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+        if (s >= p.kv_split) break;
+        const float wgt = __builtin_amdgcn_exp2f(m[s][0] - mx);
+        l = l + wgt * m[s][1];
+        o = o + wgt * v[s];
     }
     const float inv = l == 0.0f ? 0.0f : 1.0f / l;
     o = o * inv;
@@ -555,7 +577,11 @@ int fattn_kv_split(int nq, int nkv, int nh, int B, int cus) {
     // below eight key tiles the combine pass costs more than the idle CUs (Hiera-tiny's 14x14
     // windows, 4 tiles over 200 workgroups: 12.2 us split in two + 7 us combine, against one pass)
     if (cus <= 0 || wgs >= cus || ntile < 8) return 1;
-    const int64_t want = (2LL * cus + wgs - 1) / wgs;
+    // small grids: about one workgroup per CU and not a few more, since each range costs a pass
+    // over the outputs twice (1 x 4 heads, 1021 x 3999 of 96: 33.8 us in 16 ranges, 26.5 in 8;
+    // 8 heads, 1024 x 1024 of 96: 26.0 in 8, 19.7 in 4; 16 heads, 300 x 5184 of 128: 58.2 in 11,
+    // 40.5 in 5); from a third of the CUs on, two per CU (4 heads, 4096 x 4096 of 96)
+    const int64_t want = wgs * 3 <= cus ? cus / wgs : (2LL * cus + wgs - 1) / wgs;
     const int ks = (int)std::min<int64_t>(want, ntile / 2);
     return ks < 2 ? 1 : std::min(ks, 16);
 }
@@ -570,6 +596,10 @@ static void fa_launch_d(const FaArgs& a, bool qf32, bool kvf32, int B, hipStream
     const int64_t items = (int64_t)((a.nq + FA_BQ - 1) / FA_BQ) * a.nh * B * a.kv_split;
     const dim3 grid((unsigned)((items + 7) / 8 * 8));
     bool launched = false;
+    auto go = [&](auto whole, auto range) {
+        if (a.kv_split > 1) range<<<grid, FA_NT, 0, st>>>(a);
+        else whole<<<grid, FA_NT, 0, st>>>(a);
+    };
     // windows of at most one key tile and 64 queries, fp16 operands, no key split: one or two
     // wavefronts per workgroup and one K/V buffer (taken before the DMA path, which would
     // give such a window four wavefronts and two buffers)
@@ -589,19 +619,23 @@ static void fa_launch_d(const FaArgs& a, bool qf32, bool kvf32, int B, hipStream
                           reinterpret_cast<uintptr_t>(a.v) % 16 == 0 && a.v_nb1 % 16 == 0 && a.v_nb2 % 16 == 0 &&
                           a.v_nb3 % 16 == 0 && (int64_t)(a.nkv + FA_BKV) * a.v_nb1 < INT32_MAX;
         if (!launched && kdma) {
-            if (qf32) fattn_kernel<D, true, false, true><<<grid, FA_NT, 0, st>>>(a);
-            else fattn_kernel<D, false, false, true><<<grid, FA_NT, 0, st>>>(a);
+            if (qf32) go(fattn_kernel<D, true, false, true>, fattn_kernel<D, true, false, true, 4, 2, true>);
+            else go(fattn_kernel<D, false, false, true>, fattn_kernel<D, false, false, true, 4, 2, true>);
             launched = true;
         }
     }
     if (launched) {
-    } else if (qf32 && kvf32) fattn_kernel<D, true, true, false><<<grid, FA_NT, 0, st>>>(a);
-    else if (qf32) fattn_kernel<D, true, false, false><<<grid, FA_NT, 0, st>>>(a);
-    else if (kvf32) fattn_kernel<D, false, true, false><<<grid, FA_NT, 0, st>>>(a);
-    else fattn_kernel<D, false, false, false><<<grid, FA_NT, 0, st>>>(a);
+    } else if (qf32 && kvf32) go(fattn_kernel<D, true, true, false>, fattn_kernel<D, true, true, false, 4, 2, true>);
+    else if (qf32) go(fattn_kernel<D, true, false, false>, fattn_kernel<D, true, false, false, 4, 2, true>);
+    else if (kvf32) go(fattn_kernel<D, false, true, false>, fattn_kernel<D, false, true, false, 4, 2, true>);
+    else go(fattn_kernel<D, false, false, false>, fattn_kernel<D, false, false, false, 4, 2, true>);
     if (a.kv_split > 1) {
         const int64_t n = (int64_t)B * a.nh * a.nq * (D / 4);
-        fattn_combine_kernel<D><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(a, B);
+        const unsigned g = (unsigned)((n + 255) / 256);
+        if (a.kv_split <= 2) fattn_combine_kernel<D, 2><<<g, 256, 0, st>>>(a, B);
+        else if (a.kv_split <= 4) fattn_combine_kernel<D, 4><<<g, 256, 0, st>>>(a, B);
+        else if (a.kv_split <= 8) fattn_combine_kernel<D, 8><<<g, 256, 0, st>>>(a, B);
+        else fattn_combine_kernel<D, 16><<<g, 256, 0, st>>>(a, B);
     }
 }
 
@@ -611,7 +645,7 @@ hipError_t launch_fattn(const FaArgs& a_in, int D, bool qf32, bool kvf32, int B,
         return hipErrorInvalidValue;
     FaArgs a = a_in;
     a.B = B;
-    if (a.kv_split < 1 || (a.kv_split > 1 && (!a.part || a.kv_chunk % FA_BKV != 0 ||
+    if (a.kv_split < 1 || a.kv_split > 16 || (a.kv_split > 1 && (!a.part || a.kv_chunk % FA_BKV != 0 ||
                                               (int64_t)(a.kv_split - 1) * a.kv_chunk >= a.nkv)))
         return hipErrorInvalidValue;
     switch (D) {
