@@ -372,7 +372,8 @@ hipError_t launch_conv3x3_pack_f16(const uint16_t* w, int Cin, int Cout, uint16_
 // into ranges whose partial sums go to part [split][M][N] (at most part_bytes; none without
 // part) and are added, with the bias, by launch_split_reduce.
 // x16: the map is fp16 (the f32 values rounded RNE), for the DMA kernel (conv_f16_dma_fits); an F32
-// map takes the register-staged kernel, which rounds it as it loads. y16: the output too (x16 only).
+// map takes the 1x1's own DMA kernel or the register-staged one, which round it as they load.
+// y16: the output too (x16 only).
 hipError_t launch_conv_f16(int taps, const void* x, bool x16, const uint16_t* w, const float* bias, int H, int W, int C,
                            int N, bool gelu, void* y, bool y16, hipStream_t st, float* part = nullptr,
                            size_t part_bytes = 0);

@@ -638,7 +638,8 @@ __global__ __launch_bounds__(NT, 2) void mmq_f16_kernel(const MmqArgs p, const M
     const int wm = wv >> 1, wn = wv & 1, r16 = lane & 15, kg = lane >> 4;
     const int z = blockIdx.y, i12 = z % p.ne12, i13 = z / p.ne12;
     const int M = p.M, N = p.N, K = p.K;  // K % 8 == 0
-    const int s0 = split * p.sps, nst = min((K + 63) / 64 - s0, p.sps);
+    // the K split's ranges are whole 32-deep units (p.sps of them)
+    const int kb = split * p.sps * 32, ke = min(K, kb + p.sps * 32), nst = (ke - kb + 63) / 64;
     const uint8_t* Wz = p.W + (int64_t)(i12 / p.r2) * p.w_nb2 + (int64_t)(i13 / p.r3) * p.w_nb3;
     const _Float16* Az = p.A + (int64_t)i12 * p.a_s2 + (int64_t)i13 * p.a_s3;
 
@@ -656,16 +657,16 @@ __global__ __launch_bounds__(NT, 2) void mmq_f16_kernel(const MmqArgs p, const M
     const uint32_t lb[2] = {(uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[0])),
                             (uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[1]))};
     auto dma = [&](int s, uint32_t base) __attribute__((always_inline)) {
-        const int st = s0 + s;
-        if (64 * st + 64 > K) {  // the last stage: chunks past K read zero (rows continue in memory)
+        const int k0 = kb + 64 * s;
+        if (k0 + 64 > ke) {  // the last stage: chunks past the range read zero (rows continue in memory)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                if (64 * st + 8 * ch[j] >= K) aoff[j] = woff[j] = OOB;
+                if (k0 + 8 * ch[j] >= ke) aoff[j] = woff[j] = OOB;
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) dma_b128_so(ar, base + (uint32_t)offsetof(StageH, A) + 1024u * (4 * wv + j), aoff[j], 128 * st);
+        for (int j = 0; j < 4; ++j) dma_b128_so(ar, base + (uint32_t)offsetof(StageH, A) + 1024u * (4 * wv + j), aoff[j], 2 * k0);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) dma_b128_so(wr, base + (uint32_t)offsetof(StageH, B) + 1024u * (4 * wv + j), woff[j], 128 * st);
+        for (int j = 0; j < 4; ++j) dma_b128_so(wr, base + (uint32_t)offsetof(StageH, B) + 1024u * (4 * wv + j), woff[j], 2 * k0);
     };
 
     // the lane's four columns of each column tile and four rows (one per row tile)
@@ -913,9 +914,9 @@ int mmq_ksplit(int type, int64_t M, int64_t N, int64_t K, int64_t Z, int cus) {
     // same K ranges in the same order and stay bit-identical
     if (type != T_F16 && K % QK == 0) return mmq8_ksplit(M, N, K, cus);
     const int64_t T = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    const int64_t nstage = (K + 63) / 64;
-    const int64_t slots = (int64_t)cus * 2;
-    const double t_stage = 1.2;                          // us per 64-deep stage of one round of workgroups
+    const int64_t nstage = (K + 31) / 32;
+    const int64_t slots = (int64_t)cus * 3;
+    const double t_stage = 0.85;                         // us per 32-deep unit of one round of workgroups
     const double unit = (double)M * N * 4 / 4.0e6;       // us to move one M x N f32 array
     int best = 1;
     double best_cost = (double)((T + slots - 1) / slots) * nstage * t_stage;
@@ -1290,7 +1291,7 @@ static hipError_t run_mmq(const MatW& w_in, const ActF16& a, const MatD& d, int6
             }
         }
     }
-    const int nstage = w.type != T_F16 ? (int)(((a.K / QK) + BKB - 1) / BKB) : (int)((kk + 63) / 64);
+    const int nstage = w.type != T_F16 ? (int)(((a.K / QK) + BKB - 1) / BKB) : (int)((kk + 31) / 32);
     const bool split = sp.ks > 1 && !dots && ne12 * ne13 == 1;
     p.ksplit = split ? sp.ks : 1;
     p.sps = split ? (nstage + sp.ks - 1) / sp.ks : nstage;

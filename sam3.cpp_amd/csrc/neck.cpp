@@ -208,7 +208,8 @@ mi355_status conv(mi355_context* ctx, const mi355_tensor* w, const float* b, con
         // the fp16 map and the K split's partial sums follow the repacked kernel
         char* next = scratch + (k == 3 ? align_up((size_t)(K * Cout * 2)) : 0);
         const void* xm = x;
-        if (!x16 && conv_f16_dma_fits(k * k, P, Cin, Cout)) {
+        // (an F32 map under a 1x1 with an F32 output is rounded by its own kernel)
+        if (!x16 && (k == 3 || y16) && conv_f16_dma_fits(k * k, P, Cin, Cout)) {
             st = half_map(ctx, x, P, Cin, next);
             if (st != MI355_STATUS_SUCCESS) return st;
             xm = next;

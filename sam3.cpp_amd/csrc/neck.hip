@@ -268,14 +268,14 @@ __global__ __launch_bounds__(256, 2) void conv_f16_dma_kernel(const uint16_t* __
     const int wm = wv >> 1, wn = wv & 1;
     const int r16 = lane & 15, kg = lane >> 4;
     // XCD-aware tile order (each XCD a contiguous band of tiles); with a K split (taps 1 and
-    // 9) the split is the slowest index: slot (split, tile) runs stages [split * sps, + sps)
+    // 9) the split is the slowest index: slot (split, tile) runs slices [split * sps, + sps)
     const int tiles_n = (N + CT - 1) / CT, tiles = ((M + CT - 1) / CT) * tiles_n;
     const int TT = tiles * ksplit, per_xcd = (TT + 7) / 8;
     const int tls = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if (tls >= TT) return;
     const int split = tls / tiles, tl = tls - split * tiles;
     const int m0 = (tl / tiles_n) * CT, n0 = (tl % tiles_n) * CT;
-    const int s0 = split * sps, nst = min((nsl + 1) / 2 - s0, sps);  // this split's first stage and stage count
+    const int sl0 = split * sps, sl1 = min(nsl, sl0 + sps), nst = (sl1 - sl0 + 1) / 2;  // this split's slices, stages
 
     // DMA instruction j moves rows 8 (4 wv + j) + lane / 8: LDS slot lane % 8, global chunk
     // slot ^ hswz(row), slice chunk / 4. Per lane the byte offset of its chunk within the slice at
@@ -299,7 +299,7 @@ __global__ __launch_bounds__(256, 2) void conv_f16_dma_kernel(const uint16_t* __
     const uint32_t lb[2] = {(uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[0])),
                             (uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[1]))};
     // the next stage to load, in order: its first slice, that slice's tap and channel slice
-    int dsl = 2 * s0, dtap = TAPS == 9 ? dsl / cps : 0, dcs = dsl - dtap * cps;
+    int dsl = sl0, dtap = TAPS == 9 ? dsl / cps : 0, dcs = dsl - dtap * cps;
     int voff[4];  // PAIR: the lanes' map offsets of tap dtap
     auto at_tap = [&]() __attribute__((always_inline)) {
         const int off = TAPS == 9 ? ((dtap / 3 - 1) * W + dtap % 3 - 1) * C * 2 : 0;
@@ -340,7 +340,7 @@ __global__ __launch_bounds__(256, 2) void conv_f16_dma_kernel(const uint16_t* __
                 ++dcs;
             }
         }
-        const bool odd = dsl + 1 >= nsl;  // no second slice (the last stage of an odd count)
+        const bool odd = dsl + 1 >= sl1;  // no second slice (the last stage of an odd count)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const bool in = !(odd && half[j]) && (TAPS != 9 || ((tmask[j] >> (half[j] ? tap[1] : tap[0])) & 1));
@@ -458,6 +458,112 @@ __global__ __launch_bounds__(256, 2) void conv_f16_dma_kernel(const uint16_t* __
     }
 }
 
+// The 1x1 over an F32 map: the same GEMM with the map staged as it is (128 bytes per pixel and
+// 32-deep stage) and rounded to fp16 (RNE, f2h) as the fragments are read, so no pass over the map
+// goes before it: 288 x 288, 256 -> 256 channels 41 us, against 25 for that pass and 30 for
+// conv_f16_dma_kernel. The same operands, products and order over K: the same bits.
+// Map rows of 8 chunks of 16 bytes, chunk c of row r in slot c ^ (r >> 1 & 7); weight rows of
+// four, csw<4>.
+namespace {
+struct Conv1Stage {
+    float A[CT * 32];     // 128 map rows x 32 channels, fp32
+    uint16_t B[CT * 32];  // 128 weight rows x 32 K, fp16
+};
+}  // namespace
+__global__ __launch_bounds__(256, 3) void conv1x1_f32map_kernel(const float* __restrict__ x, const uint16_t* __restrict__ w,
+                                                                const float* __restrict__ bias, int M, int C, int N,
+                                                                float* __restrict__ y, int ksplit, int sps,
+                                                                float* __restrict__ part) {
+    __shared__ __attribute__((aligned(16))) Conv1Stage sb[2];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wv & 1, wn = wv >> 1;
+    const int lr = lane & 31, g = lane >> 5;
+    const int tiles_n = (N + CT - 1) / CT, tiles = ((M + CT - 1) / CT) * tiles_n;
+    const int TT = tiles * ksplit, per_xcd = (TT + 7) / 8;
+    const int tls = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (tls >= TT) return;
+    const int split = tls / tiles, tl = tls - split * tiles;
+    const int m0 = (tl / tiles_n) * CT, n0 = (tl % tiles_n) * CT;
+    const int s0 = split * sps, nst = min(C / 32 - s0, sps);
+    // map DMA instruction j of wavefront wv: rows 8 (4 wv + j) + lane / 8; weights: rows
+    // 16 (2 wv + j) + lane / 4; the stage is the loads' scalar offset
+    const v4i xr = make_rsrc(x, (int64_t)M * C * 4), wr = make_rsrc(w, (int64_t)N * C * 2);
+    int xoff[4], woff[2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int row = 8 * (4 * wv + j) + (lane >> 3), p = m0 + row;
+        xoff[j] = p < M ? p * C * 4 + (((lane & 7) ^ hswz(row)) << 4) : CONV_OOB;
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int row = 16 * (2 * wv + j) + (lane >> 2), n = n0 + row;
+        woff[j] = n < N ? n * C * 2 + (((lane & 3) ^ csw<4>(row)) << 4) : CONV_OOB;
+    }
+    const uint32_t lb[2] = {(uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[0])),
+                            (uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[1]))};
+    auto dma = [&](int s, uint32_t base) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            dma_b128_so(xr, base + (uint32_t)offsetof(Conv1Stage, A) + 1024u * (4 * wv + j), xoff[j], s * 128);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            dma_b128_so(wr, base + (uint32_t)offsetof(Conv1Stage, B) + 1024u * (2 * wv + j), woff[j], s * 64);
+    };
+    const v16f zf = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    v16f acc[2][2] = {{zf, zf}, {zf, zf}};
+    auto compute = [&](const Conv1Stage& b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            v8h a[2], bf[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int ra = wm * 64 + i * 32 + lr, rb = wn * 64 + i * 32 + lr, c = 4 * kk + 2 * g;
+                const v4f lo = *reinterpret_cast<const v4f*>(&b.A[ra * 32 + ((c ^ hswz(ra)) << 2)]);
+                const v4f hi = *reinterpret_cast<const v4f*>(&b.A[ra * 32 + (((c + 1) ^ hswz(ra)) << 2)]);
+                const uint4 q = {(uint32_t)f2h(lo[0]) | ((uint32_t)f2h(lo[1]) << 16), (uint32_t)f2h(lo[2]) | ((uint32_t)f2h(lo[3]) << 16),
+                                 (uint32_t)f2h(hi[0]) | ((uint32_t)f2h(hi[1]) << 16), (uint32_t)f2h(hi[2]) | ((uint32_t)f2h(hi[3]) << 16)};
+                a[i] = __builtin_bit_cast(v8h, q);
+                bf[i] = *reinterpret_cast<const v8h*>(&b.B[rb * 32 + (((2 * kk + g) ^ csw<4>(rb)) << 3)]);
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], bf[j], acc[i][j], 0, 0, 0);
+        }
+    };
+    dma(s0, lb[0]);
+    if (nst > 1) {
+        dma(s0 + 1, lb[1]);
+        wait_vmcnt<6>();
+    } else {
+        wait_vmcnt<0>();
+    }
+    __syncthreads();
+    for (int s = 0; s < nst; ++s) {
+        compute(sb[s & 1]);
+        if (s + 1 < nst) {
+            wait_vmcnt<0>();  // stage s + 1 has landed
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // and stage s's buffer is read
+            if (s + 2 < nst) dma(s0 + s + 2, lb[s & 1]);
+        }
+    }
+    float* D = ksplit > 1 ? part + (int64_t)split * M * N : y;  // a split's partial sums, no bias
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int n = n0 + wn * 64 + j * 32 + lr;
+        if (n >= N) continue;
+        const float bv = ksplit > 1 ? 0.0f : bias[n];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
+                if (m < M) D[(int64_t)m * N + n] = ksplit > 1 ? acc[i][j][r] : acc[i][j][r] + bv;
+            }
+    }
+}
+
 // y[r][c] += b[c], four channels per thread (C % 4 == 0)
 __global__ __launch_bounds__(256) void bias_rows_kernel(float* __restrict__ y, const float* __restrict__ b, int64_t rows,
                                                         int C) {
@@ -535,17 +641,24 @@ bool conv_f16_dma_fits(int taps, int64_t M, int64_t C, int64_t N) {
     return M * C * 4 < CONV_OOB - 4096 && N * (taps == 9 ? 9 : 1) * C * 2 < CONV_OOB - 4096;
 }
 namespace {
-// K split of the DMA kernel (taps 1 and 9): grids below one tile per CU; one 64-deep stage of
-// a tile takes about 0.9 us alone on a CU
-int conv_f16_ksplit(int taps, int64_t M, int64_t C, int64_t N) {
+// K split of the DMA kernel (taps 1 and 9), in 32-deep slices: grids below one tile per CU; a
+// slice of a tile counts 0.9 us. Ranges of an odd number of slices get one more where C % 64 == 0,
+// so that every stage's two slices lie in one tap.
+int conv_f16_ksplit(int taps, int64_t M, int64_t C, int64_t N, int64_t* sps) {
+    const int64_t nsl = (taps == 9 ? 9 : 1) * C / 32;
+    *sps = nsl;
     if (taps == 4 || !conv_f16_dma_fits(taps, M, C, N)) return 1;
     const int64_t tiles = ((M + CT - 1) / CT) * ((N + CT - 1) / CT);
-    return gemm_ksplit(tiles, 256, M, N, ((taps == 9 ? 9 : 1) * C / 32 + 1) / 2, 0.9);
+    const int S = gemm_ksplit(tiles, 256, M, N, nsl, 0.9);
+    *sps = (nsl + S - 1) / S;
+    if (S > 1 && C % 64 == 0) *sps += *sps & 1;
+    return (int)((nsl + *sps - 1) / *sps);
 }
 }  // namespace
 
 size_t conv_f16_part_bytes(int taps, int64_t M, int64_t C, int64_t N) {
-    const int S = conv_f16_ksplit(taps, M, C, N);
+    int64_t sps;
+    const int S = conv_f16_ksplit(taps, M, C, N, &sps);
     return S > 1 ? (size_t)S * (size_t)M * (size_t)N * 4 : 0;
 }
 
@@ -559,15 +672,17 @@ hipError_t launch_conv_f16(int taps, const void* x, bool x16, const uint16_t* w,
     const int tiles = (int)(((M + CT - 1) / CT) * ((N + CT - 1) / CT));
     const unsigned grid = (unsigned)((tiles + 7) / 8 * 8);
     const int gl = gelu ? 1 : 0;
-    if (x16) {
-        if (!conv_f16_dma_fits(taps, M, C, N)) return hipErrorInvalidValue;
+    if (x16 && !conv_f16_dma_fits(taps, M, C, N)) return hipErrorInvalidValue;
+    const bool map32 = taps == 1 && !x16 && !y16 && conv_f16_dma_fits(taps, M, C, N);
+    if (x16 || map32) {
         // the K split, when the caller gave room for its partial sums
         // (the reduce stores float4 rows: y and part on 16 bytes; N % 4 == 0 in the split choice)
         const bool a16 = ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(part) |
                            reinterpret_cast<uintptr_t>(bias)) & 15) == 0;
-        int S = part && a16 ? conv_f16_ksplit(taps, M, C, N) : 1;
-        if ((size_t)S * (size_t)M * (size_t)N * 4 > part_bytes) S = 1;
-        const int nst = ((taps == 9 ? 9 : 1) * C / 32 + 1) / 2, sps = (nst + S - 1) / S;
+        int64_t sps64;
+        int S = conv_f16_ksplit(taps, M, C, N, &sps64);
+        if (!part || !a16 || (size_t)S * (size_t)M * (size_t)N * 4 > part_bytes) S = 1;
+        const int sps = S > 1 ? (int)sps64 : (taps == 9 ? 9 : 1) * C / 32;
         const unsigned gs = (unsigned)((tiles * S + 7) / 8 * 8);
         const uint16_t* xh = static_cast<const uint16_t*>(x);
         const bool pair = C % 64 == 0;
@@ -575,7 +690,8 @@ hipError_t launch_conv_f16(int taps, const void* x, bool x16, const uint16_t* w,
             if (pair) even<<<gs, 256, 0, st>>>(xh, w, bias, H, W, C, N, gl, y, S, sps, part);
             else any<<<gs, 256, 0, st>>>(xh, w, bias, H, W, C, N, gl, y, S, sps, part);
         };
-        if (taps == 9 && !y16) go(conv_f16_dma_kernel<9, false, true>, conv_f16_dma_kernel<9, false, false>);
+        if (map32) conv1x1_f32map_kernel<<<gs, 256, 0, st>>>(static_cast<const float*>(x), w, bias, (int)M, C, N, static_cast<float*>(y), S, sps, part);
+        else if (taps == 9 && !y16) go(conv_f16_dma_kernel<9, false, true>, conv_f16_dma_kernel<9, false, false>);
         else if (taps == 4 && y16) go(conv_f16_dma_kernel<4, true, true>, conv_f16_dma_kernel<4, true, false>);
         else if (taps == 4) go(conv_f16_dma_kernel<4, false, true>, conv_f16_dma_kernel<4, false, false>);
         else if (taps == 1 && y16) go(conv_f16_dma_kernel<1, true, true>, conv_f16_dma_kernel<1, true, false>);
