@@ -141,6 +141,11 @@ __device__ __forceinline__ double lane_swap_d(double v) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
+// LDS staging of the results of swapped 16 x 16 MFMAs (a lane holds four consecutive columns of
+// one row) in rows of 64 floats: 4-float chunk c of row r in slot c ^ (r & 15), so the sixteen
+// rows of one write and the sixteen chunks (or 64 columns) of one row's read cover the 64 banks.
+__device__ __forceinline__ int row64_chunk(int r, int c) { return 64 * r + 4 * ((c & 15) ^ (r & 15)); }
+
 // LDS staging of a 32x32 fp32 MFMA tile in 1024 floats: rows 2k and 2k + 1 share the 64
 // floats (one line of the 64 4-byte banks) at 64 k, row r in half (r ^ r >> 2) & 1, so a write
 // of one accumulator element (lanes 0..31 row R, lanes 32..63 row R + 4) and each 16-lane

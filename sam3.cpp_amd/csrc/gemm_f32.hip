@@ -758,6 +758,41 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const GemmF32Arg
     const int64_t pitch = parts ? 4LL * N : p.d_nb1;
     const float* add = parts ? nullptr : p.add;
     const bool v4 = N % 4 == 0 && ((reinterpret_cast<uintptr_t>(D) | (uintptr_t)pitch | reinterpret_cast<uintptr_t>(add)) & 15) == 0;
+    if (!v4) {
+        // rows that are no multiple of four, or unaligned: through the wavefront's 16 KB of the stage
+        // buffers (rows of 128 columns as two of 64), 64 columns of a row per store
+        __syncthreads();  // every wavefront has read its last fragments
+        float* t = reinterpret_cast<float*>(sb) + 4096 * wv;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                *reinterpret_cast<v4f*>(&t[row64_chunk(2 * (16 * i + r16) + (j >> 2), 4 * j + kg)]) = acc[i][j];
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int n = n0 + 64 * h + lane;
+            const float bn = !parts && p.bias && n < N ? p.bias[n] : 0.0f;
+            for (int r0 = 0; r0 < 32; r0 += 8) {
+                float v[8], a[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const int m = m0 + 32 * wv + r0 + k;
+                    v[k] = t[row64_chunk(2 * (r0 + k) + h, lane >> 2) + (lane & 3)];
+                    a[k] = add && m < M && n < N ? add[(int64_t)m * N + n] : 0.0f;
+                }
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const int m = m0 + 32 * wv + r0 + k;
+                    float o = parts ? v[k] : v[k] + bn;
+                    if (add) o = o + a[k];
+                    if (m < M && n < N) *(reinterpret_cast<float*>(D + (int64_t)m * pitch) + n) = o;
+                }
+            }
+        }
+        return;
+    }
     v4f ad[2][8];
     if (add) {
 #pragma unroll
@@ -765,21 +800,16 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const GemmF32Arg
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const int m = m0 + 32 * wv + 16 * i + r16, n = n0 + 16 * j + 4 * kg;
-                const float* src = add + (int64_t)m * N + n;
-                if (v4 && m < M && n < N) {
-                    ad[i][j] = *reinterpret_cast<const v4f*>(src);
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) ad[i][j][r] = m < M && n + r < N ? src[r] : 0.0f;
-                }
+                ad[i][j] = m < M && n < N ? *reinterpret_cast<const v4f*>(add + (int64_t)m * N + n) : v4f{0, 0, 0, 0};
             }
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int n = n0 + 16 * j + 4 * kg;
+        if (n >= N) continue;
         float bn[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) bn[r] = !parts && p.bias && n + r < N ? p.bias[n + r] : 0.0f;
+        for (int r = 0; r < 4; ++r) bn[r] = !parts && p.bias ? p.bias[n + r] : 0.0f;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int m = m0 + 32 * wv + 16 * i + r16;
@@ -789,18 +819,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const GemmF32Arg
 #pragma unroll
                 for (int r = 0; r < 4; ++r) v[r] = v[r] + bn[r];
             }
-            if (add) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] = v[r] + ad[i][j][r];
-            }
-            float* d = reinterpret_cast<float*>(D + (int64_t)m * pitch) + n;
-            if (v4) {
-                if (n < N) *reinterpret_cast<v4f*>(d) = v;
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (n + r < N) d[r] = v[r];
-            }
+            if (add) v = v + ad[i][j];
+            *reinterpret_cast<v4f*>(reinterpret_cast<float*>(D + (int64_t)m * pitch) + n) = v;
         }
     }
 }

@@ -12,7 +12,8 @@
 // acc = fma(isum, S, acc).  The Q4_1 offset term sum_b m_w s_a is a plain
 // fp16 GEMM over blocks, accumulated straight into acc by MFMA.
 //
-// F16 weights: mmq_f16_kernel.
+// F16 weights with a short K: the same tiles, acc = MFMA(a, w, acc) over k; longer K and the fused
+// epilogues: mmq_f16_kernel.
 //
 // Tiling: workgroup 128(m) x 128(n), four wavefronts; wavefront w owns all
 // 128 rows and the 32 columns n0+32w..+31 (4 MFMA tiles along m).  K
@@ -131,13 +132,15 @@ __device__ __forceinline__ void stage_barrier() { asm volatile("s_waitcnt lgkmcn
 // DMA still landing in the stage after next.
 template <int WT>
 struct Stage {
-    static constexpr int SKH = BKH;                      // halves of K per stage
+    static constexpr bool QUANT = WT != T_F16;
+    static constexpr int SKH = QUANT ? BKH : 32;         // halves of K per stage (F16: 32, keeps 3 stages in LDS)
     static constexpr int CH = SKH / 8;                   // 16-byte chunks per tile row
-    static constexpr int WB = WInfo<WT>::bytes;
+    static constexpr int WB = WInfo<WT == T_F16 ? T_Q8_0 : WT>::bytes;
     static constexpr int RD = (2 * WB) / 4;              // dwords of a row's 2-block stage segment
     static constexpr int RLD = (BN * RD + NT - 1) / NT;  // raw dword DMA instructions per wavefront
     _Float16 A[BM * SKH];                                // activation tile, swizzled 16-byte chunks
-    uint32_t W[RLD * NT];                                // raw weight segments, lane-linear dwords
+    _Float16 Bf[QUANT ? 8 : BN * SKH];                   // F16 weight tile (same swizzle)
+    uint32_t W[QUANT ? RLD * NT : 4];                    // raw weight segments, lane-linear dwords
     _Float16 Ad[BM][BKB];                                // activation scales of the two blocks, per row
     _Float16 As[WT == T_Q4_1 ? BM : 1][BKB];             // Q8_1 sums (Q4_1), per row
 };
@@ -158,13 +161,14 @@ struct Stage {
 template <int WT, bool DOTS, int EPI>
 __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEpi e) {
     using St = Stage<WT>;
-    constexpr int WB = St::WB, HDR = WInfo<WT>::hdr;
+    constexpr bool QUANT = St::QUANT;
+    constexpr int WB = St::WB, HDR = WInfo<WT == T_F16 ? T_Q8_0 : WT>::hdr;
     constexpr int RD = St::RD, RLD = St::RLD, SKH = St::SKH, CH = St::CH;
     constexpr int MT = BM / 32;       // m tiles per wavefront
     constexpr int RPI = 64 / CH;      // tile rows per DMA instruction
     constexpr int NI = BM / 4 / RPI;  // tile DMA instructions per wavefront
     // per-wavefront DMA instructions of one stage (plus one scale load on some wavefronts)
-    constexpr int NL = NI + RLD;
+    constexpr int NL = QUANT ? NI + RLD : 2 * NI;
     __shared__ __attribute__((aligned(16))) St st0;
     __shared__ __attribute__((aligned(16))) St st1;
     __shared__ __attribute__((aligned(16))) St st2;
@@ -191,34 +195,35 @@ __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEp
     const int k0s = split * p.sps * SKH;
     const int M = p.M, N = p.N, K = min(p.K - k0s, p.sps * SKH);
     const int nb = K / QK;
-    const int nstage = (nb + BKB - 1) / BKB;
-    const int64_t wsh = (int64_t)(k0s / QK) * WB;  // weight bytes skipped per row
+    const int nstage = QUANT ? (nb + BKB - 1) / BKB : (K + SKH - 1) / SKH;
+    const int64_t wsh = QUANT ? (int64_t)(k0s / QK) * WB : 2LL * k0s;  // weight bytes skipped per row
     const uint8_t* Wz = p.W + (int64_t)(i12 / p.r2) * p.w_nb2 + (int64_t)(i13 / p.r3) * p.w_nb3 + wsh;
     const int64_t w_extent = p.w_extent - wsh, a_extent = p.a_extent - 2LL * k0s;
     const _Float16* Az = p.A + (int64_t)i12 * p.a_s2 + (int64_t)i13 * p.a_s3 + k0s;
     const int dp = p.dp;
     const int64_t sc_extent = 2LL * M * dp - 2LL * (k0s / QK);
-    const _Float16* Adz = p.Ad + (int64_t)z * M * dp + k0s / QK;
+    const _Float16* Adz = !QUANT ? nullptr : p.Ad + (int64_t)z * M * dp + k0s / QK;
     const _Float16* Asz = WT == T_Q4_1 ? p.As + (int64_t)z * M * dp + k0s / QK : nullptr;
     // wavefronts 0, 1 load the two blocks' d; for Q4_1, 2 and 3 load the two blocks' s
-    const bool xload = wn < 2 || WT == T_Q4_1;
+    const bool xload = QUANT && (wn < 2 || WT == T_Q4_1);
 
     // ---- DMA offsets, fixed for the whole K loop
-    // activation tile, instruction i of wavefront w: rows (NI*w+i)*RPI + lane/CH,
+    // activation / F16-weight tile, instruction i of wavefront w: rows (NI*w+i)*RPI + lane/CH,
     // slot lane%CH <- chunk (lane%CH) ^ (row%CH)
     const int trow = lane / CH;
-    int aoff[NI], tch[NI];
+    int aoff[NI], foff[NI], tch[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int row = (wn * NI + i) * RPI + trow;
         tch[i] = (lane % CH) ^ swz<CH>(row);
         aoff[i] = m0 + row < M ? ((m0 + row) * (int)p.a_s1 + tch[i] * 8) * 2 : OOB;
+        foff[i] = !QUANT && n0 + row < N ? (n0 + row) * (int)p.w_nb1 + tch[i] * 16 : OOB;
     }
-    int woff[RLD];  // raw weight dword j = NT*i + 64w + lane -> (row j / RD, dword j % RD)
+    int woff[QUANT ? RLD : 1];  // raw weight dword j = NT*i + 64w + lane -> (row j / RD, dword j % RD)
 #pragma unroll
-    for (int i = 0; i < RLD; ++i) {
+    for (int i = 0; i < (QUANT ? RLD : 1); ++i) {
         const int j = tid + NT * i, row = j / RD, c = j - row * RD;
-        woff[i] = j < BN * RD && n0 + row < N ? (n0 + row) * (int)p.w_nb1 + 4 * c : OOB;
+        woff[i] = QUANT && j < BN * RD && n0 + row < N ? (n0 + row) * (int)p.w_nb1 + 4 * c : OOB;
     }
 
     auto dma_stage = [&](int s, St& b) {
@@ -228,7 +233,7 @@ __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEp
 #pragma unroll
         for (int i = 0; i < NI; ++i)
             dma_b128(ar, &b.A[(wn * NI + i) * RPI * SKH], tail && k0 + tch[i] * 8 >= K ? OOB : aoff[i]);
-        {
+        if (QUANT) {
             const int64_t seg = (int64_t)s * BKB * WB;
             const auto wrs = make_rsrc(Wz + seg, w_extent - seg);
 #pragma unroll
@@ -242,6 +247,11 @@ __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEp
             } else if (WT == T_Q4_1) {
                 dma_b32(make_rsrc(Asz, sc_extent), &b.As[WT == T_Q4_1 ? 64 * (wn & 1) : 0][0], soff);
             }
+        } else {
+            const auto fr = make_rsrc(Wz + 2LL * k0, w_extent - 2LL * k0);
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+                dma_b128(fr, &b.Bf[(wn * NI + i) * RPI * SKH], tail && k0 + tch[i] * 8 >= K ? OOB : foff[i]);
         }
     };
 
@@ -260,7 +270,7 @@ __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEp
     };
 
     auto compute = [&](int s, const St& b) {
-        {
+        if (QUANT) {
             const uint32_t* rowp = &b.W[wrow * RD];
             const uint16_t* hrow = reinterpret_cast<const uint16_t*>(rowp);
             if (WT == T_Q4_1 && !DOTS) {
@@ -336,6 +346,15 @@ __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEp
                         }
                     }
                 }
+            }
+        } else {
+#pragma unroll
+            for (int kk = 0; kk < SKH / 16; ++kk) {
+                const v8h bfr = frag(b.Bf, wrow, 2 * kk + g);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                    acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag(b.A, mt * 32 + lr, 2 * kk + g), bfr,
+                                                                     acc[mt], 0, 0, 0);
             }
         }
     };
@@ -482,7 +501,7 @@ __global__ __launch_bounds__(NT, 2) void mmq_kernel(const MmqArgs p, const MmqEp
         }
         stage_barrier();
         if (s + 2 < nstage) dma_stage(s + 2, refill);
-        if (!DOTS) {
+        if (QUANT && !DOTS) {
             compute_q(s, cur);
         } else {
             compute(s, cur);
@@ -734,20 +753,31 @@ __global__ __launch_bounds__(NT, 2) void mmq_f16_kernel(const MmqArgs p, const M
 
     if (EPI == MMQ_EPI_STORE) {
         char* Dz = reinterpret_cast<char*>(p.D) + (int64_t)i12 * p.d_nb2 + (int64_t)i13 * p.d_nb3 + split * p.d_split;
+        // the wavefront's 64 x 64 results through its quarter of the stage buffers: whole 256-byte
+        // row segments leave, as float4 or (rows that are no multiple of four) 64 columns at a time
+        __syncthreads();  // every wavefront has read its last fragments
+        float* t = reinterpret_cast<float*>(sb) + 4096 * wv;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if (rr[i] < 0) continue;
-            char* row = Dz + (int64_t)rr[i] * p.d_nb1;
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                float* d = reinterpret_cast<float*>(row) + nc[j];
-                if (p.d_v4) {
-                    if (nc[j] < N) *reinterpret_cast<v4f*>(d) = acc[i][j];
-                } else {
+            for (int j = 0; j < 4; ++j) *reinterpret_cast<v4f*>(&t[row64_chunk(16 * i + r16, 4 * j + kg)]) = acc[i][j];
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        __builtin_amdgcn_wave_barrier();
+        const int mw = m0 + 64 * wm, nw = n0 + 64 * wn;
+        if (p.d_v4) {
+            const int n = nw + 4 * r16;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (nc[j] + r < N) d[r] = acc[i][j][r];
-                }
+            for (int it = 0; it < 16; ++it) {
+                const int r = 4 * it + kg;
+                const v4f v = *reinterpret_cast<const v4f*>(&t[row64_chunk(r, r16)]);
+                if (mw + r < M && n < N) *reinterpret_cast<v4f*>(Dz + (int64_t)(mw + r) * p.d_nb1 + 4LL * n) = v;
+            }
+        } else {
+            const int n = nw + lane;
+#pragma unroll 16
+            for (int r = 0; r < 64; ++r) {
+                const float v = t[row64_chunk(r, lane >> 2) + (lane & 3)];
+                if (mw + r < M && n < N) *reinterpret_cast<float*>(Dz + (int64_t)(mw + r) * p.d_nb1 + 4LL * n) = v;
             }
         }
         return;
@@ -860,11 +890,17 @@ __global__ __launch_bounds__(256) void mmq_reduce_kernel(const float* __restrict
     }
 }
 
-// F16 weights
+// F16 weights. Plain stores with K < 640 take mmq_kernel (three stage buffers of 32-deep steps: the
+// first stage is multiplied sooner, and there are too few for mmq_f16_kernel's rate to pay: 38481 x
+// 638 x 128 31.9 us and 37.3 there, 24551 x 1000 x 256 36.7 and 38.6, 894 x 40 x 576 11.7 and 12.6,
+// 66 x 1363 x 608 14.9 and 15.4; 5 x 147 x 736 15.1 and 13.8). Both add the products in the same
+// order; fused epilogues are shorter on mmq_f16_kernel.
 static void launch_f16(const MmqArgs& a, int Z, const MmqEpi* e, hipStream_t st) {
     const int TT = a.tiles_m * a.tiles_n * a.ksplit;
     const dim3 grid((unsigned)(((TT + 7) / 8) * 8), (unsigned)Z);
-    if (a.ksplit > 1 || !e || e->kind == MMQ_EPI_STORE) mmq_f16_kernel<MMQ_EPI_STORE><<<grid, NT, 0, st>>>(a, MmqEpi{});
+    const bool store = a.ksplit > 1 || !e || e->kind == MMQ_EPI_STORE;
+    if (store && a.K < 640) mmq_kernel<T_F16, false, MMQ_EPI_STORE><<<grid, NT, 0, st>>>(a, MmqEpi{});
+    else if (store) mmq_f16_kernel<MMQ_EPI_STORE><<<grid, NT, 0, st>>>(a, MmqEpi{});
     else if (e->kind == MMQ_EPI_RESIDUAL) mmq_f16_kernel<MMQ_EPI_RESIDUAL><<<grid, NT, 0, st>>>(a, *e);
     else mmq_f16_kernel<MMQ_EPI_QKV><<<grid, NT, 0, st>>>(a, *e);
 }
@@ -948,9 +984,9 @@ int mmq_ksplit(int type, int64_t M, int64_t N, int64_t K, int64_t Z, int cus) {
 // instructions on the same operands (integer block sums by two MFMAs, the
 // d_a (x) d_w outer product by one, acc = fma(isum, S, acc) in block order,
 // the Q4_1 offset term by MFMA per pair of blocks), so the results are
-// bit-identical to mmq_kernel's.  F16 weights stay on mmq_kernel: at 2 bytes
+// bit-identical to mmq_kernel's.  F16 weights stay on the tiled kernels: at 2 bytes
 // per element their LDS copy leaves one workgroup per CU, and the tiled
-// kernel is faster there.
+// kernels are faster there.
 namespace {
 constexpr int SKMAX = 128;  // largest K
 }  // namespace
@@ -1161,8 +1197,8 @@ static hipError_t try_skinny(const MatW& w, const ActF16& a, const MatD& d, int6
                              int32_t* dots, const MmqEpi* epi, const MmqSplit& sp, hipStream_t st, bool* done) {
     *done = false;
     if (!sp.skinny || dots || (epi && epi->kind != MMQ_EPI_STORE) || ne12 * ne13 != 1 || a.M < 4096) return hipSuccess;
-    // F16 weights stay on the tiled kernel: their LDS rows (2 bytes per element) leave
-    // one workgroup per CU, and the tiled kernel is faster there
+    // F16 weights stay on the tiled kernels: their LDS rows (2 bytes per element) leave
+    // one workgroup per CU, and those are faster there
     if (w.type == T_F16 || a.dp > 4 || a.dp % 2 != 0) return hipSuccess;
     const int dp = (int)a.dp;
     int wpitch = 0;
