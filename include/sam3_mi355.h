@@ -530,8 +530,9 @@ mi355_status mi355_context_set_fusion(mi355_context* ctx, int enable);
  * Q4_0 under MI355_MMQ_AUTO) the same shapes (N % 4 == 0, no K split) run on
  * an int8 skinny kernel that keeps each wavefront's activation fragments in
  * registers and reads the small weight matrix from L2, again bit-identical to
- * the tiled int8 kernel.  Off routes both to the tiled kernels (for
- * comparisons). */
+ * the tiled int8 kernel, and MUL_MATs of at most 64 F32 activation rows with
+ * K <= 512 on one that quantizes the rows itself.  Off routes all to the tiled
+ * kernels (for comparisons). */
 mi355_status mi355_context_set_skinny(mi355_context* ctx, int enable);
 
 /* The kernel behind 2-D MUL_MATs with Q8_0 / Q4_0 / Q4_1 weights in the

@@ -315,6 +315,10 @@ mi355_status mul_mat_run(mi355_context* ctx, const mi355_tensor* s0, const mi355
                            "repack_weights launch");
             if (st != MI355_STATUS_SUCCESS) return st;
         }
+        if (ctx->skinny && mmq8_few_ok(wr, view_of(s1))) {
+            Timed tf(tctx, "mmq8_few");
+            return hip_check(ctx, tf.done(launch_mmq8_few(wr, view_of(s1), matd_of(d), pl.ks, ctx->stream)), "mmq8_few launch");
+        }
         const ActI8 a8 = act_i8(ws, pl, s0->type, M, K);
         {
             Timed tq8(tctx, "quantize_mmq_i8");

@@ -922,6 +922,179 @@ static bool launch8_skinny(const Mmq8Args& a, int wtype, const MmqEpi* e, int cu
     return true;
 }
 
+// ---- few activation rows (M <= 64, K <= 512, F32 rows as they are)
+// A prompt's few tokens: the quantize pass and the tiled kernel took 8.7 us a call at 9 x 256 x 256,
+// nearly all of it launches and latency; this kernel alone takes 5.5 (17 x 381 x 448: 12.3 -> 8.1).
+// Its blocks run one after another, so a longer K is the tiled kernel's, which splits it
+// (64 x 1024 x 1024: 16.7 us here, 12.8 there). The four wavefronts of a workgroup
+// quantize the blocks of 32 rows between them (from_float x86, as the quantize pass) straight into
+// MFMA fragments in LDS, and after one barrier each computes one 32-column tile, its weight
+// fragments read from global memory a chunk of four blocks ahead. The arithmetic is the tiled
+// kernel's in its order, K split included (range sums added in range order), so the results are
+// bit-identical.
+namespace {
+constexpr int FEW_M = 64, FEW_KB = 16;  // most rows; most blocks of K
+struct FewArgs {
+    const char* X;
+    int64_t x_nb1;
+    const int8_t* W;
+    int64_t w_s1;
+    const _Float16 *Wd, *Wm;
+    float* D;
+    int64_t d_nb1;
+    int M, N, nb, nst, sps;
+};
+}  // namespace
+template <int WT>
+__global__ __launch_bounds__(256) void mmq8_few_kernel(const FewArgs p) {
+    constexpr bool Q41 = WT == T_Q4_1;
+    __shared__ __attribute__((aligned(16))) v4i sA[FEW_KB][64];  // [block][lane]: quants 16 g .. + 15 of row lr
+    __shared__ uint32_t sD[FEW_KB][32];                          // [block][row]: d in the half of its k-slot
+    __shared__ uint16_t sS[Q41 ? FEW_KB : 1][32];                // Q8_1 sums
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lr = lane & 31, g = lane >> 5;
+    const int ntn = (p.N + 31) / 32, ngr = (ntn + 3) / 4;
+    const int mt = blockIdx.x / ngr, j = (blockIdx.x - mt * ngr) * 4 + w;
+    const int m0 = 32 * mt, n = 32 * j + lr;
+    const int nb = p.nb, nstg = (nb + 1) / 2;
+    const bool mv = m0 + lr < p.M, nv = j < ntn && n < p.N;
+    // the first chunk of weight fragments, in flight under the quantization
+    v4i wf[2][4];
+    v2i dw[2][2];
+    int mw[2][2] = {{0, 0}, {0, 0}};
+    auto load_w = [&](int c, v4i (&f)[4], v2i (&d)[2], int (&mm)[2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            f[i] = nv && 4 * c + i < nb ? *reinterpret_cast<const v4i*>(p.W + (int64_t)n * p.w_s1 + 32 * (4 * c + i) + 16 * g) : v4i{0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const bool in = nv && g == 0 && 2 * c + i < nstg;
+            d[i] = v2i{in ? (int)reinterpret_cast<const uint32_t*>(p.Wd)[(int64_t)n * p.nst + 2 * c + i] : 0, 0};
+            if (Q41) mm[i] = in ? (int)reinterpret_cast<const uint32_t*>(p.Wm)[(int64_t)n * p.nst + 2 * c + i] : 0;
+        }
+    };
+    load_w(0, wf[0], dw[0], mw[0]);
+    for (int b = w; b < 2 * nstg; b += 4) {
+        v4i q4 = {0, 0, 0, 0};
+        float d = 0.0f;
+        int isum = 0;
+        if (b < nb) {  // (uniform) a block past an odd count is zero
+            float x[16];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const v4f v = mv ? *reinterpret_cast<const v4f*>(p.X + (int64_t)(m0 + lr) * p.x_nb1 + 128LL * b + 64 * g + 16 * i)
+                                 : v4f{0, 0, 0, 0};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[4 * i + e] = v[e];
+            }
+            float amax = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(x[i]));
+            amax = fmaxf(amax, lane_swap_f<32>(amax));
+            d = amax / 127.0f;
+            const float id = amax != 0.0f ? 127.0f / amax : 0.0f;
+            int q[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                q[i] = (int)rintf(x[i] * id);
+                isum += q[i];
+            }
+            if (Q41) isum += lane_swap<32>(isum);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                q4[i] = (q[4 * i] & 0xff) | ((q[4 * i + 1] & 0xff) << 8) | ((q[4 * i + 2] & 0xff) << 16) | (q[4 * i + 3] << 24);
+        }
+        sA[b][lane] = q4;
+        if (g == 0) {
+            sD[b][lr] = b < nb ? (uint32_t)f2h(d) << (16 * (b & 1)) : 0u;
+            if (Q41) sS[Q41 ? b : 0][lr] = b < nb ? f2h(d * (float)isum) : (uint16_t)0;
+        }
+    }
+    __syncthreads();
+    if (j >= ntn) return;
+    const v16i zi = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    const v16f zf = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    v16f acc = zf, tot = zf;
+    int left = p.sps;  // stages left in this K range
+    bool first = true;
+    auto chunk = [&](int c, const v4i (&f)[4], const v2i (&dv)[2], const int (&mm)[2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int st = 2 * c + i;
+            if (st >= nstg) break;
+            if (left == 0) {  // a range is done: its sum joins the ranges before it
+                tot = first ? acc : tot + acc;
+                acc = zf;
+                first = false;
+                left = p.sps;
+            }
+            --left;
+            if (Q41) {
+                const uint32_t s2 = (uint32_t)sS[Q41 ? 2 * st : 0][lr] | ((uint32_t)sS[Q41 ? 2 * st + 1 : 0][lr] << 16);
+                const v4i saf = {(int)s2, 0, 0, 0}, mwf = {mm[i], 0, 0, 0};
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, saf), __builtin_bit_cast(v8h, mwf), acc, 0, 0, 0);
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int b = 2 * st + h;
+                const v2i da = {(int)sD[b][lr], 0};
+                const v16i I = __builtin_amdgcn_mfma_i32_32x32x32_i8(sA[b][lane], f[2 * i + h], zi, 0, 0, 0);
+                const v16f S = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, da), __builtin_bit_cast(v4h, dv[i]), zf, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[e] = __builtin_fmaf((float)I[e], S[e], acc[e]);
+            }
+        }
+    };
+    const int nch = (nstg + 1) / 2;
+    for (int c = 0; c < nch; c += 2) {
+        if (c + 1 < nch) load_w(c + 1, wf[1], dw[1], mw[1]);
+        chunk(c, wf[0], dw[0], mw[0]);
+        if (c + 1 >= nch) break;
+        if (c + 2 < nch) load_w(c + 2, wf[0], dw[0], mw[0]);
+        chunk(c + 1, wf[1], dw[1], mw[1]);
+    }
+    if (!first) acc = tot + acc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const int m = m0 + 8 * (e >> 2) + 4 * g + (e & 3);
+        if (m < p.M && nv) *reinterpret_cast<float*>(reinterpret_cast<char*>(p.D) + (int64_t)m * p.d_nb1 + 4LL * n) = acc[e];
+    }
+}
+
+bool mmq8_few_ok(const WRep& w, const SrcView& x) {
+    return x.type == T_F32 && x.ne[1] <= FEW_M && x.ne[1] > 0 && x.ne[2] * x.ne[3] == 1 && x.ne[0] == w.K && w.K % QK == 0 &&
+           w.K > 0 && w.K / QK <= FEW_KB && w.N > 0 && x.nb[0] == 4 && x.nb[1] % 16 == 0 &&
+           (reinterpret_cast<uintptr_t>(x.data) & 15) == 0 && w.q_s1 % 16 == 0 && (reinterpret_cast<uintptr_t>(w.q) & 15) == 0 &&
+           (reinterpret_cast<uintptr_t>(w.d) & 3) == 0 && (w.type != T_Q4_1 || (reinterpret_cast<uintptr_t>(w.m) & 3) == 0);
+}
+
+hipError_t launch_mmq8_few(const WRep& w, const SrcView& x, const MatD& d, int ks, hipStream_t st) {
+    if (!mmq8_few_ok(w, x) || !d.data) return hipErrorInvalidValue;
+    FewArgs p;
+    p.X = x.data;
+    p.x_nb1 = x.nb[1];
+    p.W = w.q;
+    p.w_s1 = w.q_s1;
+    p.Wd = w.d;
+    p.Wm = w.m;
+    p.D = d.data;
+    p.d_nb1 = d.nb1;
+    p.M = (int)x.ne[1];
+    p.N = (int)w.N;
+    p.nb = (int)(w.K / QK);
+    p.nst = (int)(mmq_scale_pitch(w.K) / 2);
+    const int nstage = (p.nb + 1) / 2;
+    p.sps = ks > 1 ? (nstage + ks - 1) / ks : nstage;
+    const unsigned grid = (unsigned)(((p.M + 31) / 32) * (((p.N + 31) / 32 + 3) / 4));
+    switch (w.type) {
+        case T_Q8_0: mmq8_few_kernel<T_Q8_0><<<grid, 256, 0, st>>>(p); break;
+        case T_Q4_0: mmq8_few_kernel<T_Q4_0><<<grid, 256, 0, st>>>(p); break;
+        case T_Q4_1: mmq8_few_kernel<T_Q4_1><<<grid, 256, 0, st>>>(p); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 template <int WT, int TM>
 static void launch8_t(const Mmq8Args& a, const MmqEpi* e, hipStream_t st) {
     const int TT = a.tiles_m * a.tiles_n * a.ksplit;
