@@ -544,8 +544,8 @@ mi355_status mi355_context_set_skinny(mi355_context* ctx, int enable);
  * - MI355_MMQ_INT8: src1 quantized to one-byte quants, weights repacked into
  *   int8 rows with separate scale arrays on each call, block sums on
  *   v_mfma_i32_32x32x32_i8;
- * - MI355_MMQ_AUTO (the default): MI355_MMQ_INT8 for Q8_0 and Q4_0 weights,
- *   MI355_MMQ_F16 for Q4_1 (the faster per call with the repack counted).
+ * - MI355_MMQ_AUTO (the default): the faster per call with the repack counted:
+ *   MI355_MMQ_INT8, except for few activation rows over a large weight.
  * Prepared weights always take the int8 kernel; other MUL_MATs keep their
  * own kernels. */
 typedef enum {

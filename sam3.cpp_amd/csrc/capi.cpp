@@ -160,8 +160,7 @@ int device_cus(int device) {
 // kernel: the MI355_MMQ_* route when the operands are eligible for it
 MmPlan mm_plan(const mi355_tensor* s0, const mi355_tensor* s1, int cus, bool split = true, int kernel = 0) {
     const bool prep = s0->layout == MI355_LAYOUT_INT8;
-    const bool i8 = prep || kernel == MI355_MMQ_INT8 ||
-                    (kernel == MI355_MMQ_AUTO && (s0->type == T_Q8_0 || s0->type == T_Q4_0));
+    const bool i8 = prep || kernel != MI355_MMQ_F16;
     MmPlan pl;
     if (s0->type == T_F32) return pl;
     const int64_t K = s1->ne[0], M = s1->ne[1], Z = s1->ne[2] * s1->ne[3];
@@ -188,6 +187,38 @@ MmPlan mm_plan(const mi355_tensor* s0, const mi355_tensor* s1, int cus, bool spl
     return pl;
 }
 
+// The route of a MUL_MAT with ggml-layout quantized weights under MI355_MMQ_AUTO: int8 with the
+// repack in the call (1297 x 771 x 736 Q4_1 25.9 us on the fp16 route, 17.7 on this one;
+// 5184 x 3072 x 1024 76 and 70; 2000 x 1024 x 1024 30.3 and 21.1), except
+// - few rows over a large weight, where the repack costs more than the kernel saves (1 x 4736 x 1024
+//   13.5 and 18.3; 64 x 1024 x 1024 14.2 and 15.8; 26 x 668 x 480 13.3 and 14.1); shorter K takes the
+//   few-row kernel, and with N % 4 != 0 the fp16 route cannot split K;
+// - Q4_1 where the fp16 route's skinny kernel serves it (4445 x 36 x 96 9.3 and 12.3), and grids of
+//   200 tiles or more with N % 4 != 0 (1255 x 4258 x 4704 151 and 176).
+int mm_route(const mi355_tensor* s0, const mi355_tensor* s1, int kernel) {
+    if (kernel != MI355_MMQ_AUTO || s0->layout != MI355_LAYOUT_GGML || !mm_i8_eligible(s0, s1) || !f16_extents_ok(s0, s1))
+        return kernel;
+    const int64_t K = s0->ne[0], N = s0->ne[1], M = s1->ne[1];
+    const bool few = M <= 64 && K >= 480 && N % 4 == 0 && N * K >= ((int64_t)1 << 18);
+    const bool q41 = s0->type == T_Q4_1 && ((M >= 4096 && K <= 128) || (N % 4 != 0 && ((M + 127) / 128) * ((N + 127) / 128) >= 200));
+    return few || q41 ? MI355_MMQ_F16 : MI355_MMQ_INT8;
+}
+
+bool dst_split_ok(const mi355_tensor* d) {
+    return d->nb[1] % 16 == 0 && (reinterpret_cast<uintptr_t>(d->data) & 15) == 0;
+}
+
+// The plan of mm_route's route or, where that needs more than limit bytes of scratch, of the other
+// route if it fits (AUTO only; both give the same bits).
+MmPlan mm_plan_in(const mi355_context* ctx, const mi355_tensor* s0, const mi355_tensor* s1, const mi355_tensor* d, size_t limit) {
+    const bool split = dst_split_ok(d);
+    const MmPlan pl = mm_plan(s0, s1, ctx->cus, split, mm_route(s0, s1, ctx->mmq_kernel));
+    if (pl.total() <= limit || ctx->mmq_kernel != MI355_MMQ_AUTO || s0->type == T_F16 || pl.prep || !f16_extents_ok(s0, s1))
+        return pl;
+    const MmPlan other = mm_plan(s0, s1, ctx->cus, split, pl.i8 ? MI355_MMQ_F16 : MI355_MMQ_INT8);
+    return other.total() <= limit ? other : pl;
+}
+
 // ggml_soft_max_ext(a, mask, scale, max_bias) shape rules plus what softmax.hip implements.
 mi355_status check_soft_max(mi355_context* ctx, const mi355_tensor* src, const mi355_tensor* mask, float max_bias,
                             const mi355_tensor* dst) {
@@ -201,9 +232,6 @@ mi355_status check_soft_max(mi355_context* ctx, const mi355_tensor* src, const m
     return MI355_STATUS_SUCCESS;
 }
 
-bool dst_split_ok(const mi355_tensor* d) {
-    return d->nb[1] % 16 == 0 && (reinterpret_cast<uintptr_t>(d->data) & 15) == 0;
-}
 mi355_status ensure_ws(mi355_context* ctx, size_t bytes) { return ensure_buffer(ctx, &ctx->ws, &ctx->ws_size, bytes); }
 
 
@@ -791,7 +819,12 @@ mi355_status mi355_mul_mat(mi355_context* ctx, const mi355_tensor* s0, const mi3
             (void)hipGetLastError();
         return mul_mat_f32(ctx, s0, s1, d, static_cast<char*>(ctx->ws), ctx->ws_size, true);
     }
-    const MmPlan pl = mm_plan(s0, s1, ctx->cus, dst_split_ok(d), ctx->mmq_kernel);
+    MmPlan pl = mm_plan(s0, s1, ctx->cus, dst_split_ok(d), mm_route(s0, s1, ctx->mmq_kernel));
+    if (pl.total() > ctx->ws_size) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
+            pl = mm_plan_in(ctx, s0, s1, d, ctx->ws_size);  // nothing can be allocated now
+    }
     st = ensure_ws(ctx, pl.total());
     if (st != MI355_STATUS_SUCCESS) return st;
     return mul_mat_run(ctx, s0, s1, d, pl, static_cast<char*>(ctx->ws), true);
@@ -814,7 +847,7 @@ mi355_status mi355_mul_mat_noalloc(mi355_context* ctx, const mi355_tensor* s0, c
     if (!ctx->scratch)
         return fail(ctx, MI355_STATUS_FAILED, "mul_mat_noalloc: no static scratch on device %d (%s)", ctx->device,
                     ctx->scratch_error.c_str());
-    const MmPlan pl = mm_plan(s0, s1, ctx->cus, dst_split_ok(d), ctx->mmq_kernel);
+    const MmPlan pl = mm_plan_in(ctx, s0, s1, d, MI355_NOALLOC_SCRATCH_BYTES);
     if (pl.total() > MI355_NOALLOC_SCRATCH_BYTES)
         return fail(ctx, MI355_STATUS_UNSUPPORTED,
                     "mul_mat_noalloc: these operands need %zu bytes of scratch, the static scratch holds %zu",
