@@ -36,6 +36,7 @@
 // aligned or K not a multiple of 4.
 #include "common.cuh"
 #include "kernels.h"
+#include "pack.cuh"
 
 namespace mi355 {
 
@@ -431,9 +432,8 @@ void gemm_f32_dma_kernel(const GemmF32Args p, int ksplit, int sps) {
 // The same GEMM on the bf16 matrix cores: an fp32 value is the exact sum of three bf16 values
 // (x = h + m + l, each rounded to nearest even from what the ones before left: 8 + 8 + 8 bits),
 // and six of the nine products, hh + hm + mh + hl + lh + mm, carry everything down to 2^-24 of
-// the term. v_mfma_f32_32x32x16_bf16 makes the sixteen products of one pair in 32 cycles where
-// eight v_mfma_f32_32x32x2f32 take 512, so six pairs cost 192: 2.7 times less matrix time for
-// the same fp32 accumulators, which round six times per 16 terms instead of eight.
+// the term. The bf16 matrix cores make sixteen products in the time of one fp32 MFMA product, so
+// six cost 2.7 times less matrix time for the same fp32 accumulators, which round less often.
 //
 // The weights come split already (split_w_kernel: per row and 32 of K the three planes' 64 bytes
 // side by side, 192 bytes); the activations arrive as fp32 by LDS DMA and are split as the
@@ -452,16 +452,11 @@ void gemm_f32_dma_kernel(const GemmF32Args p, int ksplit, int sps) {
 // m = l = 0). Among finite operands only activations that round up to an infinite bf16 need it.
 namespace {
 typedef __bf16 v8b __attribute__((ext_vector_type(8)));
-typedef __bf16 v2b __attribute__((ext_vector_type(2)));
 struct SplitStage {
     float A[TM * 32];
     uint16_t B[TN * 96];  // row: plane p (h, m, l), 32 K each; chunk q of plane p in slot 4 p + (q ^ (row >> 2 & 3))
 };
 constexpr int SPLIT_NL = 10;  // DMA instructions per wavefront and stage: 4 activation, 6 weight
-__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
-    const v2f v = {a, b};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, v2b));
-}
 // eight fp32 values -> their three bf16 planes
 __device__ __forceinline__ void split8(const v4f (&x)[2], v8b& h, v8b& m, v8b& l) {
     v4i hh, mm, ll;
@@ -481,49 +476,10 @@ __device__ __forceinline__ void split8(const v4f (&x)[2], v8b& h, v8b& m, v8b& l
 }
 }  // namespace
 
-// planes of weight rows [N][K] (row pitch nb1 bytes; F32 or F16; or, taps == 9, a 3x3 kernel
-// [N][C][3][3] read in (tap, channel) order) -> [N][KP / 32][3][32] bf16, zero past K. One thread
-// per eight consecutive K.
+// the planes alone (split_w_item); one thread per item
 __global__ __launch_bounds__(256) void split_w_kernel(const char* __restrict__ w, int64_t nb1, int f16, int taps, int N, int K,
                                                       int KP, uint16_t* __restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int k8 = KP / 8;
-    if (i >= (int64_t)N * k8) return;
-    const int n = (int)(i / k8), k0 = (int)(i - (int64_t)n * k8) * 8;
-    const int C = K / taps;
-    uint16_t h[8], m[8], l[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int k = k0 + j;
-        float x = 0.0f;
-        if (k < K) {
-            const int64_t e = taps == 1 ? k : (int64_t)(k % C) * taps + k / C;
-            const char* row = w + (int64_t)n * nb1;
-            x = f16 ? h2f(reinterpret_cast<const uint16_t*>(row)[e]) : reinterpret_cast<const float*>(row)[e];
-        }
-        const uint32_t u = __float_as_uint(x);
-        uint32_t a = pk_bf16(x, 0.0f) & 0xffffu;
-        if ((a & 0x7f80u) == 0x7f80u) a = u >> 16;  // infinite, NaN, or rounded up to infinity: the top bits
-        if ((u & 0x7f800000u) == 0x7f800000u) {
-            if (u & 0x007fffffu) a |= 0x40u;  // a NaN stays one
-            h[j] = (uint16_t)a;
-            m[j] = l[j] = 0;
-            continue;
-        }
-        const float r = x - __uint_as_float(a << 16);
-        const uint32_t b = pk_bf16(r, 0.0f) & 0xffffu;
-        h[j] = (uint16_t)a;
-        m[j] = (uint16_t)b;
-        l[j] = (uint16_t)(pk_bf16(r - __uint_as_float(b << 16), 0.0f) & 0xffffu);
-    }
-    uint16_t* o = out + (int64_t)n * KP * 3 + (k0 >> 5) * 96 + (k0 & 31);
-    auto put = [&](uint16_t* d, const uint16_t (&v)[8]) {
-        *reinterpret_cast<uint4*>(d) = make_uint4(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16,
-                                                  v[4] | (uint32_t)v[5] << 16, v[6] | (uint32_t)v[7] << 16);
-    };
-    put(o, h);
-    put(o + 32, m);
-    put(o + 64, l);
+    split_w_item((int64_t)blockIdx.x * blockDim.x + threadIdx.x, w, nb1, f16, taps, N, K, KP, out);
 }
 
 template <bool CONV>

@@ -365,6 +365,15 @@ hipError_t launch_im2col_pad(const float* img, float* cols, int C, int Hin, int 
 hipError_t launch_pad_rows_f32(const void* src, bool f16, int64_t rows, int K, int kp, float* dst, hipStream_t st);
 // SimpleFPN neck passes (neck.hip); activations token-major [H*W][C]
 hipError_t launch_deconv_pack(const void* w, int wtype, int Cin, int Cout, uint16_t* out, hipStream_t st);
+// A kernel of the neck to repack: k = 2 the conv-transpose's rows (launch_deconv_pack), k = 3 of F16
+// launch_conv3x3_pack_f16's, k = 1 or 3 of F32 launch_split_w's planes
+struct NeckPack {
+    const void* w;
+    uint16_t* out;
+    int type, k, Cin, Cout;
+};
+constexpr int NECK_PACKS = 11;
+hipError_t launch_neck_pack(const NeckPack* jobs, int n, hipStream_t st);
 hipError_t launch_deconv_scatter(const float* D, const float* b, int H, int W, int Cout, bool gelu, float* y,
                                  hipStream_t st);
 hipError_t launch_im2col3x3(const float* x, int H, int W, int C, bool f16, void* cols, hipStream_t st);

@@ -95,9 +95,10 @@ mi355_status half_map(mi355_context* ctx, const float* x, int64_t P, int64_t C, 
 
 // conv_transpose_2d_p0(kernel [2, 2, Cout, Cin], stride 2) + bias (+ GELU):
 // x [H*W][Cin] -> y [(2H)*(2W)][Cout]
-// (x16 / y16: fp16 maps, the fused neck's intermediates; F16 kernels on the implicit path only)
+// (x16 / y16: fp16 maps, the fused neck's intermediates; F16 kernels on the implicit path only;
+// pre: the kernel as neck_pack left it)
 mi355_status deconv(mi355_context* ctx, const mi355_tensor* w, const float* b, const void* xv, int H, int W, bool gelu,
-                    void* yv, char* scratch, bool x16 = false, bool y16 = false) {
+                    void* yv, char* scratch, bool x16 = false, bool y16 = false, const char* pre = nullptr) {
     const float* x = static_cast<const float*>(xv);
     float* y = static_cast<float*>(yv);
     mi355_status st = check_kernel(ctx, w, b, 2, "neck_deconv");
@@ -105,9 +106,9 @@ mi355_status deconv(mi355_context* ctx, const mi355_tensor* w, const float* b, c
     const int Cout = (int)w->ne[2], Cin = (int)w->ne[3];
     const int64_t P = (int64_t)H * W;
     if (Cout % 4 != 0) return fail(ctx, MI355_STATUS_UNSUPPORTED, "neck_deconv: Cout %% 4 != 0");
-    uint16_t* packed = reinterpret_cast<uint16_t*>(scratch);
+    uint16_t* packed = reinterpret_cast<uint16_t*>(pre ? const_cast<char*>(pre) : scratch);
     float* D = reinterpret_cast<float*>(scratch + align_up((size_t)(4 * Cout * Cin * 2)));
-    {
+    if (!pre) {
         Timed t(ctx, "neck_deconv_pack");
         st = hip_check(ctx, t.done(launch_deconv_pack(w->data, w->type, Cin, Cout, packed, ctx->stream)), "deconv pack");
         if (st != MI355_STATUS_SUCCESS) return st;
@@ -135,8 +136,9 @@ mi355_status deconv(mi355_context* ctx, const mi355_tensor* w, const float* b, c
 }
 
 // conv_2d_sk_p0 (1x1) or conv_2d_s1_ph (3x3) + bias: x [H*W][Cin] -> y [H*W][Cout]
+// (pre: the kernel as neck_pack left it, read where the path is the one it was packed for)
 mi355_status conv(mi355_context* ctx, const mi355_tensor* w, const float* b, const void* xv, int H, int W, void* yv,
-                  char* scratch, bool x16 = false, bool y16 = false) {
+                  char* scratch, bool x16 = false, bool y16 = false, const char* pre = nullptr) {
     const float* x = static_cast<const float*>(xv);
     float* y = static_cast<float*>(yv);
     if (!w) return fail(ctx, MI355_STATUS_INVALID_ARG, "neck_conv: null kernel");
@@ -179,11 +181,13 @@ mi355_status conv(mi355_context* ctx, const mi355_tensor* w, const float* b, con
         g.Wd = W;
         g.C = Cin;
         if (gemm_f32_split_ok(g, 1)) {
-            g.wsplit = reinterpret_cast<const uint16_t*>(scratch);
-            Timed t(ctx, "neck_conv_split_w");
-            st = hip_check(ctx, t.done(launch_split_w(w->data, 4 * K, false, k * k, Cout, (int)K,
-                                                      reinterpret_cast<uint16_t*>(scratch), ctx->stream)),
-                           "conv kernel split");
+            g.wsplit = reinterpret_cast<const uint16_t*>(pre ? pre : scratch);
+            if (!pre) {
+                Timed t(ctx, "neck_conv_split_w");
+                st = hip_check(ctx, t.done(launch_split_w(w->data, 4 * K, false, k * k, Cout, (int)K,
+                                                          reinterpret_cast<uint16_t*>(scratch), ctx->stream)),
+                               "conv kernel split");
+            }
         } else if (k == 3) {
             Timed t(ctx, "neck_conv3x3_pack");
             st = hip_check(ctx, t.done(launch_conv3x3_pack(static_cast<const float*>(w->data), Cin, Cout,
@@ -197,14 +201,14 @@ mi355_status conv(mi355_context* ctx, const mi355_tensor* w, const float* b, con
     if (w->type == T_F16 && implicit_ok(x, Cin) && (k == 3 || (reinterpret_cast<uintptr_t>(w->data) & 15) == 0)) {
         // F16 kernels: an implicit GEMM on fp16 MFMA (the map rounded to fp16 as it
         // is loaded), bias in its epilogue; the 3x3 kernel repacked to (tap, channel)
-        if (k == 3) {
+        if (k == 3 && !pre) {
             Timed t(ctx, "neck_conv3x3_pack");
             st = hip_check(ctx, t.done(launch_conv3x3_pack_f16(static_cast<const uint16_t*>(w->data), Cin, Cout,
                                                                reinterpret_cast<uint16_t*>(scratch), ctx->stream)),
                            "conv3x3 pack");
             if (st != MI355_STATUS_SUCCESS) return st;
         }
-        const uint16_t* wk = k == 3 ? reinterpret_cast<const uint16_t*>(scratch) : static_cast<const uint16_t*>(w->data);
+        const uint16_t* wk = k == 3 ? reinterpret_cast<const uint16_t*>(pre ? pre : scratch) : static_cast<const uint16_t*>(w->data);
         // the fp16 map and the K split's partial sums follow the repacked kernel
         char* next = scratch + (k == 3 ? align_up((size_t)(K * Cout * 2)) : 0);
         const void* xm = x;
@@ -264,11 +268,35 @@ bool fp16_maps(const float* x, int E, const mi355_neck_scale* s) {
     return f16(s[0].deconv2_w) && s[0].deconv2_w->ne[3] % 32 == 0;
 }
 
-// Buffer plan of the whole neck: two map buffers, the input rounded to fp16, and the largest op
-// scratch.
+// the neck's kernels in order: per scale the conv-transposes, the 1x1, the 3x3
+struct NeckKernel {
+    const mi355_tensor* w;
+    const float* b;
+    int k;
+};
+void neck_kernels(const mi355_neck_scale* s, NeckKernel (&o)[NECK_PACKS]) {
+    int n = 0;
+    for (int i = 0; i < 4; ++i) {
+        if (i < 2) o[n++] = {s[i].deconv1_w, s[i].deconv1_b, 2};
+        if (i == 0) o[n++] = {s[i].deconv2_w, s[i].deconv2_b, 2};
+        o[n++] = {s[i].conv1x1_w, s[i].conv1x1_b, 1};
+        o[n++] = {s[i].conv3x3_w, s[i].conv3x3_b, 3};
+    }
+}
+// bytes of a kernel repacked for the implicit path, 0 where that reads it as it is (an F16 1x1) or
+// its channel counts do not take it
+size_t neck_pack_bytes(const NeckKernel& n) {
+    const int64_t Cin = n.k == 2 ? n.w->ne[3] : n.w->ne[2], Cout = n.k == 2 ? n.w->ne[2] : n.w->ne[3];
+    if (n.k == 2) return align_up((size_t)(4 * Cout * Cin * 2));
+    if (n.w->type == T_F32 ? Cin % (n.k == 1 ? 4 : 32) != 0 : n.k == 1 || Cin % 32 != 0) return 0;
+    return align_up(n.w->type == T_F32 ? gemm_f32_split_bytes(Cout, (int64_t)n.k * n.k * Cin) : (size_t)(9 * Cin * Cout * 2));
+}
+
+// Buffer plan of the whole neck: two map buffers, the input rounded to fp16, the repacked kernels,
+// and the largest op scratch.
 struct NeckPlan {
-    size_t map = 0, half = 0, scratch = 0;
-    size_t total() const { return 2 * map + half + scratch; }
+    size_t map = 0, half = 0, pack = 0, scratch = 0;
+    size_t total() const { return 2 * map + half + pack + scratch; }
 };
 
 bool neck_plan(int E, int G, const mi355_neck_scale* s, NeckPlan* pl) {
@@ -278,6 +306,9 @@ bool neck_plan(int E, int G, const mi355_neck_scale* s, NeckPlan* pl) {
             return false;
     const int64_t G2 = (int64_t)G * G;
     pl->half = align_up((size_t)(G2 * E * 2));
+    NeckKernel nk[NECK_PACKS];
+    neck_kernels(s, nk);
+    for (const NeckKernel& n : nk) pl->pack += neck_pack_bytes(n);
     auto mapb = [&](int64_t P, int64_t C) { pl->map = std::max(pl->map, align_up((size_t)(P * C * 4))); };
     auto scr = [&](size_t b) { pl->scratch = std::max(pl->scratch, b); };
     // scale 0: deconv E->C1 (2G), GELU, deconv C1->D (4G), 1x1, 3x3
@@ -375,7 +406,8 @@ mi355_status mi355_sam3_neck(mi355_context* ctx, const float* x, int E, int G, c
     float* A = reinterpret_cast<float*>(base);
     float* B = reinterpret_cast<float*>(base + pl.map);
     char* xh = base + 2 * pl.map;
-    char* scr = xh + pl.half;
+    char* packs = xh + pl.half;
+    char* scr = packs + pl.pack;
 #define TRY(e)                                     \
     do {                                           \
         st = (e);                                  \
@@ -397,22 +429,42 @@ mi355_status mi355_sam3_neck(mi355_context* ctx, const float* x, int E, int G, c
     if (xh_ok) TRY(half_map(ctx, x, P, E, xh));
     const void* xd = xh_ok ? static_cast<const void*>(xh) : x;
     const bool hx = h && xh_ok;
+    // every kernel's repack in one launch
+    NeckKernel nk[NECK_PACKS];
+    neck_kernels(s, nk);
+    NeckPack jobs[NECK_PACKS];
+    const char* pre[NECK_PACKS] = {};
+    int nj = 0;
+    for (int i = 0; i < NECK_PACKS; ++i) {
+        TRY(check_kernel(ctx, nk[i].w, nk[i].b, nk[i].k, nk[i].k == 2 ? "neck_deconv" : "neck_conv"));
+        const size_t n = neck_pack_bytes(nk[i]);
+        if (!n) continue;
+        const int d = nk[i].k == 2 ? 1 : 0;
+        jobs[nj++] = {nk[i].w->data, reinterpret_cast<uint16_t*>(packs), nk[i].w->type, nk[i].k, (int)nk[i].w->ne[2 + d],
+                      (int)nk[i].w->ne[3 - d]};
+        pre[i] = packs;
+        packs += n;
+    }
+    {
+        Timed t(ctx, "neck_pack");
+        TRY(hip_check(ctx, t.done(launch_neck_pack(jobs, nj, ctx->stream)), "neck pack launch"));
+    }
     // scale 0 (4x): deconv + GELU, deconv, 1x1, 3x3
-    TRY(deconv(ctx, s[0].deconv1_w, s[0].deconv1_b, xd, G, G, true, A, scr, xh_ok, hd));
-    TRY(deconv(ctx, s[0].deconv2_w, s[0].deconv2_b, A, 2 * G, 2 * G, false, B, scr, hd, h));
-    TRY(conv(ctx, s[0].conv1x1_w, s[0].conv1x1_b, B, 4 * G, 4 * G, A, scr, h, h));
-    TRY(conv(ctx, s[0].conv3x3_w, s[0].conv3x3_b, A, 4 * G, 4 * G, out[0], scr, h, false));
+    TRY(deconv(ctx, s[0].deconv1_w, s[0].deconv1_b, xd, G, G, true, A, scr, xh_ok, hd, pre[0]));
+    TRY(deconv(ctx, s[0].deconv2_w, s[0].deconv2_b, A, 2 * G, 2 * G, false, B, scr, hd, h, pre[1]));
+    TRY(conv(ctx, s[0].conv1x1_w, s[0].conv1x1_b, B, 4 * G, 4 * G, A, scr, h, h, pre[2]));
+    TRY(conv(ctx, s[0].conv3x3_w, s[0].conv3x3_b, A, 4 * G, 4 * G, out[0], scr, h, false, pre[3]));
     // scale 1 (2x): deconv, 1x1, 3x3
-    TRY(deconv(ctx, s[1].deconv1_w, s[1].deconv1_b, xd, G, G, false, A, scr, xh_ok, h));
-    TRY(conv(ctx, s[1].conv1x1_w, s[1].conv1x1_b, A, 2 * G, 2 * G, B, scr, h, h));
-    TRY(conv(ctx, s[1].conv3x3_w, s[1].conv3x3_b, B, 2 * G, 2 * G, out[1], scr, h, false));
+    TRY(deconv(ctx, s[1].deconv1_w, s[1].deconv1_b, xd, G, G, false, A, scr, xh_ok, h, pre[4]));
+    TRY(conv(ctx, s[1].conv1x1_w, s[1].conv1x1_b, A, 2 * G, 2 * G, B, scr, h, h, pre[5]));
+    TRY(conv(ctx, s[1].conv3x3_w, s[1].conv3x3_b, B, 2 * G, 2 * G, out[1], scr, h, false, pre[6]));
     // scale 2 (1x): 1x1, 3x3
-    TRY(conv(ctx, s[2].conv1x1_w, s[2].conv1x1_b, hx ? xd : x, G, G, A, scr, hx, h));
-    TRY(conv(ctx, s[2].conv3x3_w, s[2].conv3x3_b, A, G, G, out[2], scr, h, false));
+    TRY(conv(ctx, s[2].conv1x1_w, s[2].conv1x1_b, hx ? xd : x, G, G, A, scr, hx, h, pre[7]));
+    TRY(conv(ctx, s[2].conv3x3_w, s[2].conv3x3_b, A, G, G, out[2], scr, h, false, pre[8]));
     // scale 3 (0.5x): max-pool, 1x1, 3x3
     TRY(pool(ctx, hx ? xd : x, G, G, E, B, hx));
-    TRY(conv(ctx, s[3].conv1x1_w, s[3].conv1x1_b, B, G / 2, G / 2, A, scr, hx, h));
-    TRY(conv(ctx, s[3].conv3x3_w, s[3].conv3x3_b, A, G / 2, G / 2, out[3], scr, h, false));
+    TRY(conv(ctx, s[3].conv1x1_w, s[3].conv1x1_b, B, G / 2, G / 2, A, scr, hx, h, pre[9]));
+    TRY(conv(ctx, s[3].conv3x3_w, s[3].conv3x3_b, A, G / 2, G / 2, out[3], scr, h, false, pre[10]));
 #undef TRY
     return MI355_STATUS_SUCCESS;
 }

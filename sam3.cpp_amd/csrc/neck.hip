@@ -1,17 +1,18 @@
 // SAM3 SimpleFPN neck kernels (sam3_build_neck_graph, sam3.cpp:3867-3925) on
-// token-major activations [H*W][C] (ggml [C, W, H]).  conv_f16_dma_kernel (and
-// conv_f16_kernel, its register-staged form for operands beyond 32-bit buffer
-// offsets) is the fp16-MFMA implicit GEMM of the F16-kernel convolutions (3x3,
+// token-major activations [H*W][C] (ggml [C, W, H]).  conv_f16_dma_kernel (over
+// fp16 maps; conv1x1_f32map_kernel for a 1x1 over an F32 one, and conv_f16_kernel,
+// register-staged, for the rest and operands beyond 32-bit buffer offsets) is the fp16-MFMA implicit GEMM of the F16-kernel convolutions (3x3,
 // 1x1 and the 2x2 / stride-2 conv-transpose with its scatter, bias and GELU in
 // the epilogue; the 3x3 and 1x1 split K on grids smaller than the CU count, the
 // partial sums added by gemm_f32.hip's reduce); F32-kernel convolutions run on
 // gemm_f32.hip.  The rest are
 // HBM-bound passes: the conv-transpose kernel repack + F16 cast, the 3x3
-// kernel repacks for the implicit GEMMs, and, for maps the implicit GEMMs do
+// kernel repacks for the implicit GEMMs (one launch for all of a neck's), and, for maps the implicit GEMMs do
 // not take, im2col, the conv-transpose scatter and bias adds; the 2x2
 // max-pool.
 #include "common.cuh"
 #include "kernels.h"
+#include "pack.cuh"
 
 namespace mi355 {
 
@@ -19,18 +20,37 @@ namespace {
 unsigned nblk(int64_t n) { return (unsigned)((n + 255) / 256); }
 }
 
-// ggml conv-transpose kernel [kW=2, kH=2, Cout, Cin] (memory [ci][co][kh][kw]),
-// F32 or F16, -> F16 MUL_MAT weight rows [4*Cout][Cin], row n = (kh*2 + kw)*Cout + co.
-// The F32 -> F16 cast rounds to nearest even, as ggml_cast does
-// (sam3_conv_transpose_weight, sam3.cpp:1087-1090).
+// a conv-transpose kernel's F16 GEMM rows (deconv_pack_block)
 __global__ __launch_bounds__(256) void deconv_pack_kernel(const void* __restrict__ w, int wtype, int Cin, int Cout,
                                                           uint16_t* __restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= 4LL * Cout * Cin) return;
-    const int ci = (int)(i % Cin);
-    const int n = (int)(i / Cin), t = n / Cout, co = n % Cout;
-    const int64_t src = (((int64_t)ci * Cout + co) * 2 + (t >> 1)) * 2 + (t & 1);
-    out[i] = wtype == T_F16 ? static_cast<const uint16_t*>(w)[src] : f2h(static_cast<const float*>(w)[src]);
+    __shared__ uint16_t t[PACK_LDS];
+    deconv_pack_block(blockIdx.x, w, wtype, Cin, Cout, out, t);
+}
+
+// Every kernel of a neck repacked in one launch. Alone each of the seven to eleven repacks moves a few
+// MB in 4 to 17 us, most of it the launch and the latency of one pass of scattered reads; together
+// they overlap. A block serves one repack: the first whose end lies past it.
+namespace {
+struct NeckPacks {
+    NeckPack j[NECK_PACKS];
+    unsigned end[NECK_PACKS];  // block after the repack's last
+    int n;
+};
+}  // namespace
+__global__ __launch_bounds__(256) void neck_pack_kernel(const NeckPacks p) {
+    __shared__ uint16_t t[PACK_LDS];
+    int i = 0;
+    while (i + 1 < p.n && blockIdx.x >= p.end[i]) ++i;
+    const NeckPack& j = p.j[i];
+    const int64_t blk = blockIdx.x - (i ? p.end[i - 1] : 0), it = blk * 256 + threadIdx.x;
+    if (j.k == 2) {
+        deconv_pack_block(blk, j.w, j.type, j.Cin, j.Cout, j.out, t);
+    } else if (j.type == T_F16) {
+        conv3x3_pack_f16_item(it, static_cast<const uint16_t*>(j.w), j.Cin, j.Cout, j.out);
+    } else {
+        const int taps = j.k * j.k, K = taps * j.Cin;
+        split_w_item(it, static_cast<const char*>(j.w), 4LL * K, 0, taps, j.Cout, K, (K + 31) / 32 * 32, j.out);
+    }
 }
 
 // y[(2py + kh)(2W) + 2px + kw][co] = D[py*W + px][(kh*2 + kw)*Cout + co] + b[co]
@@ -90,12 +110,7 @@ __global__ __launch_bounds__(256) void conv3x3_pack_kernel(const float* __restri
 // F16 3x3 kernel [Cout][Cin][3][3] -> rows [Cout][tap][Cin] (the implicit GEMM's K order)
 __global__ __launch_bounds__(256) void conv3x3_pack_f16_kernel(const uint16_t* __restrict__ w, int Cin, int Cout,
                                                                uint16_t* __restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= 9LL * Cin * Cout) return;
-    const int ci = (int)(i % Cin);
-    const int64_t r = i / Cin;
-    const int tap = (int)(r % 9), co = (int)(r / 9);
-    out[i] = w[((int64_t)co * Cin + ci) * 9 + tap];
+    conv3x3_pack_f16_item((int64_t)blockIdx.x * blockDim.x + threadIdx.x, w, Cin, Cout, out);
 }
 
 // ggml_conv_2d_s1_ph (TAPS = 9) or ggml_conv_2d_sk_p0 1x1 (TAPS = 1) with an F16
@@ -603,8 +618,27 @@ __global__ __launch_bounds__(256) void maxpool2_kernel(const void* __restrict__ 
 }
 
 hipError_t launch_deconv_pack(const void* w, int wtype, int Cin, int Cout, uint16_t* out, hipStream_t st) {
-    const int64_t n = 4LL * Cout * Cin;
-    if (n > 0) deconv_pack_kernel<<<nblk(n), 256, 0, st>>>(w, wtype, Cin, Cout, out);
+    const int64_t n = deconv_pack_blocks(Cin, Cout);
+    if (n > 0) deconv_pack_kernel<<<(unsigned)n, 256, 0, st>>>(w, wtype, Cin, Cout, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_neck_pack(const NeckPack* jobs, int n, hipStream_t st) {
+    if (n <= 0) return hipSuccess;
+    if (n > NECK_PACKS) return hipErrorInvalidValue;
+    NeckPacks p{};
+    int64_t end = 0;
+    for (int i = 0; i < n; ++i) {
+        const NeckPack& j = jobs[i];
+        const int64_t K = (int64_t)j.k * j.k * j.Cin;
+        const int64_t items = j.type == T_F16 ? K * j.Cout : (K + 31) / 32 * 4 * j.Cout;
+        end += j.k == 2 ? deconv_pack_blocks(j.Cin, j.Cout) : (items + 255) / 256;
+        p.j[i] = j;
+        p.end[i] = (unsigned)end;
+    }
+    p.n = n;
+    if (end > 0x7fffffff) return hipErrorInvalidValue;
+    neck_pack_kernel<<<(unsigned)end, 256, 0, st>>>(p);
     return hipGetLastError();
 }
 
