@@ -615,7 +615,6 @@ mi355_status mi355_hiera_encode(mi355_context* ctx, const mi355_hiera_hparams* h
     (void)hipSetDevice(ctx->device);
     Bufs b;
     TRY(get_bufs(ctx, hp, infos, &b));
-    hipStream_t st = ctx->stream;
     const int S0 = hp->img_size / 4;
     TRY(patch_embed(ctx, hp, image, patch_w, patch_b, pos_embed, b, b.x0));
     float* cur = b.x0;
