@@ -403,18 +403,10 @@ mi355_status mul_mat_run(mi355_context* ctx, const mi355_tensor* s0, const mi355
                      "mmq launch");
 }
 
-// Scratch of the F32 MUL_MAT's split weight (its bf16 planes), 0 where it runs without: batches
-// and short K keep the fp32 MFMA kernels.
-size_t f32_split_scratch(const mi355_tensor* s0, const mi355_tensor* s1) {
-    if (s0->type != T_F32 || s0->layout != MI355_LAYOUT_GGML || s1->ne[2] * s1->ne[3] != 1 || s0->ne[0] < F32_SPLIT_MIN_K)
-        return 0;
-    return align_up(gemm_f32_split_bytes(s0->ne[1], s0->ne[0]));
-}
-
-// MUL_MAT with F32 weights: the bf16-MFMA GEMM over the weight's planes where the operands fit it
-// and the scratch ws holds them, else the fp32 MFMA GEMM, which needs none.
+// MUL_MAT with F32 weights: the fp32 MFMA GEMM, no workspace. (On the bf16 planes of the neck's
+// convolutions, which are as exact, it would need six bytes of scratch per weight on each call.)
 mi355_status mul_mat_f32(mi355_context* ctx, const mi355_tensor* s0, const mi355_tensor* s1, const mi355_tensor* d,
-                         char* ws, size_t ws_bytes, bool timed) {
+                         bool timed) {
     GemmF32Args g;
     g.W = static_cast<const float*>(s0->data);
     g.w_nb1 = s0->nb[1]; g.w_nb2 = s0->nb[2]; g.w_nb3 = s0->nb[3];
@@ -426,15 +418,6 @@ mi355_status mul_mat_f32(mi355_context* ctx, const mi355_tensor* s0, const mi355
     g.ne12 = (int)s1->ne[2];
     g.r2 = (int)(s1->ne[2] / s0->ne[2]);
     g.r3 = (int)(s1->ne[3] / s0->ne[3]);
-    const size_t need = f32_split_scratch(s0, s1);
-    if (need && ws && need <= ws_bytes && gemm_f32_split_ok(g, 1)) {
-        Timed tw(timed ? ctx : nullptr, "split_w");
-        const mi355_status st = hip_check(ctx, tw.done(launch_split_w(g.W, g.w_nb1, false, 1, g.N, g.K,
-                                                                      reinterpret_cast<uint16_t*>(ws), ctx->stream)),
-                                          "split_w launch");
-        if (st != MI355_STATUS_SUCCESS) return st;
-        g.wsplit = reinterpret_cast<const uint16_t*>(ws);
-    }
     Timed tg(timed ? ctx : nullptr, "gemm_f32");
     return hip_check(ctx, tg.done(launch_gemm_f32(g, (int)(s1->ne[2] * s1->ne[3]), ctx->stream)), "gemm_f32 launch");
 }
@@ -472,15 +455,6 @@ mi355_status mul_mat_epi(mi355_context* ctx, const mi355_tensor* s0, const ActF1
     d.nb[2] = d.nb[3] = d.nb[1] * a.M;
     d.data = e.kind == MMQ_EPI_RESIDUAL ? static_cast<void*>(e.out) : static_cast<void*>(e.q);
     return mul_mat_act(ctx, s0, a, &d, &e);
-}
-
-mi355_status mul_mat_f32_in(mi355_context* ctx, const mi355_tensor* s0, const mi355_tensor* s1, const mi355_tensor* d,
-                            void* scratch, size_t scratch_bytes) {
-    const mi355_status st = check_mul_mat(ctx, s0, s1, d);
-    if (st != MI355_STATUS_SUCCESS) return st;
-    if (s0->type != T_F32 || s0->ne[0] == 0 || s0->ne[1] == 0 || s1->ne[1] == 0 || f32_split_scratch(s0, s1) > scratch_bytes)
-        return mi355_mul_mat(ctx, s0, s1, d);
-    return mul_mat_f32(ctx, s0, s1, d, static_cast<char*>(scratch), scratch_bytes, true);
 }
 
 // mul_mat_act for a prepared weight: the int8 kernel over an ACT_I8 / ACT_I8S operand.
@@ -754,7 +728,6 @@ size_t mi355_mul_mat_workspace_size(const mi355_tensor* s0, const mi355_tensor* 
     // the most any MUL_MAT route (mi355_context_set_mmq_kernel) needs
     const int cus = device_cus(dev);
     size_t bytes = 0;
-    if (s0->type == T_F32) return f32_split_scratch(s0, s1);
     for (int k : {MI355_MMQ_F16, MI355_MMQ_INT8, MI355_MMQ_AUTO}) bytes = std::max(bytes, mm_plan(s0, s1, cus, true, k).total());
     return bytes;
 }
@@ -808,17 +781,7 @@ mi355_status mi355_mul_mat(mi355_context* ctx, const mi355_tensor* s0, const mi3
     if (!ctx) return fail(nullptr, MI355_STATUS_INVALID_ARG, "mul_mat: null context");
     (void)hipSetDevice(ctx->device);
     if (s0->ne[0] == 0 || s0->ne[1] == 0 || s1->ne[1] == 0 || s1->ne[2] * s1->ne[3] == 0) return MI355_STATUS_SUCCESS;
-    if (s0->type == T_F32) {
-        // the workspace grows for the split weight where it can (not under capture, where no
-        // memory may be allocated); a call it does not fit runs without
-        const size_t need = f32_split_scratch(s0, s1);
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (need > ctx->ws_size &&
-            (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
-             ensure_ws(ctx, need) != MI355_STATUS_SUCCESS))
-            (void)hipGetLastError();
-        return mul_mat_f32(ctx, s0, s1, d, static_cast<char*>(ctx->ws), ctx->ws_size, true);
-    }
+    if (s0->type == T_F32) return mul_mat_f32(ctx, s0, s1, d, true);
     MmPlan pl = mm_plan(s0, s1, ctx->cus, dst_split_ok(d), mm_route(s0, s1, ctx->mmq_kernel));
     if (pl.total() > ctx->ws_size) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -837,13 +800,7 @@ mi355_status mi355_mul_mat_noalloc(mi355_context* ctx, const mi355_tensor* s0, c
     if (!ctx) return fail(nullptr, MI355_STATUS_INVALID_ARG, "mul_mat_noalloc: null context");
     (void)hipSetDevice(ctx->device);
     if (s0->ne[0] == 0 || s0->ne[1] == 0 || s1->ne[1] == 0 || s1->ne[2] * s1->ne[3] == 0) return MI355_STATUS_SUCCESS;
-    if (s0->type == T_F32) {
-        const size_t need = f32_split_scratch(s0, s1);
-        if (!need || need > MI355_NOALLOC_SCRATCH_BYTES || !ctx->scratch) return mul_mat_f32(ctx, s0, s1, d, nullptr, 0, false);
-        return noalloc_run(ctx, [&] {
-            return mul_mat_f32(ctx, s0, s1, d, static_cast<char*>(ctx->scratch), MI355_NOALLOC_SCRATCH_BYTES, false);
-        });
-    }
+    if (s0->type == T_F32) return mul_mat_f32(ctx, s0, s1, d, false);
     if (!ctx->scratch)
         return fail(ctx, MI355_STATUS_FAILED, "mul_mat_noalloc: no static scratch on device %d (%s)", ctx->device,
                     ctx->scratch_error.c_str());

@@ -88,11 +88,6 @@ mi355_status flash_attn_act(mi355_context* ctx, const mi355_tensor* q, const mi3
 // exists.
 mi355_status mul_mat_epi(mi355_context* ctx, const mi355_tensor* s0, const ActF16& a, const MmqEpi& e);
 
-// mi355_mul_mat with F32 weights whose split planes may use the caller's device scratch (256-byte
-// aligned) instead of the context's workspace; where it is too small the call is mi355_mul_mat's.
-mi355_status mul_mat_f32_in(mi355_context* ctx, const mi355_tensor* s0, const mi355_tensor* s1, const mi355_tensor* d,
-                            void* scratch, size_t scratch_bytes);
-
 // Resolves the device address of the static scratch array of
 // mi355_mul_mat_noalloc on ctx's device (current) into ctx->scratch; the
 // lookup runs once per device.

@@ -16,9 +16,10 @@
 // are walked XCD-aware (each XCD a contiguous band), so the n-tiles of one
 // m-tile read their activation rows through one L2.
 //
-// gemm_f32_split_kernel is the form that most calls take (2-D, K >= 128 in a MUL_MAT, every neck
-// convolution, both patch embeddings): each fp32 value as three bf16 ones on the bf16 matrix
-// cores. The kernels above it serve batches, short K and what its buffer offsets don't reach.
+// gemm_f32_split_kernel is the form that the neck's convolutions and Hiera's patch embedding take,
+// which have scratch for its weight planes: each fp32 value as three bf16 ones on the bf16 matrix
+// cores. The kernels above it serve every MUL_MAT, which takes no scratch, and what its buffer
+// offsets don't reach.
 //
 // The same kernel runs a 3x3 / stride-1 / pad-1 convolution as an implicit
 // GEMM over a token-major [H*W][C] map (C % 32 == 0): a stage of 32 K values

@@ -245,10 +245,6 @@ struct GemmF32Args {
 // gemm_f32_split_bytes(N, K) bytes at out, 16-byte aligned
 hipError_t launch_split_w(const void* w, int64_t nb1, bool f16, int taps, int N, int K, uint16_t* out, hipStream_t st);
 size_t gemm_f32_split_bytes(int64_t N, int64_t K);
-// below this K a MUL_MAT keeps the fp32 MFMA kernels: the weight's own pass (about 4 us) costs what
-// the matrix cores save (K = 64: 9.3 -> 12.5 us at 1 x 256, 13.6 -> 14.5 at 5184 x 256; K = 128:
-// 16.9 -> 15.9 at 577 x 192; K = 256: 21.1 -> 19.3 at 1 x 256)
-constexpr int F32_SPLIT_MIN_K = 128;
 // whether the shapes and alignments of a (Z batches) fit the bf16-MFMA kernel
 bool gemm_f32_split_ok(const GemmF32Args& a, int Z);
 hipError_t launch_gemm_f32(const GemmF32Args& a, int Z, hipStream_t st);

@@ -271,10 +271,7 @@ mi355_status mi355_vit_prefix(mi355_context* ctx, const mi355_vit_hparams* hp, c
     w.nb[2] = w.nb[3] = w.nb[1] * E;
     const mi355_tensor cols = dev_tensor(b.big, T_F32, K, M);
     const mi355_tensor out = dev_tensor(b.xn, T_F32, E, M);
-    // an F32 weight's planes go where the blocks' attention operands will be, from qkv to big
-    st = w.type == T_F32 ? mul_mat_f32_in(ctx, &w, &cols, &out, b.qkv,
-                                          (size_t)(reinterpret_cast<char*>(b.big) - reinterpret_cast<char*>(b.qkv)))
-                         : mi355_mul_mat(ctx, &w, &cols, &out);
+    st = mi355_mul_mat(ctx, &w, &cols, &out);
     if (st != MI355_STATUS_SUCCESS) return st;
     return mi355_vit_layer_norm(ctx, b.xn, pos_embed, hp->pos_grid, ln_pre_w, ln_pre_b, x, M, E, G, 0, hp->eps);
 }

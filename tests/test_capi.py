@@ -152,6 +152,13 @@ def test_workspace_size(mi):
     assert mi.lib().mi355_mul_mat_workspace_size(C.byref(s0), C.byref(s1)) >= 4736 * 1024
 
 
+@pytest.mark.parametrize("K,N,M", [(588, 1024, 5184), (4736, 1024, 1), (1023, 64, 7)])
+def test_workspace_size_of_f32_is_zero(mi, K, N, M):
+    """F32 MUL_MATs use no library memory."""
+    s0, s1, d = mm(mi, t0=0, K=K, N=N, M=M)
+    assert mi.lib().mi355_mul_mat_workspace_size(C.byref(s0), C.byref(s1)) == 0
+
+
 def test_every_entry_point_rejects_null_arguments(mi):
     """Every entry point called with a NULL context / handle and null or zero
     arguments returns an error status (sizes return 0; the frees and the

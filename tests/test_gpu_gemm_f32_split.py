@@ -1,9 +1,9 @@
-"""F32 MUL_MATs and neck convolutions on the bf16-MFMA kernel (each fp32 value
-as three bf16 ones, six products): against float64, at the edges of its tiles
-(128 x 128, 32 of K), its K remainders and its K split, and with infinities
+"""F32 MUL_MATs (fp32 MFMAs) and neck convolutions on the bf16-MFMA kernel (each
+fp32 value as three bf16 ones, six products): against float64, at the edges of
+their tiles (128 x 128, 32 of K), K remainders and K split, and with infinities
 and NaN.
 
-Bound: an output adds six products per 32 of K into an fp32 accumulator, each
+Bound, of the bf16-MFMA kernel, which the fp32 sums stay below too: an output adds six products per 32 of K into an fp32 accumulator, each
 addition rounding by at most 2^-23 of a running sum that stays below
 S = sum |w x|, and drops three products of at most 2^-24 S each:
 (6 ceil(K / 32) + 4) 2^-23 S; a K split adds one rounding per range."""
