@@ -16,10 +16,10 @@
 // are walked XCD-aware (each XCD a contiguous band), so the n-tiles of one
 // m-tile read their activation rows through one L2.
 //
-// gemm_f32_split_kernel is the form that the neck's convolutions and Hiera's patch embedding take,
-// which have scratch for its weight planes: each fp32 value as three bf16 ones on the bf16 matrix
-// cores. The kernels above it serve every MUL_MAT, which takes no scratch, and what its buffer
-// offsets don't reach.
+// gemm_f32_split_kernel is the form that the neck's convolutions take: each fp32 value as three
+// bf16 ones on the bf16 matrix cores. The kernels above it serve the MUL_MATs, which take no scratch
+// for its weight planes, the patch embeddings (the encoders' quantizers turn a last-bit difference
+// into a flipped quant), and what its buffer offsets don't reach.
 //
 // The same kernel runs a 3x3 / stride-1 / pad-1 convolution as an implicit
 // GEMM over a token-major [H*W][C] map (C % 32 == 0): a stage of 32 K values

@@ -199,7 +199,7 @@ Sizes all_sizes(const mi355_hiera_hparams* hp, const std::vector<Info>& infos) {
     }
     const size_t S0 = (size_t)(hp->img_size / 4);
     z.cols = S0 * S0 * PATCH_KP * 4;
-    z.w32 = gemm_f32_split_bytes(hp->embed_dim, PATCH_KP);  // (the zero-padded fp32 rows are smaller)
+    z.w32 = (size_t)PATCH_KP * hp->embed_dim * 4;
     z.x = std::max(z.x, S0 * S0 * (size_t)hp->embed_dim * 4);
     return z;
 }
@@ -495,6 +495,7 @@ mi355_status patch_embed(mi355_context* ctx, const mi355_hiera_hparams* hp, cons
         TRY(hip_check(ctx, t.done(launch_im2col_pad(image, b.cols, 3, IMG, IMG, 7, 7, 4, 3, S0, S0, PATCH_KP, w16, st)),
                       "im2col launch"));
     }
+    TRY(hip_check(ctx, launch_pad_rows_f32(patch_w->data, w16, E, 147, PATCH_KP, b.w32, st), "patch weight pad"));
     GemmF32Args g;
     g.W = b.w32;
     g.w_nb1 = 4LL * PATCH_KP;
@@ -511,13 +512,6 @@ mi355_status patch_embed(mi355_context* ctx, const mi355_hiera_hparams* hp, cons
     g.ne12 = g.r2 = g.r3 = 1;
     g.bias = patch_b;
     g.add = pos_embed;
-    if (gemm_f32_split_ok(g, 1)) {
-        uint16_t* planes = reinterpret_cast<uint16_t*>(b.w32);
-        TRY(hip_check(ctx, launch_split_w(patch_w->data, patch_w->nb[3], w16, 1, E, 147, planes, st), "patch weight split"));
-        g.wsplit = planes;
-    } else {
-        TRY(hip_check(ctx, launch_pad_rows_f32(patch_w->data, w16, E, 147, PATCH_KP, b.w32, st), "patch weight pad"));
-    }
     Timed t(ctx, "gemm_f32");
     return hip_check(ctx, t.done(launch_gemm_f32(g, 1, st)), "gemm_f32 launch");
 }

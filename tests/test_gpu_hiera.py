@@ -138,6 +138,24 @@ def test_hiera_prefix(mi, ctx, orc, img_size, wtype):
     assert (err <= tol).all(), float((err / tol).max())
 
 
+@pytest.mark.parametrize("scale", [1.0, 1e-36, 2e-38])
+def test_hiera_prefix_error_at_every_magnitude(mi, ctx, orc, scale):
+    """An F32 patch embedding sums its 147 terms in fp32 whatever their magnitude: rms error of
+    sqrt(147) roundings of 2^-24 each (bias and pos_embed zero, kernel entries of order 64)."""
+    hp, E, S0 = mi.hiera_tiny(128), 96, 32
+    img = (orc.uniform(3 * 128 * 128, 14, 1) * np.float32(scale)).reshape(3, 128, 128)
+    pw = (orc.normal(E * 147, 14, 2) * np.float32(64)).reshape(E, 147)
+    imgd, wd, zero = dev(img), dev(pw), torch.zeros(S0 * S0 * E, device="cuda")
+    x = torch.full((S0 * S0, E), float("nan"), dtype=torch.float32, device="cuda")
+    ctx.hiera_prefix(hp, _p(imgd), mi.from_torch(wd, mi.F32, [7, 7, 3, E]), _p(zero), _p(zero), _p(x))
+    ctx.synchronize()
+    pad = np.pad(img, ((0, 0), (3, 3), (3, 3))).astype(np.float64)
+    win = np.lib.stride_tricks.sliding_window_view(pad, (7, 7), axis=(1, 2))[:, ::4, ::4][:, :S0, :S0]
+    ref = win.transpose(1, 2, 0, 3, 4).reshape(S0 * S0, 147) @ pw.astype(np.float64).T
+    err = np.sqrt(np.mean((x.cpu().numpy() - ref) ** 2) / np.mean(ref ** 2))
+    assert err <= 147 ** 0.5 * 2.0 ** -24, err
+
+
 def test_hiera_encode_patch_and_stages(mi, ctx, orc):
     """Whole backbone at 128x128 (Q4_0): every stage output is finite and a
     second run reproduces it bit for bit; the stage-0 output (block 0 on the
