@@ -115,10 +115,10 @@ __device__ __forceinline__ uint2 lds_read_tr16(const void* a) {
 // several times more windows are in flight; the arithmetic per query is the same.
 // KDMA: fp16 K and V with 16-byte rows reach LDS by DMA (buffer_load ... lds) and the loop
 // is software-pipelined; otherwise they pass through registers.
-// RESET (key-split launches): halfway through its range a workgroup takes the reference of the
-// probabilities anew from that tile's own maximum, as at the range's start, rescaling O and the
-// sums. The largest probability of each half is then exactly 1 in fp16, so one workgroup's range
-// is as precise as two ranges of half its length.
+// RESET (a workgroup with several key ranges, fattn_ranges): at the first tile of each further range
+// the reference of the probabilities becomes that tile's own maximum, as at the first one's, O and the
+// sums rescaled. Every probability is then rounded to fp16 against the reference it has when
+// each range has a workgroup of its own; only fp32 roundings differ.
 template <int D, bool QF32, bool KVF32, bool KDMA, int NW = 4, int NBUF = 2, bool RESET = false>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fattn_kernel(const FaArgs p) {
     static_assert(!KDMA || (!KVF32 && (D == 64 || D == 96 || D == 128)), "K/V DMA staging: fp16 K and V, D = 64, 96 or 128");
@@ -336,7 +336,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fattn_kernel(const F
             }
             const float mx = xmax32(fmaxf(fmaxf(m4[0], m4[1]), fmaxf(m4[2], m4[3])));
             float m_new = fmaxf(m_run, mx * c);
-            if (RESET && fresh && m_run - mx * c < 8.0f) m_new = mx * c;  // (a far lower maximum weighs nothing)
+            // (2^64 below the ranges before a key's weight is nothing in fp32, and up to
+            // there the rescaled O stays finite)
+            if (RESET && fresh && m_run - mx * c < 64.0f) m_new = mx * c;
             const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
             m_run = m_new;
             ls = probs(m_new);
@@ -347,6 +349,12 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fattn_kernel(const F
                 for (int e = 0; e < 16; ++e) O[db][e] *= alpha;
         }
         l_run += ls;
+    };
+    int reset_at = p.kv_reset;  // the tile with which the workgroup's next range begins
+    auto fresh_at = [&](int t) {
+        if (t != reset_at) return false;
+        reset_at += p.kv_reset;
+        return true;
     };
     // O^T += V^T P^T over the 64 keys of V buffer vbuf (four 16-key MFMA chunks)
     // V^T fragment rows by transposing reads of the DMA-staged V tile: lane (lr, g) of
@@ -415,7 +423,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fattn_kernel(const F
             if (t + 1 < ntile) dma_v(kv0 + FA_BKV, cb ^ 1);
             if (kv0 + FA_BKV > nkv) mask(Sc, kv0);
             score(cb ^ 1, Sn);  // tile t + 1 (past the last tile: stale LDS, never used)
-            softmax(Sc, P, RESET && t == ntile / 2);
+            softmax(Sc, P, RESET && fresh_at(t));
             pv(cb, P);
         };
         for (int t = 0; t < ntile; t += 2) {
@@ -437,7 +445,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fattn_kernel(const F
             uint32_t P[2][8];
             score(cb, S);
             if (kv0 + FA_BKV > nkv) mask(S, kv0);
-            softmax(S, P, RESET && t == ntile / 2);
+            softmax(S, P, RESET && fresh_at(t));
             pv(cb, P);
             if (NBUF == 2 && t + 1 < ntile) {
                 store_tile(cb ^ 1);
@@ -571,19 +579,29 @@ __global__ __launch_bounds__(256) void fattn_combine_kernel(const FaArgs p, int 
         act_store_chunk(p.out, (int64_t)b * p.nq + qi, (int64_t)p.nh * D, ((int64_t)h * D) / 4 + c, o);
 }
 
-int fattn_kv_split(int nq, int nkv, int nh, int B, int cus) {
+FaRanges fattn_ranges(int nq, int nkv, int nh, int B, int cus) {
     const int64_t wgs = (int64_t)((nq + FA_BQ - 1) / FA_BQ) * nh * B;
     const int ntile = (nkv + FA_BKV - 1) / FA_BKV;
+    FaRanges r{1, nkv, 0};
     // below eight key tiles the combine pass costs more than the idle CUs (Hiera-tiny's 14x14
     // windows, 4 tiles over 200 workgroups: 12.2 us split in two + 7 us combine, against one pass)
-    if (cus <= 0 || wgs >= cus || ntile < 8) return 1;
-    // small grids: about one workgroup per CU and not a few more, since each range costs a pass
-    // over the outputs twice (1 x 4 heads, 1021 x 3999 of 96: 33.8 us in 16 ranges, 26.5 in 8;
-    // 8 heads, 1024 x 1024 of 96: 26.0 in 8, 19.7 in 4; 16 heads, 300 x 5184 of 128: 58.2 in 11,
-    // 40.5 in 5); from a third of the CUs on, two per CU (4 heads, 4096 x 4096 of 96)
-    const int64_t want = wgs * 3 <= cus ? cus / wgs : (2LL * cus + wgs - 1) / wgs;
-    const int ks = (int)std::min<int64_t>(want, ntile / 2);
-    return ks < 2 ? 1 : std::min(ks, 16);
+    if (cus <= 0 || wgs >= cus || ntile < 8) return r;
+    const int64_t want = (2LL * cus + wgs - 1) / wgs;
+    const int ks = (int)std::min<int64_t>({want, ntile / 2, 16}), per = (ntile + ks - 1) / ks;
+    r.split = (ntile + per - 1) / per;  // no empty range
+    r.chunk = per * FA_BKV;
+    // small grids of more workgroups than there are CUs: several ranges to a workgroup, so that one
+    // pass over the CUs serves them, since the combine writes and reads every workgroup's output once
+    // more (4 heads, 1021 x 3999 of 96: 32 us with a workgroup per range, 25 with two ranges to a
+    // workgroup; 8 heads, 1024 x 1024 of 96: 25 and 19; 16 heads, 300 x 5184 of 128: 58, 65 with two,
+    // which is 288 workgroups, 47 with three)
+    if (wgs * 3 <= cus && r.split * wgs > cus) {
+        const int n = cus / (int)wgs, m = (r.split + n - 1) / n;
+        r.split = (r.split + m - 1) / m;
+        r.chunk *= m;
+        r.reset = per;
+    }
+    return r;
 }
 
 size_t fattn_part_bytes(int D, int nq, int nh, int B, int kv_split) {
@@ -596,9 +614,9 @@ static void fa_launch_d(const FaArgs& a, bool qf32, bool kvf32, int B, hipStream
     const int64_t items = (int64_t)((a.nq + FA_BQ - 1) / FA_BQ) * a.nh * B * a.kv_split;
     const dim3 grid((unsigned)((items + 7) / 8 * 8));
     bool launched = false;
-    auto go = [&](auto whole, auto range) {
-        if (a.kv_split > 1) range<<<grid, FA_NT, 0, st>>>(a);
-        else whole<<<grid, FA_NT, 0, st>>>(a);
+    auto go = [&](auto one, auto several) {
+        if (a.kv_reset > 0) several<<<grid, FA_NT, 0, st>>>(a);
+        else one<<<grid, FA_NT, 0, st>>>(a);
     };
     // windows of at most one key tile and 64 queries, fp16 operands, no key split: one or two
     // wavefronts per workgroup and one K/V buffer (taken before the DMA path, which would
@@ -645,7 +663,7 @@ hipError_t launch_fattn(const FaArgs& a_in, int D, bool qf32, bool kvf32, int B,
         return hipErrorInvalidValue;
     FaArgs a = a_in;
     a.B = B;
-    if (a.kv_split < 1 || a.kv_split > 16 || (a.kv_split > 1 && (!a.part || a.kv_chunk % FA_BKV != 0 ||
+    if (a.kv_split < 1 || a.kv_split > 16 || (a.kv_reset > 0 && a.kv_split == 1) || (a.kv_split > 1 && (!a.part || a.kv_chunk % FA_BKV != 0 ||
                                               (int64_t)(a.kv_split - 1) * a.kv_chunk >= a.nkv)))
         return hipErrorInvalidValue;
     switch (D) {

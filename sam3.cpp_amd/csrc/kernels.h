@@ -211,9 +211,13 @@ struct FaArgs {
     int kv_split, kv_chunk;     // keys split into kv_split ranges of kv_chunk (a multiple of 64);
     float* part;                // > 1: per range unnormalised O [D] and (max, sum) per query,
                                 // combined by a second kernel; fattn_part_bytes() of workspace
+    int kv_reset;               // > 0: a chunk holds several ranges of this many 64-key tiles
 };
-// Key-range split for grids too small to fill the GPU (1 = none), and its workspace.
-int fattn_kv_split(int nq, int nkv, int nh, int B, int cus);
+// Key ranges for grids too small to fill the GPU (split 1: none), and their workspace.
+struct FaRanges {
+    int split, chunk, reset;    // FaArgs' kv_split, kv_chunk, kv_reset
+};
+FaRanges fattn_ranges(int nq, int nkv, int nh, int B, int cus);
 size_t fattn_part_bytes(int D, int nq, int nh, int B, int kv_split);
 hipError_t launch_fattn(const FaArgs& a, int D, bool qf32, bool kvf32, int B, hipStream_t st);
 
