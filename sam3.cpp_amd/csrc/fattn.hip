@@ -535,8 +535,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fattn_kernel(const F
 // Key-split combine: thread per (batch, head, query, 4 outputs); m* = max of the
 // ranges' maxima, O = sum_s 2^(m_s - m*) O_s, l likewise, out = O / l.  The
 // operand output keeps 8 consecutive threads on one 32-block.  Bound by the partial outputs it
-// reads and by their latency, so the loads of all (at most KS) ranges are issued before the
-// first is used; with the ranges in a runtime loop each one's latency was paid in turn.
+// reads and by their latency: up to eight ranges' loads are all issued before the first is used
+// (KS of them; 2 heads, 700 x 700 of 128 in 5 ranges 15.4 us with the loop over them, 14.4 so).
+// KS = 0 is the loop, for more ranges: sixteen loads and their registers leave too few wavefronts
+// (4 heads, 640 x 1500 of 128 in 12 ranges 28.1 us, 24.5 with the loop).
 template <int D, int KS>
 __global__ __launch_bounds__(256) void fattn_combine_kernel(const FaArgs p, int B) {
     constexpr int CPR = D / 4;
@@ -548,28 +550,38 @@ __global__ __launch_bounds__(256) void fattn_combine_kernel(const FaArgs p, int 
     const int qi = (int)(pr % p.nq), h = (int)((pr / p.nq) % p.nh), b = (int)(pr / ((int64_t)p.nq * p.nh));
     const float* ml = p.part + (int64_t)p.kv_split * rows * D + 2 * pr;
     const float* po = p.part + pr * D + 4 * c;
-    v2f m[KS];
-    v4f v[KS];
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-        m[s] = v2f{-__builtin_inff(), 0.0f};
-        v[s] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        if (s < p.kv_split) {
-            m[s] = *reinterpret_cast<const v2f*>(&ml[2 * s * rows]);
-            v[s] = *reinterpret_cast<const v4f*>(&po[s * rows * D]);
-        }
-    }
-    float mx = m[0][0];
-#pragma unroll
-    for (int s = 1; s < KS; ++s) mx = fmaxf(mx, m[s][0]);
     float l = 0.0f;
     v4f o = {0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (KS == 0) {
+        float mx = -__builtin_inff();
+        for (int s = 0; s < p.kv_split; ++s) mx = fmaxf(mx, ml[2 * s * rows]);
+        for (int s = 0; s < p.kv_split; ++s) {
+            const float wgt = __builtin_amdgcn_exp2f(ml[2 * s * rows] - mx);
+            l = l + wgt * ml[2 * s * rows + 1];
+            o = o + wgt * *reinterpret_cast<const v4f*>(&po[s * rows * D]);
+        }
+    } else {
+        v2f m[KS];
+        v4f v[KS];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-        if (s >= p.kv_split) break;
-        const float wgt = __builtin_amdgcn_exp2f(m[s][0] - mx);
-        l = l + wgt * m[s][1];
-        o = o + wgt * v[s];
+        for (int s = 0; s < KS; ++s) {
+            m[s] = v2f{-__builtin_inff(), 0.0f};
+            v[s] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            if (s < p.kv_split) {
+                m[s] = *reinterpret_cast<const v2f*>(&ml[2 * s * rows]);
+                v[s] = *reinterpret_cast<const v4f*>(&po[s * rows * D]);
+            }
+        }
+        float mx = m[0][0];
+#pragma unroll
+        for (int s = 1; s < KS; ++s) mx = fmaxf(mx, m[s][0]);
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            if (s >= p.kv_split) break;
+            const float wgt = __builtin_amdgcn_exp2f(m[s][0] - mx);
+            l = l + wgt * m[s][1];
+            o = o + wgt * v[s];
+        }
     }
     const float inv = l == 0.0f ? 0.0f : 1.0f / l;
     o = o * inv;
@@ -650,10 +662,9 @@ static void fa_launch_d(const FaArgs& a, bool qf32, bool kvf32, int B, hipStream
     if (a.kv_split > 1) {
         const int64_t n = (int64_t)B * a.nh * a.nq * (D / 4);
         const unsigned g = (unsigned)((n + 255) / 256);
-        if (a.kv_split <= 2) fattn_combine_kernel<D, 2><<<g, 256, 0, st>>>(a, B);
-        else if (a.kv_split <= 4) fattn_combine_kernel<D, 4><<<g, 256, 0, st>>>(a, B);
+        if (a.kv_split <= 4) fattn_combine_kernel<D, 4><<<g, 256, 0, st>>>(a, B);
         else if (a.kv_split <= 8) fattn_combine_kernel<D, 8><<<g, 256, 0, st>>>(a, B);
-        else fattn_combine_kernel<D, 16><<<g, 256, 0, st>>>(a, B);
+        else fattn_combine_kernel<D, 0><<<g, 256, 0, st>>>(a, B);
     }
 }
 
