@@ -241,7 +241,8 @@ struct GemmF32Args {
     // part_bytes) and are then added in split order, with the bias, by a reduce pass
     float* part = nullptr;
     size_t part_bytes = 0;
-    // optional: W as launch_split_w's planes (conv: taps = 9), for the bf16-MFMA kernel; W is then not read
+    // optional: W as launch_split_w's planes (conv: taps = 9), for the bf16-MFMA kernel; W is then the
+    // kernel in file order, read where an output is not finite
     const uint16_t* wsplit = nullptr;
 };
 // The planes of weight rows [N][K] (row pitch nb1 bytes, F32 or F16; taps = 9: a 3x3 kernel

@@ -159,7 +159,7 @@ mi355_status conv(mi355_context* ctx, const mi355_tensor* w, const float* b, con
         return fail(ctx, MI355_STATUS_FAILED, "neck_conv: fp16 maps off the implicit F16 path");
     if (w->type == T_F32 && aligned && (k == 1 || implicit_ok(x, Cin))) {
         GemmF32Args g;
-        g.W = k == 3 ? reinterpret_cast<const float*>(scratch) : static_cast<const float*>(w->data);
+        g.W = static_cast<const float*>(w->data);
         // the K split's partial sums follow the kernel's planes (or its repacked rows)
         g.part = reinterpret_cast<float*>(scratch + align_up(gemm_f32_split_bytes(Cout, K)));
         g.part_bytes = gemm_f32_part_bytes(P, Cout, K);
@@ -189,6 +189,7 @@ mi355_status conv(mi355_context* ctx, const mi355_tensor* w, const float* b, con
                                "conv kernel split");
             }
         } else if (k == 3) {
+            g.W = reinterpret_cast<const float*>(scratch);
             Timed t(ctx, "neck_conv3x3_pack");
             st = hip_check(ctx, t.done(launch_conv3x3_pack(static_cast<const float*>(w->data), Cin, Cout,
                                                            reinterpret_cast<float*>(scratch), ctx->stream)),

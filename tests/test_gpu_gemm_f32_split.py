@@ -7,6 +7,8 @@ Bound, of the bf16-MFMA kernel, which the fp32 sums stay below too: an output ad
 addition rounding by at most 2^-23 of a running sum that stays below
 S = sum |w x|, and drops three products of at most 2^-24 S each:
 (6 ceil(K / 32) + 4) 2^-23 S; a K split adds one rounding per range."""
+from time import perf_counter
+
 import numpy as np
 import pytest
 import torch
@@ -107,3 +109,29 @@ def test_neck_conv_f32_split(mi, ctx, H, W, Cin, Cout, k, special):
     assert np.array_equal(np.isinf(got), np.isinf(ref)) and np.array_equal(got[~fin], ref[~fin])
     err = np.abs(got[fin] - (ref + b)[fin])
     assert (err <= _bound(Cin * k * k, s[fin], 20) + 2.0 ** -23 * (np.abs(ref[fin]) + np.abs(np.broadcast_to(b, ref.shape)[fin]))).all()
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_neck_conv_f32_non_finite_takes_no_hundredfold(mi, ctx, value):
+    """Outputs that are not finite are summed again by the whole wavefront: one infinite pixel makes
+    a 72 x 72 call some three times as long (the other wavefronts wait), not a hundred times."""
+    H, C = 72, 256
+    g = torch.Generator(device="cuda").manual_seed(1)
+    w, b = torch.randn((C, C, 3, 3), generator=g, device="cuda"), torch.zeros(C, device="cuda")
+    x, y = torch.randn((H * H, C), generator=g, device="cuda"), torch.empty((H * H, C), device="cuda")
+
+    def time():
+        best = float("inf")
+        for _ in range(5):
+            ctx.synchronize()
+            t = perf_counter()
+            for _ in range(4):
+                ctx.neck_conv(mi.from_torch(w, mi.F32, [3, 3, C, C]), b.data_ptr(), x.data_ptr(), H, H, y.data_ptr())
+            ctx.synchronize()
+            best = min(best, perf_counter() - t)
+        return best
+
+    finite = time()
+    x[H * H // 2 + 5, 3] = value
+    assert time() <= 15 * finite
+    assert int((~torch.isfinite(y)).sum()) == 9 * C
