@@ -438,19 +438,26 @@ void gemm_f32_dma_kernel(const GemmF32Args p, int ksplit, int sps) {
 //
 // The weights come split already (split_w_kernel: per row and 32 of K the three planes' 64 bytes
 // side by side, 192 bytes); the activations arrive as fp32 by LDS DMA and are split as the
-// fragments are read, eleven VALU instructions per pair of values. A wavefront therefore owns
+// fragments are read, thirteen VALU instructions per pair of values. A wavefront therefore owns
 // 32 whole rows of the 128 x 128 tile: each value is split once per workgroup, and its rows are
 // read by no other wavefront. Stages of 32 K (16 KB + 24 KB), two buffers, two workgroups per CU.
 //
 // Measured: the 288 x 288 3x3 convolution of 256 channels (97.8 GFLOP, 587 of them as bf16)
-// 1014 -> 489 us (1.2 PFLOP/s of bf16; about 400 without the stage DMA, 370 without the split too:
-// the MFMAs alone run at the chip's power limit), 5184 x 1024 x 588 90 -> 57 us, weight pass included;
-// error against 64 bits 5.7e-7 -> 4.9e-7 at K = 1024. With 32 x 32 x 16 MFMAs 539 us.
+// 904 -> 493 us (1.2 PFLOP/s of bf16; some 90 less without the stage DMA, 120 without the split too:
+// the MFMAs alone run at the chip's power limit; with 32 x 32 x 16 MFMAs 50 more), weight pass
+// included; error against 64 bits 5.0e-7 -> 4.2e-7 at 72 x 72 (K = 2304), 2.1e-7 -> 1.6e-7 of a 1x1 at
+// K = 1024.
+//
+// Both operands are split after an exact multiplication by 2^24 (SPLIT_UP), which the result undoes:
+// fp32 values are multiples of 2^-149, so the planes' lowest bits are normal bf16 values at every
+// magnitude and the sum of three is exact down to the smallest subnormal (unscaled, operands of 1e-36
+// had an rms error of 3e-5). Above 2^104 a value, or 2^80 an output, the sums overflow and the output
+// is summed again as below.
 //
 // Infinities and NaN: a split infinity leaves NaN in m, and an infinite weight times a zero
 // plane is NaN too, so any output that is not finite is summed again in fp32 from the unsplit
 // operands, a wavefront's sixteen rows at a time on fp32 MFMAs, until those outputs are done or NaN.
-// Among finite operands only activations that round up to an infinite bf16 need it. 3x3 convolution
+// 3x3 convolution
 // of 256 channels, 288 x 288 / 72 x 72: finite 566 / 56 us, one infinite pixel 724 / 155, a map of
 // NaN 659 / 118.
 namespace {
@@ -460,12 +467,12 @@ struct SplitStage {
     uint16_t B[TN * 96];  // row: plane p (h, m, l), 32 K each; chunk q of plane p in slot 4 p + (q ^ (row >> 2 & 3))
 };
 constexpr int SPLIT_NL = 10;  // DMA instructions per wavefront and stage: 4 activation, 6 weight
-// eight fp32 values -> their three bf16 planes
+// eight fp32 values, times SPLIT_UP -> their three bf16 planes
 __device__ __forceinline__ void split8(const v4f (&x)[2], v8b& h, v8b& m, v8b& l) {
     v4i hh, mm, ll;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const float a = x[i >> 1][2 * (i & 1)], b = x[i >> 1][2 * (i & 1) + 1];
+        const float a = SPLIT_UP * x[i >> 1][2 * (i & 1)], b = SPLIT_UP * x[i >> 1][2 * (i & 1) + 1];
         const uint32_t u = pk_bf16(a, b);
         const float ra = a - __uint_as_float(u << 16), rb = b - __uint_as_float(u & 0xffff0000u);
         const uint32_t v = pk_bf16(ra, rb);
@@ -662,6 +669,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const GemmF32Arg
         if (s + 1 < nst) stage(s + 1, a1, a0);
     }
 
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[i][j][r] *= 1.0f / SPLIT_UP / SPLIT_UP;
     // outputs that are not finite: their sixteen rows again on fp32 MFMAs from the unsplit operands
 #pragma unroll
     for (int i = 0; i < 2; ++i) {

@@ -12,9 +12,13 @@ __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, v2b));
 }
 
-// item i of the planes of weight rows [N][K] (row pitch nb1 bytes; F32 or F16; or, taps == 9, a 3x3
-// kernel [N][C][3][3] read in (tap, channel) order) -> [N][KP / 32][3][32] bf16, zero past K: eight
-// consecutive K
+// The factor, exact in fp32, by which both operands of the split GEMM are multiplied before they are
+// split: the lowest plane of the smallest fp32 values is then a normal bf16.
+constexpr float SPLIT_UP = 16777216.0f;
+
+// item i of the planes of SPLIT_UP times weight rows [N][K] (row pitch nb1 bytes; F32 or F16; or,
+// taps == 9, a 3x3 kernel [N][C][3][3] read in (tap, channel) order) -> [N][KP / 32][3][32] bf16, zero
+// past K: eight consecutive K
 __device__ __forceinline__ void split_w_item(int64_t i, const char* __restrict__ w, int64_t nb1, int f16, int taps, int N, int K,
                                              int KP, uint16_t* __restrict__ out) {
     const int k8 = KP / 8;
@@ -31,15 +35,8 @@ __device__ __forceinline__ void split_w_item(int64_t i, const char* __restrict__
             const char* row = w + (int64_t)n * nb1;
             x = f16 ? h2f(reinterpret_cast<const uint16_t*>(row)[e]) : reinterpret_cast<const float*>(row)[e];
         }
-        const uint32_t u = __float_as_uint(x);
-        uint32_t a = pk_bf16(x, 0.0f) & 0xffffu;
-        if ((a & 0x7f80u) == 0x7f80u) a = u >> 16;  // infinite, NaN, or rounded up to infinity: the top bits
-        if ((u & 0x7f800000u) == 0x7f800000u) {
-            if (u & 0x007fffffu) a |= 0x40u;  // a NaN stays one
-            h[j] = (uint16_t)a;
-            m[j] = l[j] = 0;
-            continue;
-        }
+        x *= SPLIT_UP;
+        const uint32_t a = pk_bf16(x, 0.0f) & 0xffffu;
         const float r = x - __uint_as_float(a << 16);
         const uint32_t b = pk_bf16(r, 0.0f) & 0xffffu;
         h[j] = (uint16_t)a;

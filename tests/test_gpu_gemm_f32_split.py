@@ -135,3 +135,26 @@ def test_neck_conv_f32_non_finite_takes_no_hundredfold(mi, ctx, value):
     x[H * H // 2 + 5, 3] = value
     assert time() <= 15 * finite
     assert int((~torch.isfinite(y)).sum()) == 9 * C
+
+
+@pytest.mark.parametrize("xs,ws", [(1.0, 1.0), (1e-36, 1.0), (1.0, 1e-36), (2e-38, 64.0), (1e-42, 1e6), (1e6, 1e-42), (1e-20, 1e-13),
+                                   (1e30, 1e-30), (1e33, 1e-3), (1e-3, 1e33), (1e20, 1e10)])
+@pytest.mark.parametrize("k,Cin,Cout", [(1, 588, 140), (3, 64, 36)])
+def test_neck_conv_f32_error_at_every_magnitude(mi, ctx, k, Cin, Cout, xs, ws):
+    """rms error of sqrt(K) roundings of 2^-24 each, from subnormal operands to outputs of 1e33."""
+    H, W, K = 13, 11, k * k * Cin
+    rng = np.random.default_rng(17)
+    w = (rng.standard_normal((Cout, Cin, k, k)) * ws).astype(np.float32)
+    x = (rng.standard_normal((H, W, Cin)) * xs).astype(np.float32)
+    wd, bd, xd = torch.from_numpy(w).cuda(), torch.zeros(Cout, device="cuda"), torch.from_numpy(x).cuda()
+    y = torch.full((H * W, Cout), float("nan"), dtype=torch.float32, device="cuda")
+    ctx.neck_conv(mi.from_torch(wd, mi.F32, [k, k, Cin, Cout]), bd.data_ptr(), xd.data_ptr(), H, W, y.data_ptr())
+    ctx.synchronize()
+    pad = np.zeros((H + k - 1, W + k - 1, Cin))
+    pad[k // 2:k // 2 + H, k // 2:k // 2 + W] = x
+    ref = np.zeros((H * W, Cout))
+    for i in range(k):
+        for j in range(k):
+            ref += pad[i:i + H, j:j + W].reshape(H * W, Cin) @ w[:, :, i, j].astype(np.float64).T
+    err = np.sqrt(np.mean((y.cpu().numpy() - ref) ** 2) / np.mean(ref ** 2))
+    assert err <= K ** 0.5 * 2.0 ** -24, err
