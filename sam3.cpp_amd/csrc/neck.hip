@@ -290,7 +290,9 @@ __global__ __launch_bounds__(256, 2) void conv_f16_dma_kernel(const uint16_t* __
     if (tls >= TT) return;
     const int split = tls / tiles, tl = tls - split * tiles;
     const int m0 = (tl / tiles_n) * CT, n0 = (tl % tiles_n) * CT;
-    const int sl0 = split * sps, sl1 = min(nsl, sl0 + sps), nst = (sl1 - sl0 + 1) / 2;  // this split's slices, stages
+    // this split's slices and stages (PAIR: stages begin at even slices, so a range of odd bounds has
+    // a first or last stage of one slice)
+    const int sl0 = split * sps, sl1 = min(nsl, sl0 + sps), nst = PAIR ? (sl1 + 1) / 2 - sl0 / 2 : (sl1 - sl0 + 1) / 2;
 
     // DMA instruction j moves rows 8 (4 wv + j) + lane / 8: LDS slot lane % 8, global chunk
     // slot ^ hswz(row), slice chunk / 4. Per lane the byte offset of its chunk within the slice at
@@ -314,7 +316,7 @@ __global__ __launch_bounds__(256, 2) void conv_f16_dma_kernel(const uint16_t* __
     const uint32_t lb[2] = {(uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[0])),
                             (uint32_t)__builtin_amdgcn_readfirstlane(lds_addr(&sb[1]))};
     // the next stage to load, in order: its first slice, that slice's tap and channel slice
-    int dsl = sl0, dtap = TAPS == 9 ? dsl / cps : 0, dcs = dsl - dtap * cps;
+    int dsl = PAIR ? sl0 & ~1 : sl0, dtap = TAPS == 9 ? dsl / cps : 0, dcs = dsl - dtap * cps;
     int voff[4];  // PAIR: the lanes' map offsets of tap dtap
     auto at_tap = [&]() __attribute__((always_inline)) {
         const int off = TAPS == 9 ? ((dtap / 3 - 1) * W + dtap % 3 - 1) * C * 2 : 0;
@@ -327,6 +329,11 @@ __global__ __launch_bounds__(256, 2) void conv_f16_dma_kernel(const uint16_t* __
     if (PAIR) at_tap();
     auto dma = [&](uint32_t base) __attribute__((always_inline)) {
         if (PAIR) {
+            if (dsl + 1 >= sl1) {  // the range ends within the stage: its second slice reads zero
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (half[j]) voff[j] = woff[j] = CONV_OOB;
+            }
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 dma_b128_so(xr, base + (uint32_t)offsetof(ConvStage, A) + 1024u * (4 * wv + j), voff[j], dcs * 64);
@@ -394,7 +401,20 @@ __global__ __launch_bounds__(256, 2) void conv_f16_dma_kernel(const uint16_t* __
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    dma(lb[0]);
+    if (PAIR && (sl0 & 1)) {  // the range begins within its first stage, whose first slice reads zero
+        int w0[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            w0[j] = woff[j];
+            if (!half[j]) voff[j] = woff[j] = CONV_OOB;
+        }
+        dma(lb[0]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) woff[j] = w0[j];
+        at_tap();
+    } else {
+        dma(lb[0]);
+    }
     if (nst > 1) {
         dma(lb[1]);
         wait_vmcnt<NL>();
@@ -676,8 +696,7 @@ bool conv_f16_dma_fits(int taps, int64_t M, int64_t C, int64_t N) {
 }
 namespace {
 // K split of the DMA kernel (taps 1 and 9), in 32-deep slices: grids below one tile per CU; a
-// slice of a tile counts 0.9 us. Ranges of an odd number of slices get one more where C % 64 == 0,
-// so that every stage's two slices lie in one tap.
+// slice of a tile counts 0.9 us.
 int conv_f16_ksplit(int taps, int64_t M, int64_t C, int64_t N, int64_t* sps) {
     const int64_t nsl = (taps == 9 ? 9 : 1) * C / 32;
     *sps = nsl;
@@ -685,8 +704,7 @@ int conv_f16_ksplit(int taps, int64_t M, int64_t C, int64_t N, int64_t* sps) {
     const int64_t tiles = ((M + CT - 1) / CT) * ((N + CT - 1) / CT);
     const int S = gemm_ksplit(tiles, 256, M, N, nsl, 0.9);
     *sps = (nsl + S - 1) / S;
-    if (S > 1 && C % 64 == 0) *sps += *sps & 1;
-    return (int)((nsl + *sps - 1) / *sps);
+    return S;
 }
 }  // namespace
 

@@ -55,3 +55,20 @@ def test_deconv_f16_tiles(mi, ctx, H, W, Cin, Cout):
     a, t = x.astype(np.float16).astype(np.float64), w.astype(np.float16).astype(np.float64).reshape(Cin, -1)
     place = lambda v: v.reshape(H, W, Cout, 2, 2).transpose(0, 3, 1, 4, 2).reshape(4 * H * W, Cout)
     _close(y.cpu().numpy(), place(a @ t), place(np.abs(a) @ np.abs(t)), b, Cin)
+
+
+def test_conv_f16_ranges_of_odd_length(mi, ctx):
+    """A K split keeps its ranges where they are odd: 36 x 36 of 256 channels sums 72 slices of 32 in
+    ranges of seven, and longer ones would round more. 2^24 in slice 6, 1 in slice 7 and -2^24 in
+    slice 8 come out as 1 exactly, since a new range begins with slice 7 (with it in the first
+    range 2^24 + 1 rounds to 2^24)."""
+    H, C, N = 36, 256, 256
+    w = np.zeros((N, C, 3, 3), np.float16)
+    w[:, 200, 0, 0], w[:, 230, 0, 0], w[:, 5, 0, 1] = 4096, 1, -4096
+    x = np.zeros((H, H, C), np.float32)
+    x[..., 200], x[..., 230], x[..., 5] = 4096, 1, 4096
+    wd, bd, xd = torch.from_numpy(w.view(np.int16)).cuda(), torch.zeros(N, device="cuda"), torch.from_numpy(x).cuda()
+    y = torch.full((H, H, N), float("nan"), dtype=torch.float32, device="cuda")
+    ctx.neck_conv(mi.from_torch(wd, mi.F16, [3, 3, C, N]), bd.data_ptr(), xd.data_ptr(), H, H, y.data_ptr())
+    ctx.synchronize()
+    assert bool((y[1:, 1:] == 1).all()), y[1:, 1:].unique()
