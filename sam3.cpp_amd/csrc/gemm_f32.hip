@@ -457,9 +457,8 @@ void gemm_f32_dma_kernel(const GemmF32Args p, int ksplit, int sps) {
 // Infinities and NaN: a split infinity leaves NaN in m, and an infinite weight times a zero
 // plane is NaN too, so any output that is not finite is summed again in fp32 from the unsplit
 // operands, a wavefront's sixteen rows at a time on fp32 MFMAs, until those outputs are done or NaN.
-// 3x3 convolution
-// of 256 channels, 288 x 288 / 72 x 72: finite 566 / 56 us, one infinite pixel 724 / 155, a map of
-// NaN 659 / 118.
+// 3x3 convolution of 256 channels, 288 x 288 / 72 x 72: finite 566 / 56 us, one infinite pixel
+// 724 / 155, a map of NaN 659 / 118.
 namespace {
 typedef __bf16 v8b __attribute__((ext_vector_type(8)));
 struct SplitStage {
@@ -487,9 +486,9 @@ __device__ __forceinline__ void split8(const v4f (&x)[2], v8b& h, v8b& m, v8b& l
 }  // namespace
 
 // the planes alone (split_w_item); one thread per item
-__global__ __launch_bounds__(256) void split_w_kernel(const char* __restrict__ w, int64_t nb1, int f16, int taps, int N, int K,
-                                                      int KP, uint16_t* __restrict__ out) {
-    split_w_item((int64_t)blockIdx.x * blockDim.x + threadIdx.x, w, nb1, f16, taps, N, K, KP, out);
+__global__ __launch_bounds__(256) void split_w_kernel(const float* __restrict__ w, int taps, int N, int K, int KP,
+                                                      uint16_t* __restrict__ out) {
+    split_w_item((int64_t)blockIdx.x * blockDim.x + threadIdx.x, w, taps, N, K, KP, out);
 }
 
 template <bool CONV>
@@ -722,13 +721,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const GemmF32Arg
     }
 
     // outputs leave as float4 where the rows allow it: this split's partial sums without bias
-    // (part [split][M][N]), or D with the bias and the addend (all loaded before the first store:
-    // D may alias it)
+    // (part [split][M][N]), or D with the bias
     const bool parts = ksplit > 1;
     char* D = reinterpret_cast<char*>(parts ? p.part + (int64_t)split * M * N : p.D);
     const int64_t pitch = parts ? 4LL * N : p.d_nb1;
-    const float* add = parts ? nullptr : p.add;
-    const bool v4 = N % 4 == 0 && ((reinterpret_cast<uintptr_t>(D) | (uintptr_t)pitch | reinterpret_cast<uintptr_t>(add)) & 15) == 0;
+    const bool v4 = N % 4 == 0 && ((reinterpret_cast<uintptr_t>(D) | (uintptr_t)pitch) & 15) == 0;
     if (!v4) {
         // rows that are no multiple of four, or unaligned: through the wavefront's 16 KB of the stage
         // buffers (rows of 128 columns as two of 64), 64 columns of a row per store
@@ -746,33 +743,17 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const GemmF32Arg
             const int n = n0 + 64 * h + lane;
             const float bn = !parts && p.bias && n < N ? p.bias[n] : 0.0f;
             for (int r0 = 0; r0 < 32; r0 += 8) {
-                float v[8], a[8];
+                float v[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) v[k] = t[row64_chunk(2 * (r0 + k) + h, lane >> 2) + (lane & 3)];
 #pragma unroll
                 for (int k = 0; k < 8; ++k) {
                     const int m = m0 + 32 * wv + r0 + k;
-                    v[k] = t[row64_chunk(2 * (r0 + k) + h, lane >> 2) + (lane & 3)];
-                    a[k] = add && m < M && n < N ? add[(int64_t)m * N + n] : 0.0f;
-                }
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    const int m = m0 + 32 * wv + r0 + k;
-                    float o = parts ? v[k] : v[k] + bn;
-                    if (add) o = o + a[k];
-                    if (m < M && n < N) *(reinterpret_cast<float*>(D + (int64_t)m * pitch) + n) = o;
+                    if (m < M && n < N) *(reinterpret_cast<float*>(D + (int64_t)m * pitch) + n) = parts ? v[k] : v[k] + bn;
                 }
             }
         }
         return;
-    }
-    v4f ad[2][8];
-    if (add) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int m = m0 + 32 * wv + 16 * i + r16, n = n0 + 16 * j + 4 * kg;
-                ad[i][j] = m < M && n < N ? *reinterpret_cast<const v4f*>(add + (int64_t)m * N + n) : v4f{0, 0, 0, 0};
-            }
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -790,7 +771,6 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const GemmF32Arg
 #pragma unroll
                 for (int r = 0; r < 4; ++r) v[r] = v[r] + bn[r];
             }
-            if (add) v = v + ad[i][j];
             *reinterpret_cast<v4f*>(reinterpret_cast<float*>(D + (int64_t)m * pitch) + n) = v;
         }
     }
@@ -858,11 +838,11 @@ bool gemm_f32_split_ok(const GemmF32Args& a, int Z) {
     return a.K % 4 == 0 && (a.x_nb1 & 15) == 0 && (int64_t)(a.M - 1) * a.x_nb1 + 4LL * a.K < F32_OOB - 4096;
 }
 
-hipError_t launch_split_w(const void* w, int64_t nb1, bool f16, int taps, int N, int K, uint16_t* out, hipStream_t st) {
+hipError_t launch_split_w(const float* w, int taps, int N, int K, uint16_t* out, hipStream_t st) {
     const int KP = (K + 31) / 32 * 32;
     const int64_t n = (int64_t)N * (KP / 8);
     if (n > 0)
-        split_w_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(static_cast<const char*>(w), nb1, f16 ? 1 : 0, taps, N, K, KP, out);
+        split_w_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(w, taps, N, K, KP, out);
     return hipGetLastError();
 }
 
@@ -888,7 +868,7 @@ hipError_t launch_gemm_f32(const GemmF32Args& a, int Z, hipStream_t st) {
         return launch_split_reduce(a.part, S, a.M, a.N, a.bias, a.D, a.d_nb1, st);
     };
     if (a.wsplit) {
-        if (!gemm_f32_split_ok(a, Z) || (reinterpret_cast<uintptr_t>(a.wsplit) & 15)) return hipErrorInvalidValue;
+        if (!gemm_f32_split_ok(a, Z) || a.add || (reinterpret_cast<uintptr_t>(a.wsplit) & 15)) return hipErrorInvalidValue;
         const unsigned nb = (unsigned)((tiles * S + 7) / 8 * 8);
         if (a.conv) gemm_f32_split_kernel<true><<<nb, 256, 0, st>>>(a, S, sps);
         else gemm_f32_split_kernel<false><<<nb, 256, 0, st>>>(a, S, sps);

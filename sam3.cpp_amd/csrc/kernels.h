@@ -245,10 +245,9 @@ struct GemmF32Args {
     // kernel in file order, read where an output is not finite
     const uint16_t* wsplit = nullptr;
 };
-// The planes of weight rows [N][K] (row pitch nb1 bytes, F32 or F16; taps = 9: a 3x3 kernel
-// [N][K / 9][3][3], its rows in (tap, channel) order) for GemmF32Args::wsplit:
-// gemm_f32_split_bytes(N, K) bytes at out, 16-byte aligned
-hipError_t launch_split_w(const void* w, int64_t nb1, bool f16, int taps, int N, int K, uint16_t* out, hipStream_t st);
+// The planes of an F32 kernel's rows [N][K] (taps = 9: a 3x3 one [N][K / 9][3][3], its rows in
+// (tap, channel) order) for GemmF32Args::wsplit: gemm_f32_split_bytes(N, K) bytes at out, 16-byte aligned
+hipError_t launch_split_w(const float* w, int taps, int N, int K, uint16_t* out, hipStream_t st);
 size_t gemm_f32_split_bytes(int64_t N, int64_t K);
 // whether the shapes and alignments of a (Z batches) fit the bf16-MFMA kernel
 bool gemm_f32_split_ok(const GemmF32Args& a, int Z);

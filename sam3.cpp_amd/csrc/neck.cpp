@@ -184,8 +184,8 @@ mi355_status conv(mi355_context* ctx, const mi355_tensor* w, const float* b, con
             g.wsplit = reinterpret_cast<const uint16_t*>(pre ? pre : scratch);
             if (!pre) {
                 Timed t(ctx, "neck_conv_split_w");
-                st = hip_check(ctx, t.done(launch_split_w(w->data, 4 * K, false, k * k, Cout, (int)K,
-                                                          reinterpret_cast<uint16_t*>(scratch), ctx->stream)),
+                st = hip_check(ctx, t.done(launch_split_w(g.W, k * k, Cout, (int)K, reinterpret_cast<uint16_t*>(scratch),
+                                                          ctx->stream)),
                                "conv kernel split");
             }
         } else if (k == 3) {

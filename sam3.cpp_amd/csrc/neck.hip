@@ -49,7 +49,7 @@ __global__ __launch_bounds__(256) void neck_pack_kernel(const NeckPacks p) {
         conv3x3_pack_f16_item(it, static_cast<const uint16_t*>(j.w), j.Cin, j.Cout, j.out);
     } else {
         const int taps = j.k * j.k, K = taps * j.Cin;
-        split_w_item(it, static_cast<const char*>(j.w), 4LL * K, 0, taps, j.Cout, K, (K + 31) / 32 * 32, j.out);
+        split_w_item(it, static_cast<const float*>(j.w), taps, j.Cout, K, (K + 31) / 32 * 32, j.out);
     }
 }
 
@@ -747,13 +747,12 @@ hipError_t launch_conv_f16(int taps, const void* x, bool x16, const uint16_t* w,
         else if (taps == 4 && y16) go(conv_f16_dma_kernel<4, true, true>, conv_f16_dma_kernel<4, true, false>);
         else if (taps == 4) go(conv_f16_dma_kernel<4, false, true>, conv_f16_dma_kernel<4, false, false>);
         else if (taps == 1 && y16) go(conv_f16_dma_kernel<1, true, true>, conv_f16_dma_kernel<1, true, false>);
-        else if (taps == 1) go(conv_f16_dma_kernel<1, false, true>, conv_f16_dma_kernel<1, false, false>);
         else return hipErrorInvalidValue;
         const hipError_t e = hipGetLastError();
         if (S == 1 || e != hipSuccess) return e;
         return launch_split_reduce(part, S, (int)M, N, bias, static_cast<float*>(y), (y16 ? 2LL : 4LL) * N, st, y16);
     }
-    // K step 32: a 64-deep step (64 KB of LDS, two workgroups per CU) measured slower
+    // K step 32: 64-deep steps, staged through registers here, measured slower
     if (y16) return hipErrorInvalidValue;  // fp16 maps: the DMA kernel only
     const float* xf = static_cast<const float*>(x);
     float* yf = static_cast<float*>(y);

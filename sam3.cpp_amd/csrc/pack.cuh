@@ -16,11 +16,11 @@ __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
 // split: the lowest plane of the smallest fp32 values is then a normal bf16.
 constexpr float SPLIT_UP = 16777216.0f;
 
-// item i of the planes of SPLIT_UP times weight rows [N][K] (row pitch nb1 bytes; F32 or F16; or,
-// taps == 9, a 3x3 kernel [N][C][3][3] read in (tap, channel) order) -> [N][KP / 32][3][32] bf16, zero
-// past K: eight consecutive K
-__device__ __forceinline__ void split_w_item(int64_t i, const char* __restrict__ w, int64_t nb1, int f16, int taps, int N, int K,
-                                             int KP, uint16_t* __restrict__ out) {
+// item i of the planes of SPLIT_UP times the rows of an F32 kernel [N][K] (taps == 9: a 3x3 one
+// [N][C][3][3] read in (tap, channel) order) -> [N][KP / 32][3][32] bf16, zero past K: eight
+// consecutive K
+__device__ __forceinline__ void split_w_item(int64_t i, const float* __restrict__ w, int taps, int N, int K, int KP,
+                                             uint16_t* __restrict__ out) {
     const int k8 = KP / 8;
     if (i >= (int64_t)N * k8) return;
     const int n = (int)(i / k8), k0 = (int)(i - (int64_t)n * k8) * 8;
@@ -32,8 +32,7 @@ __device__ __forceinline__ void split_w_item(int64_t i, const char* __restrict__
         float x = 0.0f;
         if (k < K) {
             const int64_t e = taps == 1 ? k : (int64_t)(k % C) * taps + k / C;
-            const char* row = w + (int64_t)n * nb1;
-            x = f16 ? h2f(reinterpret_cast<const uint16_t*>(row)[e]) : reinterpret_cast<const float*>(row)[e];
+            x = w[(int64_t)n * K + e];
         }
         x *= SPLIT_UP;
         const uint32_t a = pk_bf16(x, 0.0f) & 0xffffu;
