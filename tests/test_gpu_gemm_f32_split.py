@@ -158,3 +158,86 @@ def test_neck_conv_f32_error_at_every_magnitude(mi, ctx, k, Cin, Cout, xs, ws):
             ref += pad[i:i + H, j:j + W].reshape(H * W, Cin) @ w[:, :, i, j].astype(np.float64).T
     err = np.sqrt(np.mean((y.cpu().numpy() - ref) ** 2) / np.mean(ref ** 2))
     assert err <= K ** 0.5 * 2.0 ** -24, err
+
+
+def _whole(rng, shape, bits):
+    """Odd whole numbers of up to `bits` bits, either sign."""
+    return ((rng.integers(0, 2 ** (bits - 1), shape) * 2 + 1) * rng.choice([-1, 1], shape)).astype(np.float32)
+
+
+def _exact_case(rng, planes, H, W, Cin, Cout, k):
+    """A map [H, W, Cin] and a kernel [Cout, Cin, k, k] of which every output is one product, exact in
+    fp32: whole numbers of 24 bits (all three planes) on one side and +-1 on the other, or of 12 bits
+    (two planes each, of which the product of the lower ones counts) on both."""
+    x, w = np.zeros((H, W, Cin), np.float32), np.zeros((Cout, Cin, k, k), np.float32)
+    bits = {"kernel": (1, 24), "map": (24, 1), "both": (12, 12)}[planes]
+    if planes == "map":  # one tap of one channel per output
+        x = _whole(rng, x.shape, bits[0])
+        w[np.arange(Cout), rng.integers(0, Cin, Cout), rng.integers(0, k, Cout), rng.integers(0, k, Cout)] = _whole(rng, Cout, 1)
+    else:                # one channel of pixels three apart
+        at = np.ix_(range(0, H, 3), range(0, W, 3))
+        c = rng.integers(0, Cin, x[at].shape[:2])
+        x[at[0], at[1], c] = _whole(rng, c.shape, bits[0])
+        w = _whole(rng, w.shape, bits[1])
+    return x, w
+
+
+def _conv64(x, w):
+    H, W, Cin = x.shape
+    Cout, k = w.shape[0], w.shape[2]
+    pad = np.zeros((H + k - 1, W + k - 1, Cin))
+    pad[k // 2:k // 2 + H, k // 2:k // 2 + W] = x
+    return sum(pad[i:i + H, j:j + W].reshape(H * W, Cin) @ w[:, :, i, j].astype(np.float64).T for i in range(k) for j in range(k))
+
+
+@pytest.mark.parametrize("H,W,Cin,Cout,k", [(1, 1, 128, 4, 1), (16, 8, 128, 128, 1), (43, 3, 132, 124, 1), (127, 1, 160, 132, 1),
+                                            (11, 3, 588, 16, 1), (20, 15, 1020, 260, 1), (5, 1, 2304, 260, 1), (9, 13, 36, 20, 1),
+                                            (17, 11, 64, 36, 3), (16, 8, 32, 128, 3), (43, 3, 96, 124, 3), (23, 20, 256, 256, 3)])
+@pytest.mark.parametrize("planes", ["kernel", "map", "both"])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_neck_conv_f32_exact_integers(mi, ctx, H, W, Cin, Cout, k, planes, offset):
+    """Equality where an error bound cannot tell a missing plane or product; also with rows that
+    float4 stores cannot reach (offset: floats by which the output misses 16 bytes)."""
+    x, w = _exact_case(np.random.default_rng(H * W + Cin + k), planes, H, W, Cin, Cout, k)
+    wd, bd, xd = torch.from_numpy(w).cuda(), torch.zeros(Cout, device="cuda"), torch.from_numpy(x).cuda()
+    y = torch.full((H * W * Cout + 2,), float("nan"), dtype=torch.float32, device="cuda")
+    ctx.neck_conv(mi.from_torch(wd, mi.F32, [k, k, Cin, Cout]), bd.data_ptr(), xd.data_ptr(), H, W, y.data_ptr() + 4 * offset)
+    ctx.synchronize()
+    got = y.cpu().numpy()
+    assert np.isnan(got[:offset]).all() and np.isnan(got[offset + H * W * Cout:]).all()
+    assert np.array_equal(got[offset:offset + H * W * Cout].reshape(H * W, Cout), _conv64(x, w))
+
+
+@pytest.mark.parametrize("planes", ["kernel", "map", "both"])
+@pytest.mark.parametrize("at", ["conv1x1", "conv3x3"])
+def test_sam3_neck_f32_exact_integers(mi, ctx, planes, at):
+    """The same through the fused neck's scale 2 (1x1, then 3x3), whose kernels one launch repacks;
+    the other convolution passes its map on."""
+    E, G, C1, D = 160, 12, 64, 96
+    rng = np.random.default_rng(5)
+    one, three = np.zeros((D, E, 1, 1), np.float32), np.zeros((D, D, 3, 3), np.float32)
+    one[np.arange(D), np.arange(D), 0, 0] = three[np.arange(D), np.arange(D), 1, 1] = 1
+    x = np.zeros((G, G, E), np.float32)
+    if at == "conv1x1":
+        x, one = _exact_case(rng, planes, G, G, E, D, 1)
+    else:
+        x[..., :D], three = _exact_case(rng, planes, G, G, D, D, 3)
+    ref = _conv64(_conv64(x, one).reshape(G, G, D), three)
+    keep, scales = [], []
+    for shapes in ([("deconv1", E, C1), ("deconv2", C1, D), ("conv1x1", D, D), ("conv3x3", D, D)],
+                   [("deconv1", E, C1), ("conv1x1", D, C1), ("conv3x3", D, D)], [("conv1x1", D, E), ("conv3x3", D, D)],
+                   [("conv1x1", D, E), ("conv3x3", D, D)]):
+        s = {}
+        for n, a, b in shapes:
+            k = {"deconv1": 2, "deconv2": 2, "conv1x1": 1, "conv3x3": 3}[n]
+            w = torch.zeros((a, b, k, k)) if len(scales) != 2 else torch.from_numpy(one if n == "conv1x1" else three)
+            bias = torch.zeros(b if k == 2 else a, device="cuda")
+            keep += [w.cuda(), bias]
+            s[n + "_w"] = mi.from_torch(keep[-2], mi.F32, [k, k, b, a])
+            s[n + "_b"] = bias.data_ptr()
+        scales.append(s)
+    out = [torch.full((h * h, D), float("nan"), dtype=torch.float32, device="cuda") for h in (4 * G, 2 * G, G, G // 2)]
+    xd = torch.from_numpy(x).cuda()
+    ctx.sam3_neck(xd.data_ptr(), E, G, scales, [o.data_ptr() for o in out])
+    ctx.synchronize()
+    assert np.array_equal(out[2].cpu().numpy(), ref)
