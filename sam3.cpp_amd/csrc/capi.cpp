@@ -188,20 +188,30 @@ MmPlan mm_plan(const mi355_tensor* s0, const mi355_tensor* s1, int cus, bool spl
 }
 
 // The route of a MUL_MAT with ggml-layout quantized weights under MI355_MMQ_AUTO: int8 with the
-// repack in the call (1297 x 771 x 736 Q4_1 25.9 us on the fp16 route, 17.7 on this one;
-// 5184 x 3072 x 1024 76 and 70; 2000 x 1024 x 1024 30.3 and 21.1), except
-// - few rows over a large weight, where the repack costs more than the kernel saves (1 x 4736 x 1024
-//   13.5 and 18.3; 64 x 1024 x 1024 14.2 and 15.8; 26 x 668 x 480 13.3 and 14.1); shorter K takes the
-//   few-row kernel, and with N % 4 != 0 the fp16 route cannot split K;
-// - Q4_1 where the fp16 route's skinny kernel serves it (4445 x 36 x 96 9.3 and 12.3), and grids of
-//   200 tiles or more with N % 4 != 0 (1255 x 4258 x 4704 151 and 176).
+// repack in the call, the fp16 route where that measured faster (1185 shapes drawn up to 5184 x 4736 x
+// 1024 of work, us fp16 / int8; repeated calls, a context's first ones differ by the same):
+// - at most 64 rows that the few-row kernel does not take (K > 512) or over a large weight, where the
+//   repack costs more than the kernel saves: Q8_0 1 x 4736 x 1024 13.5 / 17.8, 64 x 1024 x 512
+//   12.7 / 13.1. Weight rows of Q8_0 and Q4_0 need K % 64 == 0, or the fp16 route copies them to an
+//   aligned pitch (9 x 2540 x 480 17.0 / 12.1), and N % 4 == 0, or it cannot split K;
+// - Q4_1 with K <= 128 (96 x 72 x 64 9.0 / 11.0, 4445 x 36 x 96 9.0 / 10.2, 5345 x 2716 x 128
+//   24.1 / 26.9; 772 x 1297 x 160 12.3 / 11.5), with up to 128 rows where the fp16 route splits K
+//   (65 x 3040 x 2176 20.7 / 22.7; 65 x 4736 x 1024, which it does not, 26.9 / 20.1), and on large
+//   grids with a long K (7789 x 1324 x 2304 134 / 154, 1297 x 2051 x 4704 112 / 120; 5747 x 1156 x 352
+//   25.8 / 25.3, 1800 x 771 x 4704 113 / 70, 8358 x 160 x 2400 75 / 64).
 int mm_route(const mi355_tensor* s0, const mi355_tensor* s1, int kernel) {
     if (kernel != MI355_MMQ_AUTO || s0->layout != MI355_LAYOUT_GGML || !mm_i8_eligible(s0, s1) || !f16_extents_ok(s0, s1))
         return kernel;
     const int64_t K = s0->ne[0], N = s0->ne[1], M = s1->ne[1];
-    const bool few = M <= 64 && K >= 480 && N % 4 == 0 && N * K >= ((int64_t)1 << 18);
-    const bool q41 = s0->type == T_Q4_1 && ((M >= 4096 && K <= 128) || (N % 4 != 0 && ((M + 127) / 128) * ((N + 127) / 128) >= 200));
-    return few || q41 ? MI355_MMQ_F16 : MI355_MMQ_INT8;
+    const bool q41 = s0->type == T_Q4_1;
+    bool f16 = false;
+    if (M <= 64)
+        f16 = N % 4 == 0 && (q41 ? K > 512 || (K >= 416 && N * K >= (int64_t)1 << 17)
+                                 : K >= 512 && K % 64 == 0 && N * K >= (int64_t)1 << 18);
+    else if (q41)
+        f16 = K <= 128 || (M <= 128 && N % 4 == 0 && K >= 768 && N < 4096) ||
+              (K > 1856 && ((M + 127) / 128) * ((N + 127) / 128) >= 128 && (N % 4 != 0 || N > 512));
+    return f16 ? MI355_MMQ_F16 : MI355_MMQ_INT8;
 }
 
 bool dst_split_ok(const mi355_tensor* d) {
