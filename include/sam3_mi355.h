@@ -180,9 +180,12 @@ mi355_status mi355_weight_prepare(mi355_context* ctx, const mi355_tensor* w, voi
  * MI355_NOALLOC_SCRATCH_BYTES per GPU, held from library load until the
  * process ends, instead of the context's workspace; the call allocates and
  * frees nothing and records no timing events.  Operands whose plan on the
- * context's current route (mi355_context_set_mmq_kernel) needs more scratch
- * than that are rejected with MI355_STATUS_UNSUPPORTED; the most any route
- * needs, mi355_mul_mat_workspace_size, bounds it from above.  Every call on
+ * context's current route (mi355_context_set_mmq_kernel; under MI355_MMQ_AUTO
+ * the int8 one, MI355_MMQ_F16 for ggml-layout Q4_1) needs more scratch than
+ * that are rejected with MI355_STATUS_UNSUPPORTED, also where AUTO prefers a
+ * route that needs less; where it prefers one that needs more than the array
+ * holds, the call takes the former.  F32 weights need no scratch.  The most
+ * any route needs, mi355_mul_mat_workspace_size, bounds it from above.  Every call on
  * one GPU uses that GPU's one array: calls through one context serialize on
  * its stream, and a call through another context first makes its stream
  * wait on an event the device's previous call recorded (each context creates
@@ -545,7 +548,8 @@ mi355_status mi355_context_set_skinny(mi355_context* ctx, int enable);
  *   int8 rows with separate scale arrays on each call, block sums on
  *   v_mfma_i32_32x32x32_i8;
  * - MI355_MMQ_AUTO (the default): the faster per call with the repack counted:
- *   MI355_MMQ_INT8, except for few activation rows over a large weight.
+ *   MI355_MMQ_INT8, except for few activation rows over a large weight, and
+ *   for Q4_1 with K <= 128, few rows and large grids with a long K.
  * Prepared weights always take the int8 kernel; other MUL_MATs keep their
  * own kernels. */
 typedef enum {

@@ -187,6 +187,13 @@ MmPlan mm_plan(const mi355_tensor* s0, const mi355_tensor* s1, int cus, bool spl
     return pl;
 }
 
+// The route that decides under MI355_MMQ_AUTO what a call needs: a weight's own one, whatever
+// mm_route prefers.
+int mm_own_route(const mi355_tensor* s0, int kernel) {
+    if (kernel != MI355_MMQ_AUTO) return kernel;
+    return s0->type == T_Q4_1 && s0->layout == MI355_LAYOUT_GGML ? MI355_MMQ_F16 : MI355_MMQ_INT8;
+}
+
 // The route of a MUL_MAT with ggml-layout quantized weights under MI355_MMQ_AUTO: int8 with the
 // repack in the call, the fp16 route where that measured faster (1185 shapes drawn up to 5184 x 4736 x
 // 1024 of work, us fp16 / int8; repeated calls, a context's first ones differ by the same):
@@ -201,7 +208,7 @@ MmPlan mm_plan(const mi355_tensor* s0, const mi355_tensor* s1, int cus, bool spl
 //   25.8 / 25.3, 1800 x 771 x 4704 113 / 70, 8358 x 160 x 2400 75 / 64).
 int mm_route(const mi355_tensor* s0, const mi355_tensor* s1, int kernel) {
     if (kernel != MI355_MMQ_AUTO || s0->layout != MI355_LAYOUT_GGML || !mm_i8_eligible(s0, s1) || !f16_extents_ok(s0, s1))
-        return kernel;
+        return mm_own_route(s0, kernel);
     const int64_t K = s0->ne[0], N = s0->ne[1], M = s1->ne[1];
     const bool q41 = s0->type == T_Q4_1;
     bool f16 = false;
@@ -218,15 +225,15 @@ bool dst_split_ok(const mi355_tensor* d) {
     return d->nb[1] % 16 == 0 && (reinterpret_cast<uintptr_t>(d->data) & 15) == 0;
 }
 
-// The plan of mm_route's route or, where that needs more than limit bytes of scratch, of the other
-// route if it fits (AUTO only; both give the same bits).
+// The plan for at most limit bytes of scratch: mm_route's if it fits, else the own route's; beyond
+// the limit where the own route's is (the call is then refused). All routes give the same bits.
 MmPlan mm_plan_in(const mi355_context* ctx, const mi355_tensor* s0, const mi355_tensor* s1, const mi355_tensor* d, size_t limit) {
     const bool split = dst_split_ok(d);
-    const MmPlan pl = mm_plan(s0, s1, ctx->cus, split, mm_route(s0, s1, ctx->mmq_kernel));
-    if (pl.total() <= limit || ctx->mmq_kernel != MI355_MMQ_AUTO || s0->type == T_F16 || pl.prep || !f16_extents_ok(s0, s1))
-        return pl;
-    const MmPlan other = mm_plan(s0, s1, ctx->cus, split, pl.i8 ? MI355_MMQ_F16 : MI355_MMQ_INT8);
-    return other.total() <= limit ? other : pl;
+    const int own = mm_own_route(s0, ctx->mmq_kernel), route = mm_route(s0, s1, ctx->mmq_kernel);
+    const MmPlan pl = mm_plan(s0, s1, ctx->cus, split, own);
+    if (route == own || pl.total() > limit) return pl;
+    const MmPlan fast = mm_plan(s0, s1, ctx->cus, split, route);
+    return fast.total() <= limit ? fast : pl;
 }
 
 // ggml_soft_max_ext(a, mask, scale, max_bias) shape rules plus what softmax.hip implements.
@@ -790,9 +797,18 @@ mi355_status mi355_mul_mat(mi355_context* ctx, const mi355_tensor* s0, const mi3
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
             pl = mm_plan_in(ctx, s0, s1, d, ctx->ws_size);  // nothing can be allocated now
+        const std::string before = ctx->last_error;
+        st = ensure_ws(ctx, pl.total());
+        if (st != MI355_STATUS_SUCCESS) {  // no memory for the repack: the own route may need less
+            const MmPlan own = mm_plan(s0, s1, ctx->cus, dst_split_ok(d), mm_own_route(s0, ctx->mmq_kernel));
+            if (own.total() >= pl.total()) return st;
+            (void)hipGetLastError();
+            ctx->last_error = before;
+            pl = own;
+            st = ensure_ws(ctx, pl.total());
+            if (st != MI355_STATUS_SUCCESS) return st;
+        }
     }
-    st = ensure_ws(ctx, pl.total());
-    if (st != MI355_STATUS_SUCCESS) return st;
     return mul_mat_run(ctx, s0, s1, d, pl, static_cast<char*>(ctx->ws), true);
 }
 
@@ -835,7 +851,7 @@ mi355_status mi355_mul_mat_block_dots(mi355_context* ctx, const mi355_tensor* s0
     if (st != MI355_STATUS_SUCCESS) return st;
     if (!ctx) return fail(nullptr, MI355_STATUS_INVALID_ARG, "block_dots: null context");
     (void)hipSetDevice(ctx->device);
-    const MmPlan pl = mm_plan(s0, s1, ctx->cus, false, ctx->mmq_kernel);
+    const MmPlan pl = mm_plan(s0, s1, ctx->cus, false, mm_own_route(s0, ctx->mmq_kernel));
     st = ensure_ws(ctx, pl.total());
     if (st != MI355_STATUS_SUCCESS) return st;
     if (pl.i8) {

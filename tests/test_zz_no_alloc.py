@@ -99,3 +99,63 @@ def test_mul_mat_noalloc_ordered_across_streams(mi, orc):
     finally:
         ca.close()
         cb.close()
+
+
+def test_mul_mat_noalloc_limit_is_the_types_own_route(mi, ctx, orc):
+    """Under the default route a call is refused where Q8_0's int8 plan (its repacked weight) does not
+    fit the scratch, also with few rows, for which the fp16 route is preferred and would fit; and a
+    Q4_1 call whose preferred int8 plan does not fit takes its own fp16 route."""
+    N, K = 8192, 8448  # 69 million one-byte quants > 64 MiB
+    for tname, M, refused in (("q8_0", 1, True), ("q4_1", 100, False)):
+        t = orc.NAME_TYPE[tname]
+        row = orc.quantize_weights(t, orc.normal(64 * K, 330, 1, std=0.02).reshape(64, K)).view(np.uint8).reshape(64, -1)
+        wd = dev(row).repeat(N // 64, 1)
+        xd = dev(orc.normal(M * K, 331, 2).reshape(M, K))
+        ref, got = (torch.zeros((M, N), dtype=torch.float32, device="cuda") for _ in range(2))
+        s0, s1 = mi.from_torch(wd, t, [K, N]), mi.from_torch(xd, mi.F32, [K, M])
+        ctx.mul_mat(s0, s1, mi.from_torch(ref, mi.F32, [N, M]))
+        if refused:
+            with pytest.raises(mi.Mi355Error) as ei:
+                ctx.mul_mat_noalloc(s0, s1, mi.from_torch(got, mi.F32, [N, M]))
+            assert ei.value.status == -3 and "scratch" in str(ei.value)
+            ctx.synchronize()
+            assert bool(ref.any()) and not got.any()
+        else:
+            ctx.mul_mat_noalloc(s0, s1, mi.from_torch(got, mi.F32, [N, M]))
+            ctx.synchronize()
+            assert bool(ref.any()) and torch.equal(got, ref)
+
+
+def test_captured_call_takes_the_route_its_workspace_holds(mi, orc):
+    """A workspace of the fp16 route's size under capture, where none can be allocated: the default
+    route, int8 here, needs more, so the captured call is the fp16 route's. Same bits on every replay,
+    with eager work between them."""
+    t, M, N, K = orc.Q4_1, 300, 772, 736
+    stream = torch.cuda.Stream()
+    c, other = mi.Context(0, stream.cuda_stream), mi.Context(0)
+    try:
+        with torch.cuda.stream(stream):
+            wd = dev(_weights(orc, t, N, K, 340).view(np.uint8))
+            xd, out, ref = dev(orc.normal(M * K, 341, 2).reshape(M, K)), torch.empty((M, N), device="cuda"), torch.empty((M, N), device="cuda")
+            args = mi.from_torch(wd, t, [K, N]), mi.from_torch(xd, mi.F32, [K, M]), mi.from_torch(out, mi.F32, [N, M])
+            c.set_mmq_kernel(mi.MMQ_F16)
+            c.mul_mat(*args)
+            c.set_mmq_kernel(mi.MMQ_AUTO)
+            c.synchronize()
+            other.mul_mat(args[0], args[1], mi.from_torch(ref, mi.F32, [N, M]))
+            other.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=stream):
+                c.mul_mat(*args)
+            for step in range(3):
+                out.fill_(float("nan"))
+                graph.replay()
+                c.synchronize()
+                assert torch.equal(out, ref), step
+                xd.mul_(0.5)
+                torch.cuda.synchronize()
+                other.mul_mat(args[0], args[1], mi.from_torch(ref, mi.F32, [N, M]))
+                other.synchronize()
+    finally:
+        c.close()
+        other.close()
