@@ -893,13 +893,17 @@ __global__ __launch_bounds__(256) void mmq_reduce_kernel(const float* __restrict
 // F16 weights. Plain stores with K < 640 take mmq_kernel (three stage buffers of 32-deep steps: the
 // first stage is multiplied sooner, and there are too few for mmq_f16_kernel's rate to pay: 38481 x
 // 638 x 128 31.9 us and 37.3 there, 24551 x 1000 x 256 36.7 and 38.6, 894 x 40 x 576 11.7 and 12.6,
-// 66 x 1363 x 608 14.9 and 15.4; 5 x 147 x 736 15.1 and 13.8). Both add the products in the same
-// order; fused epilogues are shorter on mmq_f16_kernel.
+// 66 x 1363 x 608 14.9 and 15.4; 5 x 147 x 736 15.1 and 13.8), and so do at most one workgroup per CU
+// over rows that begin within lines, unsplit since N % 4 != 0 (2657 x 137 x 2472 43.7 and 47.5, 1145 x
+// 1141 x 1352 27.7 and 29.8, on average of 75 such shapes 2.6% less; with K % 32 == 0 the lines are
+// whole: 1343 x 1307 x 3712 56.3 and 50.0; with few rows 3 x 383 x 4040 53.3 and 41.9). Both add the
+// products in the same order; fused epilogues are shorter on mmq_f16_kernel.
 static void launch_f16(const MmqArgs& a, int Z, const MmqEpi* e, hipStream_t st) {
     const int TT = a.tiles_m * a.tiles_n * a.ksplit;
     const dim3 grid((unsigned)(((TT + 7) / 8) * 8), (unsigned)Z);
     const bool store = a.ksplit > 1 || !e || e->kind == MMQ_EPI_STORE;
-    if (store && a.K < 640) mmq_kernel<T_F16, false, MMQ_EPI_STORE><<<grid, NT, 0, st>>>(a, MmqEpi{});
+    const bool ragged = a.N % 4 != 0 && a.K % 32 != 0 && a.M >= 256 && (int64_t)TT * Z <= 256;
+    if (store && (a.K < 640 || ragged)) mmq_kernel<T_F16, false, MMQ_EPI_STORE><<<grid, NT, 0, st>>>(a, MmqEpi{});
     else if (store) mmq_f16_kernel<MMQ_EPI_STORE><<<grid, NT, 0, st>>>(a, MmqEpi{});
     else if (e->kind == MMQ_EPI_RESIDUAL) mmq_f16_kernel<MMQ_EPI_RESIDUAL><<<grid, NT, 0, st>>>(a, *e);
     else mmq_f16_kernel<MMQ_EPI_QKV><<<grid, NT, 0, st>>>(a, *e);

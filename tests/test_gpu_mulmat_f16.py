@@ -30,3 +30,10 @@ def test_f16_depths_and_remainders(mi, ctx, orc, M, N, K, off):
     a, b = x.astype(np.float16).astype(np.float64), w.astype(np.float64)
     err = np.abs(got[off:off + M * N].reshape(M, N) - a @ b.T)
     assert (err <= K * 2.0 ** -23 * (np.abs(a) @ np.abs(b).T)).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(255, 129, 1000), (256, 129, 1000), (256, 129, 1024), (300, 259, 648), (16300, 257, 712),
+                                   (16500, 257, 712)])
+def test_f16_unsplit_rows_that_begin_within_lines(mi, ctx, orc, M, N, K):
+    """Both sides of the rule by which ragged shapes of one workgroup per CU take the other kernel."""
+    test_f16_depths_and_remainders(mi, ctx, orc, M, N, K, 0)
