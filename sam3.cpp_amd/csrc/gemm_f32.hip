@@ -443,7 +443,7 @@ void gemm_f32_dma_kernel(const GemmF32Args p, int ksplit, int sps) {
 // read by no other wavefront. Stages of 32 K (16 KB + 24 KB), two buffers, two workgroups per CU.
 //
 // Measured: the 288 x 288 3x3 convolution of 256 channels (97.8 GFLOP, 587 of them as bf16)
-// 904 -> 493 us (1.2 PFLOP/s of bf16; some 90 less without the stage DMA, 120 without the split too:
+// 904 -> 496 us (1.2 PFLOP/s of bf16; some 90 less without the stage DMA, 120 without the split too:
 // the MFMAs alone run at the chip's power limit; with 32 x 32 x 16 MFMAs 50 more), weight pass
 // included; error against 64 bits 5.0e-7 -> 4.2e-7 at 72 x 72 (K = 2304), 2.1e-7 -> 1.6e-7 of a 1x1 at
 // K = 1024.
@@ -643,7 +643,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const GemmF32Arg
         mul(a, b1, 3, 2, 6);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // VALU
+            __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);  // VALU
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
         }
         __builtin_amdgcn_sched_barrier(0);

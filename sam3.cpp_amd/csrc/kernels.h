@@ -178,12 +178,12 @@ int mmq8_tile_rows(int64_t M, int64_t N, int64_t K, int ks, int cus);
 // dst = W^T . A (2-D) on int8 MFMA, bit-identical to launch_mmq on the same
 // operands; epilogues and split-K as launch_mmq / launch_mmq_epi.
 // With dots != nullptr the kernel writes the exact int32 block sums [M][N][K/32] instead.
+hipError_t launch_mmq8(const WRep& w, const ActI8& a, const MatD& d, const MmqEpi* epi, const MmqSplit& sp,
+                       hipStream_t st, int32_t* dots = nullptr);
 // A MUL_MAT of few F32 activation rows (at most 64, K <= 512), quantized by the kernel itself:
 // the bits of launch_quantize_mmq_i8 + launch_mmq8 with ks K ranges
 bool mmq8_few_ok(const WRep& w, const SrcView& x);
 hipError_t launch_mmq8_few(const WRep& w, const SrcView& x, const MatD& d, int ks, hipStream_t st);
-hipError_t launch_mmq8(const WRep& w, const ActI8& a, const MatD& d, const MmqEpi* epi, const MmqSplit& sp,
-                       hipStream_t st, int32_t* dots = nullptr);
 // from_float (x86 variant) into the int8 operand layout: q [rows][s1] int8,
 // d -> dl [rows][dp / 2] followed by dh [rows][dp / 2] (uint32), s as ActF16's.
 hipError_t launch_quantize_mmq_i8(const SrcView& src, bool with_sum, int64_t s1, int64_t dp, int8_t* q, uint16_t* d,

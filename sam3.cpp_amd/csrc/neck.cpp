@@ -13,11 +13,11 @@
 //     epilogue, or (maps with Cin % 32 != 0 or unaligned rows) as a MUL_MAT
 //     and a scatter pass;
 //   - conv_2d_sk_p0 1x1: a GEMM with the kernel rows as they are, the bias in
-//     its epilogue (F32 kernels: the tiled fp32 GEMM; F16 kernels: the fp16
-//     implicit-GEMM kernel below with one tap);
+//     its epilogue (F32 kernels: the split GEMM over their three bf16 planes; F16
+//     kernels: the fp16 implicit-GEMM kernel below with one tap);
 //   - conv_2d_s1_ph 3x3: an implicit GEMM over the map (the kernel repacked to
-//     (tap, channel) rows, no im2col) on fp32 MFMA (F32 kernels) or fp16 MFMA
-//     (F16 kernels, the map rounded to fp16 as it is loaded); maps with
+//     (tap, channel) rows, no im2col) on bf16 MFMA (F32 kernels, split as for the
+//     1x1) or fp16 MFMA (F16 kernels, the map rounded to fp16 once); maps with
 //     Cin % 32 != 0 or rows not 16-byte aligned take im2col (K ordered as
 //     ggml's, ic-major) or the plain map + MUL_MAT + bias;
 //   - pool_2d MAX 2x2 / 2.
@@ -149,10 +149,10 @@ mi355_status conv(mi355_context* ctx, const mi355_tensor* w, const float* b, con
     const int Cin = (int)w->ne[2], Cout = (int)w->ne[3];
     const int64_t P = (int64_t)H * W, K = (int64_t)k * k * Cin;
     if (Cout % 4 != 0) return fail(ctx, MI355_STATUS_UNSUPPORTED, "neck_conv: Cout %% 4 != 0");
-    // F32 kernels: the tiled fp32 MFMA GEMM with the bias in its epilogue, the 3x3 as an
-    // implicit GEMM over the map (no im2col) with its kernel repacked to (tap, channel)
-    // rows; maps whose rows are not 16-byte aligned (or a 3x3 with Cin % 32 != 0) take
-    // im2col + MUL_MAT below
+    // F32 kernels: the GEMM over their bf16 planes with the bias in its epilogue, the 3x3 as
+    // an implicit GEMM over the map (no im2col), its planes in (tap, channel) rows; past that
+    // GEMM's buffer offsets the fp32 MFMA one; maps whose rows are not 16-byte aligned (or a
+    // 3x3 with Cin % 32 != 0) take im2col + MUL_MAT below
     const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15) == 0 && Cin % 4 == 0;
     if ((x16 || y16) && !(w->type == T_F16 && implicit_ok(x, Cin) &&
                           (k == 3 || (reinterpret_cast<uintptr_t>(w->data) & 15) == 0)))
@@ -200,8 +200,8 @@ mi355_status conv(mi355_context* ctx, const mi355_tensor* w, const float* b, con
         return hip_check(ctx, t.done(launch_gemm_f32(g, 1, ctx->stream)), "gemm_f32 launch");
     }
     if (w->type == T_F16 && implicit_ok(x, Cin) && (k == 3 || (reinterpret_cast<uintptr_t>(w->data) & 15) == 0)) {
-        // F16 kernels: an implicit GEMM on fp16 MFMA (the map rounded to fp16 as it
-        // is loaded), bias in its epilogue; the 3x3 kernel repacked to (tap, channel)
+        // F16 kernels: an implicit GEMM on fp16 MFMA (an F32 map rounded to fp16 first, or
+        // as its kernel loads it), bias in its epilogue; the 3x3 kernel repacked to (tap, channel)
         if (k == 3 && !pre) {
             Timed t(ctx, "neck_conv3x3_pack");
             st = hip_check(ctx, t.done(launch_conv3x3_pack_f16(static_cast<const uint16_t*>(w->data), Cin, Cout,
