@@ -615,7 +615,7 @@ mi355_status check_flash_attn(mi355_context* ctx, const mi355_tensor* q, const m
 
 mi355_status flash_attn_act(mi355_context* ctx, const mi355_tensor* q, const mi355_tensor* k, const mi355_tensor* v,
                             const mi355_tensor* mask, float scale, float max_bias, float logit_softcap,
-                            const mi355_tensor* dst, const ActOut* op) {
+                            const mi355_tensor* dst, const ActOut* op, bool group) {
     const mi355_status cs = check_flash_attn(ctx, q, k, v, mask, max_bias, logit_softcap, dst);
     if (cs != MI355_STATUS_SUCCESS) return cs;
     if (!ctx) return fail(nullptr, MI355_STATUS_INVALID_ARG, "flash_attn_ext: null context");
@@ -646,7 +646,7 @@ mi355_status flash_attn_act(mi355_context* ctx, const mi355_tensor* q, const mi3
         a.out = *op;
     }
     (void)hipSetDevice(ctx->device);
-    const FaRanges r = fattn_ranges(a.nq, a.nkv, a.nh, (int)q->ne[3], ctx->cus);
+    const FaRanges r = fattn_ranges(a.nq, a.nkv, a.nh, (int)q->ne[3], ctx->cus, group);
     a.kv_split = r.split;
     a.kv_chunk = r.chunk;
     a.kv_reset = r.reset;
@@ -1017,7 +1017,7 @@ void mi355_profile_reset(mi355_context* ctx) {
 mi355_status mi355_flash_attn_ext(mi355_context* ctx, const mi355_tensor* q, const mi355_tensor* k,
                                   const mi355_tensor* v, const mi355_tensor* mask, float scale, float max_bias,
                                   float logit_softcap, const mi355_tensor* dst) {
-    return mi355::flash_attn_act(ctx, q, k, v, mask, scale, max_bias, logit_softcap, dst, nullptr);
+    return mi355::flash_attn_act(ctx, q, k, v, mask, scale, max_bias, logit_softcap, dst, nullptr, true);
 }
 
 }  // extern "C"

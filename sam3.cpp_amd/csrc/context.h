@@ -80,10 +80,10 @@ mi355_status check_flash_attn(mi355_context* ctx, const mi355_tensor* q, const m
                               const mi355_tensor* mask, float max_bias, float logit_softcap, const mi355_tensor* dst);
 // FLASH_ATTN_EXT with the checks of mi355_flash_attn_ext; with op the output
 // goes to the next MUL_MAT's operand (rows b*n_q + iq, K = n_head*D) instead
-// of dst (which still gives the shape).
+// of dst (which still gives the shape). group: fattn_ranges'.
 mi355_status flash_attn_act(mi355_context* ctx, const mi355_tensor* q, const mi355_tensor* k, const mi355_tensor* v,
                             const mi355_tensor* mask, float scale, float max_bias, float logit_softcap,
-                            const mi355_tensor* dst, const ActOut* op);
+                            const mi355_tensor* dst, const ActOut* op, bool group = false);
 // mul_mat_act with a fused epilogue (residual or qkv split); dst [M][N] never
 // exists.
 mi355_status mul_mat_epi(mi355_context* ctx, const mi355_tensor* s0, const ActF16& a, const MmqEpi& e);

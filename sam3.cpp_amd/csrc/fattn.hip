@@ -591,7 +591,7 @@ __global__ __launch_bounds__(256) void fattn_combine_kernel(const FaArgs p, int 
         act_store_chunk(p.out, (int64_t)b * p.nq + qi, (int64_t)p.nh * D, ((int64_t)h * D) / 4 + c, o);
 }
 
-FaRanges fattn_ranges(int nq, int nkv, int nh, int B, int cus) {
+FaRanges fattn_ranges(int nq, int nkv, int nh, int B, int cus, bool group) {
     const int64_t wgs = (int64_t)((nq + FA_BQ - 1) / FA_BQ) * nh * B;
     const int ntile = (nkv + FA_BKV - 1) / FA_BKV;
     FaRanges r{1, nkv, 0};
@@ -607,7 +607,7 @@ FaRanges fattn_ranges(int nq, int nkv, int nh, int B, int cus) {
     // more (4 heads, 1021 x 3999 of 96: 32 us with a workgroup per range, 25 with two ranges to a
     // workgroup; 8 heads, 1024 x 1024 of 96: 25 and 19; 16 heads, 300 x 5184 of 128: 58, 65 with two,
     // which is 288 workgroups, 47 with three)
-    if (wgs * 3 <= cus && r.split * wgs > cus) {
+    if (group && wgs * 3 <= cus && r.split * wgs > cus) {
         const int n = cus / (int)wgs, m = (r.split + n - 1) / n;
         r.split = (r.split + m - 1) / m;
         r.chunk *= m;

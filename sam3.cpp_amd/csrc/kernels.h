@@ -213,11 +213,14 @@ struct FaArgs {
                                 // combined by a second kernel; fattn_part_bytes() of workspace
     int kv_reset;               // > 0: a chunk holds several ranges of this many 64-key tiles
 };
-// Key ranges for grids too small to fill the GPU (split 1: none), and their workspace.
+// Key ranges for grids too small to fill the GPU (split 1: none), and their workspace. group: whether
+// a workgroup may take several ranges, which changes fp32 roundings. The encoders keep one each: their
+// quantizers would make other quants of such a difference (1.3% of Hiera-tiny's output) for less than
+// a hundredth of the time (608 x 608 1000 us and 991 with groups, ViT of 4 heads and 48 x 48 332 and 330).
 struct FaRanges {
     int split, chunk, reset;    // FaArgs' kv_split, kv_chunk, kv_reset
 };
-FaRanges fattn_ranges(int nq, int nkv, int nh, int B, int cus);
+FaRanges fattn_ranges(int nq, int nkv, int nh, int B, int cus, bool group);
 size_t fattn_part_bytes(int D, int nq, int nh, int B, int kv_split);
 hipError_t launch_fattn(const FaArgs& a, int D, bool qf32, bool kvf32, int B, hipStream_t st);
 

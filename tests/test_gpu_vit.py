@@ -285,3 +285,50 @@ def test_vit_block_fusion_bit_exact(mi, ctx, orc, is_global, tname):
         ctx.set_fusion(True)
     assert np.isfinite(outs[0]).all()
     assert np.array_equal(outs[0], outs[1]), f"max diff {np.abs(outs[0] - outs[1]).max():.3e}"
+
+
+@pytest.mark.parametrize("tname", ["f16", "q8_0"])
+def test_vit_block_attention_keeps_a_workgroup_per_range(mi, ctx, orc, tname):
+    """A global block at a grid whose FLASH_ATTN_EXT call gives workgroups several key ranges (8 heads
+    of 1024 tokens) equals the block composed of its ops with attention one head at a time, where
+    each range has its own: no fp32 rounding differs, which a quantizer would make another quant of."""
+    t = orc.NAME_TYPE[tname]
+    E, NH, MLP, grid = 512, 8, 512, 32
+    HD, M = E // NH, grid * grid
+    host, devs, vec = _block_weights(mi, orc, t, E, MLP, seed=27)
+    x0 = orc.normal(M * E, 28, 1).reshape(M, E)
+    vd = {k: dev(v) for k, v in vec.items()}
+    fd = dev(axial_cis(orc, HD, grid, 24 / grid))
+    w = {n: mi.from_torch(devs[n], t, [host[n][2], host[n][1]]) for n in host}
+    blk = mi.VitBlock()
+    for n in w:
+        setattr(blk, n + "_w", w[n])
+    for k, v in vd.items():
+        setattr(blk, k, v.data_ptr())
+    blk.freqs_cis, blk.is_global = fd.data_ptr(), 1
+    got = dev(x0)
+    ctx.vit_block_forward(_hp(mi, E, NH, MLP, 16, grid, pos_grid=16), blk, _p(got))
+
+    rows = lambda n: torch.empty((M, n), dtype=torch.float32, device="cuda")
+    mm = lambda n, a, o: ctx.mul_mat(w[n], mi.from_torch(a, mi.F32, [a.shape[1], M]), mi.from_torch(o, mi.F32, [o.shape[1], M]))
+    x, y, qkv, attn, h = dev(x0), rows(E), rows(3 * E), rows(E), rows(MLP)
+    q, k, v = (torch.empty((NH, M, HD), dtype=torch.float16, device="cuda") for _ in range(3))
+    ctx.vit_layer_norm(_p(x), None, 0, _p(vd["norm1_w"]), _p(vd["norm1_b"]), _p(y), M, E, grid)
+    mm("qkv", y, qkv)
+    ctx.vit_qkv_rope(_p(qkv), _p(vd["qkv_b"]), _p(fd), _p(q), _p(k), _p(v), M, M, NH, HD)
+    for i in range(NH):
+        o = rows(HD)
+        ctx.flash_attn_ext(*(mi.from_torch(a[i], mi.F16, [HD, M, 1, 1]) for a in (q, k, v)),
+                           mi.from_torch(o, mi.F32, [HD, 1, M, 1]), HD ** -0.5)
+        ctx.synchronize()
+        attn[:, i * HD:(i + 1) * HD] = o
+    torch.cuda.synchronize()
+    mm("proj", attn, y)
+    ctx.vit_proj_residual(_p(x), _p(y), _p(vd["proj_b"]), M, E, grid)
+    ctx.vit_layer_norm(_p(x), None, 0, _p(vd["norm2_w"]), _p(vd["norm2_b"]), _p(y), M, E, grid)
+    mm("fc1", y, h)
+    ctx.vit_bias_gelu(_p(h), _p(vd["fc1_b"]), M, MLP)
+    mm("fc2", h, y)
+    ctx.vit_bias_residual(_p(x), _p(y), _p(vd["fc2_b"]), M, E)
+    ctx.synchronize()
+    assert torch.isfinite(got).all() and torch.equal(got, x)
