@@ -537,8 +537,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fattn_kernel(const F
 // operand output keeps 8 consecutive threads on one 32-block.  Bound by the partial outputs it
 // reads and by their latency: up to eight ranges' loads are all issued before the first is used
 // (KS of them; 2 heads, 700 x 700 of 128 in 5 ranges 15.4 us with the loop over them, 14.4 so).
-// KS = 0 is the loop, for more ranges: sixteen loads and their registers leave too few wavefronts
-// (4 heads, 640 x 1500 of 128 in 12 ranges 28.1 us, 24.5 with the loop).
+// KS = 0 is the loop, for more ranges (4 heads, 640 x 1500 of 128 in 12 ranges 24.5 us, 28.1 with
+// sixteen loads) and for more than four over many outputs (8 heads, 1024 x 1024 of 96 in 8 ranges
+// 25.4 and 27.3): enough wavefronts hide the latency, and the loads' registers leave fewer.
 template <int D, int KS>
 __global__ __launch_bounds__(256) void fattn_combine_kernel(const FaArgs p, int B) {
     constexpr int CPR = D / 4;
@@ -663,7 +664,7 @@ static void fa_launch_d(const FaArgs& a, bool qf32, bool kvf32, int B, hipStream
         const int64_t n = (int64_t)B * a.nh * a.nq * (D / 4);
         const unsigned g = (unsigned)((n + 255) / 256);
         if (a.kv_split <= 4) fattn_combine_kernel<D, 4><<<g, 256, 0, st>>>(a, B);
-        else if (a.kv_split <= 8) fattn_combine_kernel<D, 8><<<g, 256, 0, st>>>(a, B);
+        else if (a.kv_split <= 8 && n <= 1 << 17) fattn_combine_kernel<D, 8><<<g, 256, 0, st>>>(a, B);
         else fattn_combine_kernel<D, 0><<<g, 256, 0, st>>>(a, B);
     }
 }
