@@ -583,20 +583,30 @@ __global__ __launch_bounds__(256, 3) void conv1x1_f32map_kernel(const float* __r
             if (s + 2 < nst) dma(s0 + s + 2, lb[s & 1]);
         }
     }
-    float* D = ksplit > 1 ? part + (int64_t)split * M * N : y;  // a split's partial sums, no bias
+    // a split's partial sums go without bias, in a branch of their own: its load, also where it is
+    // only skipped, makes a store wait for the one before (9 x 9, 256 -> 52 channels 8.8 us, 13.9 so)
+    auto store = [&](float* D, bool plain, const float (&bv)[2]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int n = n0 + wn * 64 + j * 32 + lr;
-        if (n >= N) continue;
-        const float bv = ksplit > 1 ? 0.0f : bias[n];
+        for (int j = 0; j < 2; ++j) {
+            const int n = n0 + wn * 64 + j * 32 + lr;
+            if (n >= N) continue;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
-                if (m < M) D[(int64_t)m * N + n] = ksplit > 1 ? acc[i][j][r] : acc[i][j][r] + bv;
-            }
+                for (int r = 0; r < 16; ++r) {
+                    const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
+                    if (m < M) D[(int64_t)m * N + n] = plain ? acc[i][j][r] : acc[i][j][r] + bv[j];
+                }
+        }
+    };
+    if (ksplit > 1) {
+        store(part + (int64_t)split * M * N, true, {0.0f, 0.0f});
+        return;
     }
+    float bv[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) bv[j] = n0 + wn * 64 + j * 32 + lr < N ? bias[n0 + wn * 64 + j * 32 + lr] : 0.0f;
+    store(y, false, bv);
 }
 
 // y[r][c] += b[c], four channels per thread (C % 4 == 0)
