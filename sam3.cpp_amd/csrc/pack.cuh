@@ -54,30 +54,32 @@ __device__ __forceinline__ void split_w_item(int64_t i, const float* __restrict_
 
 // A conv-transpose kernel [kW=2, kH=2, Cout, Cin] (memory [ci][co][kh][kw]), F32 or F16, -> F16
 // MUL_MAT weight rows [4*Cout][Cin], row n = (kh*2 + kw)*Cout + co. The F32 -> F16 cast rounds to
-// nearest even, as ggml_cast does (sam3_conv_transpose_weight, sam3.cpp:1087-1090). Block b of 256
-// threads transposes 64 channels ci by 64 elements (co, tap) through LDS (8 KB): whole segments
+// nearest even, as ggml_cast does (sam3_conv_transpose_weight, sam3.cpp:1087-1090). Block b of WV
+// wavefronts transposes 64 channels ci by 64 elements (co, tap) through LDS (8 KB): whole segments
 // are read and written. One thread per element read 64 lines per wavefront, each line again for
 // every other element of it. t: PACK_LDS halves.
 constexpr int PACK_LDS = 64 * 66;
 __host__ __device__ inline int64_t deconv_pack_blocks(int Cin, int Cout) { return (int64_t)((Cin + 63) / 64) * ((4LL * Cout + 63) / 64); }
+template <int WV>
 __device__ __forceinline__ void deconv_pack_block(int64_t b, const void* __restrict__ w, int wtype, int Cin, int Cout,
                                                   uint16_t* __restrict__ out, uint16_t* t) {
+    constexpr int NR = 64 / WV;  // rows per wavefront
     const int nci = (Cin + 63) / 64, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int ci0 = (int)(b % nci) * 64, e0 = (int)(b / nci) * 64, ne = 4 * Cout;
-    uint16_t v[16];
+    uint16_t v[NR];
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        const int ci = ci0 + 4 * k + wv, e = e0 + lane;
+    for (int k = 0; k < NR; ++k) {
+        const int ci = ci0 + WV * k + wv, e = e0 + lane;
         const int64_t src = (int64_t)ci * ne + e;
         v[k] = 0;
         if (ci < Cin && e < ne) v[k] = wtype == T_F16 ? static_cast<const uint16_t*>(w)[src] : f2h(static_cast<const float*>(w)[src]);
     }
 #pragma unroll
-    for (int k = 0; k < 16; ++k) t[66 * lane + 4 * k + wv] = v[k];
+    for (int k = 0; k < NR; ++k) t[66 * lane + WV * k + wv] = v[k];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        const int r = 4 * k + wv, e = e0 + r, ci = ci0 + lane;  // e = co * 4 + tap
+    for (int k = 0; k < NR; ++k) {
+        const int r = WV * k + wv, e = e0 + r, ci = ci0 + lane;  // e = co * 4 + tap
         if (ci < Cin && e < ne) out[((int64_t)(e & 3) * Cout + (e >> 2)) * Cin + ci] = t[66 * r + lane];
     }
 }
