@@ -116,7 +116,11 @@ mi355_status deconv(mi355_context* ctx, const mi355_tensor* w, const float* b, c
     if (implicit_ok(x, Cin)) {
         // one fp16-MFMA GEMM whose epilogue adds the bias (+ GELU) and scatters to the 2x map
         const void* xm = x;
-        if (!x16 && conv_f16_dma_fits(4, P, Cin, 4LL * Cout)) {
+        // (few columns over a large map do not pay for a pass over it: their kernel rounds it as it
+        // reads. 191 x 191, 672 -> 32 channels 43 us and 53 with the pass, 158 x 158, 992 -> 64 48 and
+        // 57; 178 x 178, 576 -> 104 66 and 61, 200 x 200, 64 -> 32 26 and 24)
+        const bool wide = y16 || Cout > 96 || P * Cin < 10000000;
+        if (!x16 && wide && conv_f16_dma_fits(4, P, Cin, 4LL * Cout)) {
             st = half_map(ctx, x, P, Cin, D);
             if (st != MI355_STATUS_SUCCESS) return st;
             xm = D;

@@ -1,6 +1,6 @@
 // SAM3 SimpleFPN neck kernels (sam3_build_neck_graph, sam3.cpp:3867-3925) on
 // token-major activations [H*W][C] (ggml [C, W, H]).  conv_f16_dma_kernel (over
-// fp16 maps; conv1x1_f32map_kernel for a 1x1 over an F32 one, and conv_f16_kernel,
+// fp16 maps; conv_f32map_kernel for a 1x1 or conv-transpose over an F32 one, and conv_f16_kernel,
 // register-staged, for the rest and operands beyond 32-bit buffer offsets) is the fp16-MFMA implicit GEMM of the F16-kernel convolutions (3x3,
 // 1x1 and the 2x2 / stride-2 conv-transpose with its scatter, bias and GELU in
 // the epilogue; the 3x3 and 1x1 split K on grids smaller than the CU count, the
@@ -494,23 +494,25 @@ __global__ __launch_bounds__(256, 2) void conv_f16_dma_kernel(const uint16_t* __
     }
 }
 
-// The 1x1 over an F32 map: the same GEMM with the map staged as it is (128 bytes per pixel and
-// 32-deep stage) and rounded to fp16 (RNE, f2h) as the fragments are read, so no pass over the map
-// goes before it: 288 x 288, 256 -> 256 channels 41 us, against 25 for that pass and 30 for
-// conv_f16_dma_kernel. The same operands, products and order over K: the same bits.
+// The 1x1 and the conv-transpose over an F32 map: the same GEMM with the map staged as it is (128
+// bytes per pixel and 32-deep stage) and rounded to fp16 (RNE, f2h) as the fragments are read, so no
+// pass over the map goes before it: 1x1, 288 x 288, 256 -> 256 channels 36 us, against 25 for that
+// pass and 30 for conv_f16_dma_kernel. The same operands, products and order over K: the same bits.
 // Map rows of 8 chunks of 16 bytes, chunk c of row r in slot c ^ (r >> 1 & 7); weight rows of
 // four, csw<4>.
 namespace {
-struct Conv1Stage {
+struct Map32Stage {
     float A[CT * 32];     // 128 map rows x 32 channels, fp32
     uint16_t B[CT * 32];  // 128 weight rows x 32 K, fp16
 };
 }  // namespace
-__global__ __launch_bounds__(256, 3) void conv1x1_f32map_kernel(const float* __restrict__ x, const uint16_t* __restrict__ w,
-                                                                const float* __restrict__ bias, int M, int C, int N,
-                                                                float* __restrict__ y, int ksplit, int sps,
-                                                                float* __restrict__ part) {
-    __shared__ __attribute__((aligned(16))) Conv1Stage sb[2];
+template <int TAPS>
+__global__ __launch_bounds__(256, 3) void conv_f32map_kernel(const float* __restrict__ x, const uint16_t* __restrict__ w,
+                                                             const float* __restrict__ bias, int H, int W, int C, int N, int gelu,
+                                                             float* __restrict__ y, int ksplit, int sps,
+                                                             float* __restrict__ part) {
+    __shared__ __attribute__((aligned(16))) Map32Stage sb[2];
+    const int M = H * W;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wv & 1, wn = wv >> 1;
@@ -541,14 +543,14 @@ __global__ __launch_bounds__(256, 3) void conv1x1_f32map_kernel(const float* __r
     auto dma = [&](int s, uint32_t base) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            dma_b128_so(xr, base + (uint32_t)offsetof(Conv1Stage, A) + 1024u * (4 * wv + j), xoff[j], s * 128);
+            dma_b128_so(xr, base + (uint32_t)offsetof(Map32Stage, A) + 1024u * (4 * wv + j), xoff[j], s * 128);
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-            dma_b128_so(wr, base + (uint32_t)offsetof(Conv1Stage, B) + 1024u * (2 * wv + j), woff[j], s * 64);
+            dma_b128_so(wr, base + (uint32_t)offsetof(Map32Stage, B) + 1024u * (2 * wv + j), woff[j], s * 64);
     };
     const v16f zf = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     v16f acc[2][2] = {{zf, zf}, {zf, zf}};
-    auto compute = [&](const Conv1Stage& b) __attribute__((always_inline)) {
+    auto compute = [&](const Map32Stage& b) __attribute__((always_inline)) {
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
             v8h a[2], bf[2];
@@ -583,6 +585,28 @@ __global__ __launch_bounds__(256, 3) void conv1x1_f32map_kernel(const float* __r
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // and stage s's buffer is read
             if (s + 2 < nst) dma(s0 + s + 2, lb[s & 1]);
         }
+    }
+    if (TAPS == 4) {  // + bias (+ GELU), each tap to its pixel of the 2x map
+        const int Cout = N >> 2;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int n = n0 + wn * 64 + j * 32 + lr;
+            if (n >= N) continue;
+            const int t = n / Cout, co = n - t * Cout;
+            const float bv = bias[co];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
+                    if (m >= M) continue;
+                    const int qy = m / W, qx = m - qy * W;
+                    const int64_t pix = (int64_t)(2 * qy + (t >> 1)) * (2 * W) + 2 * qx + (t & 1);
+                    const float v = acc[i][j][r] + bv;
+                    y[pix * Cout + co] = gelu ? gelu_erf(v) : v;
+                }
+        }
+        return;
     }
     // a split's partial sums go without bias, in a branch of their own: its load, also where it is
     // only skipped, makes a store wait for the one before (9 x 9, 256 -> 52 channels 8.8 us, 13.9 so)
@@ -736,7 +760,7 @@ hipError_t launch_conv_f16(int taps, const void* x, bool x16, const uint16_t* w,
     const unsigned grid = (unsigned)((tiles + 7) / 8 * 8);
     const int gl = gelu ? 1 : 0;
     if (x16 && !conv_f16_dma_fits(taps, M, C, N)) return hipErrorInvalidValue;
-    const bool map32 = taps == 1 && !x16 && !y16 && conv_f16_dma_fits(taps, M, C, N);
+    const bool map32 = taps != 9 && !x16 && !y16 && conv_f16_dma_fits(taps, M, C, N);
     if (x16 || map32) {
         // the K split, when the caller gave room for its partial sums
         // (the reduce stores float4 rows: y and part on 16 bytes; N % 4 == 0 in the split choice)
@@ -753,7 +777,10 @@ hipError_t launch_conv_f16(int taps, const void* x, bool x16, const uint16_t* w,
             if (pair) even<<<gs, 256, 0, st>>>(xh, w, bias, H, W, C, N, gl, y, S, sps, part);
             else any<<<gs, 256, 0, st>>>(xh, w, bias, H, W, C, N, gl, y, S, sps, part);
         };
-        if (map32) conv1x1_f32map_kernel<<<gs, 256, 0, st>>>(static_cast<const float*>(x), w, bias, (int)M, C, N, static_cast<float*>(y), S, sps, part);
+        const float* xf = static_cast<const float*>(x);
+        float* yf = static_cast<float*>(y);
+        if (map32 && taps == 1) conv_f32map_kernel<1><<<gs, 256, 0, st>>>(xf, w, bias, H, W, C, N, 0, yf, S, sps, part);
+        else if (map32) conv_f32map_kernel<4><<<gs, 256, 0, st>>>(xf, w, bias, H, W, C, N, gl, yf, S, sps, part);
         else if (taps == 9 && !y16) go(conv_f16_dma_kernel<9, false, true>, conv_f16_dma_kernel<9, false, false>);
         else if (taps == 4 && y16) go(conv_f16_dma_kernel<4, true, true>, conv_f16_dma_kernel<4, true, false>);
         else if (taps == 4) go(conv_f16_dma_kernel<4, false, true>, conv_f16_dma_kernel<4, false, false>);

@@ -72,3 +72,23 @@ def test_conv_f16_ranges_of_odd_length(mi, ctx):
     ctx.neck_conv(mi.from_torch(wd, mi.F16, [3, 3, C, N]), bd.data_ptr(), xd.data_ptr(), H, H, y.data_ptr())
     ctx.synchronize()
     assert bool((y[1:, 1:] == 1).all()), y[1:, 1:].unique()
+
+
+@pytest.mark.parametrize("Cin,Cout", [(672, 20), (704, 96)])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_deconv_f16_large_map_few_columns(mi, ctx, Cin, Cout, gelu):
+    """A conv-transpose of few output channels over a large F32 map reads it without a pass before:
+    bit for bit its two halves by themselves, which take the pass (no output pixel sees both)."""
+    H, W = 124, 131
+    rng = np.random.default_rng(Cin)
+    wd = torch.from_numpy(rng.standard_normal((Cin, Cout, 2, 2)).astype(np.float16).view(np.int16)).cuda()
+    bd = torch.from_numpy(rng.standard_normal(Cout).astype(np.float32)).cuda()
+    xd = torch.from_numpy(rng.standard_normal((H * W, Cin)).astype(np.float32)).cuda()
+    assert H * W * Cin > 10 ** 7 > H * W * Cin // 2
+    y = torch.full((2, 4 * H * W, Cout), float("nan"), dtype=torch.float32, device="cuda")
+    wt = mi.from_torch(wd, mi.F16, [2, 2, Cout, Cin])
+    ctx.neck_deconv(wt, bd.data_ptr(), xd.data_ptr(), H, W, gelu, y[0].data_ptr())
+    for i in range(2):
+        ctx.neck_deconv(wt, bd.data_ptr(), xd[i * H * W // 2:].data_ptr(), H // 2, W, gelu, y[1, i * 2 * H * W:].data_ptr())
+    ctx.synchronize()
+    assert torch.isfinite(y).all() and torch.equal(y[0], y[1])
